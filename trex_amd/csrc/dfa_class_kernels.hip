@@ -1,0 +1,339 @@
+// DFA walks over byte classes (gfx950, wave64): contiguous strings of any
+// alignment, any alphabet.
+//
+// Bytes with equal table columns form one class; a pattern rarely has more
+// than 31. One LDS read maps a byte to its class, and one more per byte pair
+// fetches what the pair does to the state, whatever bytes the pattern uses:
+//
+//  * dfa16_cls_n10 / _n15 / _n16 (at most that many states): the pair's whole
+//    function as one 64-bit word, so the reads do not wait for the state, and a
+//    step is one, two or three instructions (Width).
+//  * dfa_cls_pair / dfa_cls_single (17 to 256 states): the successor bytes of
+//    a pair (or of one byte, where the pairs' table would not fit), read at
+//    the state.
+//
+// Every string is read by 16-byte loads from its first byte on, whatever its
+// alignment, and its last len % 16 bytes by at most four loads of 8, 4, 2 and
+// 1 bytes that are issued ahead of the walk: no byte loop, and no byte outside
+// the string is read. Missing bytes of the last vector take the identity
+// class.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "device_common.h"
+
+// Arguments of the kernels of at most 16 states (same layout in dfa.cpp).
+struct ClassArgs {
+    const uint8_t* bytes;
+    const int64_t* begin;
+    const int64_t* end;
+    int64_t n_strings;
+    const uint8_t* tab;
+    uint32_t tab_bytes;
+    uint32_t classes;     // identity class included
+    uint32_t accept;      // bit s: state s accepts
+    uint32_t start;
+    uint8_t* out_state;
+    uint8_t* out_accept;
+};
+
+namespace {
+
+using namespace trexdev;
+
+constexpr int kClsBytes = 256;    // byte -> class * 8
+constexpr int kMapBytes = 1040;   // map[257] of the wide form, padded
+constexpr int kPF = 4;            // vectors in flight ahead of the block being walked
+
+// The string each thread of a 256-thread workgroup walks: the workgroup's
+// strings in order of length, so that the lanes of a wave end together (a wave
+// lasts as long as its longest string). Lengths go to 64 buckets, exact below
+// 16 vectors and eight to the octave above. Strings of nearly equal length, or
+// of under kSortFrom vectors, stay as they are: ordering costs a pass through
+// LDS (2 us of 15 us for a million strings of 16 to 64 bytes), and gains as
+// much as the lengths differ (400,000 strings of 20 to 400 bytes: 30 us as
+// they lie, 23 us in order).
+constexpr uint32_t kOrderBytes = 64 * 4 + 256 * 2;
+constexpr uint32_t kSortFrom = 8;
+
+__device__ __forceinline__ uint32_t length_bucket(int64_t len) {
+    const uint32_t v = (uint32_t)min<int64_t>((len + 15) >> 4, 1023);
+    if (v < 16u) return v;
+    const uint32_t e = 31u - (uint32_t)__clz((int)v);   // 4 .. 9
+    return 16u + (e - 4u) * 8u + ((v >> (e - 3u)) & 7u);
+}
+
+// Called by every thread of the workgroup, after `count` was cleared and a
+// barrier: the offset of the thread's string in the workgroup's run of n_here
+// strings (>= n_here: none).
+__device__ __forceinline__ uint32_t order_by_length(uint32_t* count, uint32_t n_here, int64_t len) {
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    uint16_t* item = reinterpret_cast<uint16_t*>(count + 64);
+    const uint32_t b = length_bucket(len);
+    uint32_t rank = 0;
+    if (t < n_here) rank = atomicAdd(&count[b], 1u);
+    __syncthreads();
+    const uint32_t own = count[63u - lane];   // longest bucket first; the same in every wave
+    const uint64_t used = __ballot(own != 0u);
+    const int longest = 63 - (int)__builtin_ctzll(used), shortest = (int)__builtin_clzll(used);
+    if (longest < (int)kSortFrom || longest - shortest < 3) return t;
+    uint32_t x = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
+        if ((int)lane >= d) x += y;
+    }
+    const uint32_t at = (uint32_t)__shfl((int)(x - own), (int)(63u - b), 64) + rank;
+    if (t < n_here) item[at] = (uint16_t)t;
+    __syncthreads();
+    return t < n_here ? item[t] : t;
+}
+
+// Stages the table (its copy in LDS starts at byte 0, so that table offsets
+// are immediates) and finds the thread's string, -1 for none. Dynamic LDS:
+// tab_bytes, and kOrderBytes more in workgroups of 256 threads.
+__device__ __forceinline__ int64_t stage_and_pick(uint8_t* lds, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
+                                                  const int64_t* __restrict__ begin,
+                                                  const int64_t* __restrict__ endp, int64_t n_strings) {
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x;
+    const uint32_t n_here = (uint32_t)min<int64_t>(n_strings - first, blockDim.x);
+    const int64_t mine = first + min(threadIdx.x, n_here - 1u);
+    const int64_t len = endp[mine] - begin[mine];
+    const bool order = blockDim.x == 256u;
+    uint32_t* count = reinterpret_cast<uint32_t*>(lds + tab_bytes);
+    stage_table(lds, tabg, (int)tab_bytes);
+    if (order && threadIdx.x < 64u) count[threadIdx.x] = 0u;
+    __syncthreads();
+    const uint32_t k = order ? order_by_length(count, n_here, len) : threadIdx.x;
+    return k < n_here ? first + k : -1;
+}
+
+// Function words by number of states: the field of state s holds its successor,
+// and the walk keeps its state as the shift amount of its field, so that a step
+// is as few dependent instructions as the width allows.
+//   W10: ten 6-bit fields of 6 * successor. word >> amount is the next amount
+//        (the hardware reads the low six bits of an amount).
+//   W15: fifteen 4-bit fields from bit 2 on: word >> amount has 4 * successor in
+//        bits 2 to 5, and the field below's top bits to mask off under them.
+//   W16: sixteen 4-bit fields: a mask and a shift.
+enum Width { W10, W15, W16 };
+
+template <Width W>
+__device__ __forceinline__ uint32_t fn_step(uint64_t f, uint32_t amount) {
+    const uint32_t x = (uint32_t)(f >> (amount & 63u));
+    return W == W10 ? x : W == W15 ? x & 60u : (x & 15u) << 2;
+}
+
+template <Width W>
+struct ClassWalk {
+    const uint8_t* cls;   // [256] class * 8
+    const char* f2;       // pair functions
+    uint32_t stride;      // entries from one second class to the next
+    uint32_t ident;       // identity class * 8
+    uint32_t s;           // the state as its field's shift amount (W10: in the low six bits)
+
+    __device__ __forceinline__ uint64_t fn(uint32_t c0, uint32_t c1) const {
+        return *reinterpret_cast<const uint64_t*>(f2 + (__umul24(c1, stride) + c0));
+    }
+    __device__ __forceinline__ void vector(const uint4& v) {
+        uint32_t c[16];
+        uint64_t f[8];
+        classes(v, c);
+        functions(c, f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s = fn_step<W>(f[i], s);
+    }
+    __device__ __forceinline__ void classes(const uint4& v, uint32_t (&c)[16]) const {
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) c[i] = cls[(x[i >> 2] >> (8 * (i & 3))) & 255u];
+    }
+    __device__ __forceinline__ void functions(const uint32_t (&c)[16], uint64_t (&f)[8]) const {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = fn(c[2 * i], c[2 * i + 1]);
+    }
+    // A block of vectors as a pipeline of three stages: the class reads of
+    // vector k + 2 and the function reads of vector k + 1 go out ahead of
+    // vector k's chain of steps, so neither read's latency is waited for
+    // vector by vector (an empty asm ties each vector's words to the state, or
+    // the compiler issues the whole block's reads at once and runs out of
+    // registers).
+    template <int PF>
+    __device__ __forceinline__ void block(const uint4 (&a)[PF]) {
+        uint32_t c[16];
+        uint64_t f[8];
+        classes(a[0], c);
+        functions(c, f);
+        classes(a[1], c);
+#pragma unroll
+        for (int k = 0; k < PF; ++k) {
+            uint64_t g[8];
+            if (k + 1 < PF) functions(c, g);
+            if (k + 2 < PF) {
+                uint4 x = a[k + 2];
+                asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w) : "v"(s));
+                classes(x, c);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s = fn_step<W>(f[i], s);
+            if (k + 1 < PF) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) f[i] = g[i];
+            }
+        }
+    }
+    // bytes lo .. lo + n - 1 of a vector
+    __device__ __forceinline__ void masked(const uint4& v, uint32_t lo, uint32_t n) {
+        uint32_t c[16];
+        uint64_t f[8];
+        classes(v, c);
+#pragma unroll
+        for (uint32_t i = 0; i < 16u; ++i) c[i] = i - lo < n ? c[i] : ident;
+        functions(c, f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s = fn_step<W>(f[i], s);
+    }
+    __device__ __forceinline__ uint32_t state() const { return W == W10 ? (s & 63u) / 6u : s >> 2; }
+};
+
+// LEAVE: workgroups whose strings are alike are left to the rotated kernel.
+template <Width W, bool LEAVE>
+__device__ __forceinline__ void class_kernel(const ClassArgs& A)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    if constexpr (LEAVE) {
+        if (strings_alike(reinterpret_cast<uint32_t*>(lds), A.begin, A.end, A.n_strings)) return;
+    }
+    const int64_t sid = stage_and_pick(lds, A.tab, A.tab_bytes, A.begin, A.end, A.n_strings);
+    if (sid < 0) return;
+    const Span sp(A.bytes, A.begin[sid], A.end[sid]);
+    const uint4 first = sp.first(), last = sp.last();
+    ClassWalk<W> w{lds, reinterpret_cast<const char*>(lds) + kClsBytes, A.classes | 1u, (A.classes - 1u) * 8u,
+                   A.start * (W == W10 ? 6u : 4u)};
+    if (sp.n_first) w.masked(first, sp.lo, sp.n_first);
+    // the slower steps let half-read cache lines be evicted: whole lines there
+    // (13 states, 262,144 x 4 KiB: 304 us by fours, 254 us by eights; ten
+    // states and less: 250 us either way, and short strings run 10 to 20 %
+    // faster with the registers of four)
+    constexpr int PF = W == W10 ? kPF : 8;
+    stream_span<PF>(sp.body, sp.full, [&](const uint4 (&a)[PF]) { w.block(a); }, [&](const uint4& v) { w.vector(v); });
+    if (sp.n_last) w.masked(last, 0u, sp.n_last);
+    const uint32_t s = w.state();
+    A.out_state[sid] = (uint8_t)s;
+    A.out_accept[sid] = (uint8_t)((A.accept >> s) & 1u);
+}
+
+// 17 to 256 states. map[byte] holds the byte's class times the strides of the
+// two positions of a pair: low half for the first byte, high half for the
+// second (PAIR), or the class's row for single bytes; map[256] is the identity
+// class. A step reads succ[row + s].
+template <bool PAIR>
+struct WideWalk {
+    const uint32_t* map;    // [257]
+    const uint8_t* succ;
+    uint32_t s;
+
+    __device__ __forceinline__ void step2(uint32_t m0, uint32_t m1) {
+        if constexpr (PAIR) {
+            s = succ[(m0 & 0xffffu) + (m1 >> 16) + s];
+        } else {
+            s = succ[m0 + s];
+            s = succ[m1 + s];
+        }
+    }
+    __device__ __forceinline__ void word(uint32_t x) {
+        const uint32_t m0 = map[x & 255u], m1 = map[(x >> 8) & 255u], m2 = map[(x >> 16) & 255u], m3 = map[x >> 24];
+        step2(m0, m1);
+        step2(m2, m3);
+    }
+    __device__ __forceinline__ void vector(const uint4& v) { word(v.x); word(v.y); word(v.z); word(v.w); }
+    __device__ __forceinline__ void maps(const uint4& v, uint32_t (&m)[16]) const {
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m[i] = map[(x[i >> 2] >> (8 * (i & 3))) & 255u];
+    }
+    // the next vector's map reads go out ahead of a vector's chain of steps
+    template <int PF>
+    __device__ __forceinline__ void block(const uint4 (&a)[PF]) {
+        uint32_t m[16];
+        maps(a[0], m);
+#pragma unroll
+        for (int k = 0; k < PF; ++k) {
+            uint32_t n[16];
+            if (k + 1 < PF) {
+                uint4 x = a[k + 1];
+                asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w) : "v"(s));
+                maps(x, n);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) step2(m[i], m[i + 1]);
+            if (k + 1 < PF) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) m[i] = n[i];
+            }
+        }
+    }
+    __device__ __forceinline__ void masked(const uint4& v, uint32_t lo, uint32_t n) {
+        uint32_t m[16];
+        maps(v, m);
+        const uint32_t ident = map[256];
+#pragma unroll
+        for (uint32_t i = 0; i < 16u; ++i) m[i] = i - lo < n ? m[i] : ident;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) step2(m[i], m[i + 1]);
+    }
+};
+
+template <bool PAIR>
+__device__ __forceinline__ void wide_kernel(const uint8_t* __restrict__ bytes, const int64_t* __restrict__ begin,
+                                            const int64_t* __restrict__ endp, int64_t n_strings,
+                                            const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
+                                            const uint8_t* __restrict__ accg, uint32_t start,
+                                            uint8_t* __restrict__ out_state, uint8_t* __restrict__ out_accept)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // map (1,040 bytes), succ
+    const int64_t sid = stage_and_pick(lds, tabg, tab_bytes, begin, endp, n_strings);
+    if (sid < 0) return;
+    const Span sp(bytes, begin[sid], endp[sid]);
+    const uint4 first = sp.first(), last = sp.last();
+    WideWalk<PAIR> w{reinterpret_cast<const uint32_t*>(lds), lds + kMapBytes, start};
+    if (sp.n_first) w.masked(first, sp.lo, sp.n_first);
+    stream_span<kPF>(sp.body, sp.full, [&](const uint4 (&a)[kPF]) { w.block(a); }, [&](const uint4& v) { w.vector(v); });
+    if (sp.n_last) w.masked(last, 0u, sp.n_last);
+    out_state[sid] = (uint8_t)w.s;
+    out_accept[sid] = accg[w.s];
+}
+
+}  // namespace
+
+// tab: 256 bytes (byte -> class * 8), then the functions of the class pairs,
+// pair (c0, c1) at entry c0 + c1 * (classes | 1): an odd stride spreads pairs
+// that share their first class over the LDS banks (a power of two puts them
+// all into one). The last class is the identity. Dynamic LDS: tab_bytes (a
+// multiple of 16), 768 bytes more in workgroups of 256 threads.
+// No kernel here has LDS of fixed size: the tables' copies then start at byte 0
+// and every offset into them is an immediate (behind 256 bytes of it, 250 us
+// of 262,144 x 4 KiB became 300 us).
+#define TREX_CLASS_KERNELS(W, TAG)                                                                            \
+    extern "C" __global__ void __launch_bounds__(256) dfa16_cls_##TAG(ClassArgs A) { class_kernel<W, false>(A); } \
+    extern "C" __global__ void __launch_bounds__(256) dfa16_cls_##TAG##_left(ClassArgs A) { class_kernel<W, true>(A); }
+
+TREX_CLASS_KERNELS(W10, n10)
+TREX_CLASS_KERNELS(W15, n15)
+TREX_CLASS_KERNELS(W16, n16)
+
+// tabg: map[257] (uint32, padded to 1,040 bytes), then the successor rows of
+// the class pairs (pair) or classes (single); accg [stride]. Dynamic LDS as
+// above.
+#define TREX_WIDE_KERNEL(NAME, PAIR)                                                                          \
+    extern "C" __global__ void __launch_bounds__(256)                                                         \
+    NAME(const uint8_t* __restrict__ bytes, const int64_t* __restrict__ begin, const int64_t* __restrict__ end, \
+         int64_t n_strings, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,                             \
+         const uint8_t* __restrict__ accg, uint32_t start, uint8_t* __restrict__ out_state,                   \
+         uint8_t* __restrict__ out_accept) {                                                                  \
+        wide_kernel<PAIR>(bytes, begin, end, n_strings, tabg, tab_bytes, accg, start, out_state, out_accept); \
+    }
+
+TREX_WIDE_KERNEL(dfa_cls_pair, true)
+TREX_WIDE_KERNEL(dfa_cls_single, false)

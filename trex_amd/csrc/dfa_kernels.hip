@@ -245,19 +245,22 @@ __device__ __forceinline__ void k1_kernel(const uint8_t* __restrict__ bytes, con
 //    phase B's state (the dead state stays dead); then the tail bytes.
 // Same results as the unrotated kernel. The host picks it for automata that
 // synchronise (the function turns constant within a few bytes); one that
-// never does would compose a whole phase A.
+// never does would compose a whole phase A. With `only_alike`, workgroups whose
+// strings are not alike (strings_alike) are left to the class kernel.
 template <int PF>
 __device__ __forceinline__ void rot_kernel(const uint8_t* __restrict__ bytes, const int64_t* __restrict__ begin,
                                            const int64_t* __restrict__ endp, int64_t n_strings,
                                            const uint8_t* __restrict__ f2g, const uint8_t* __restrict__ t2g,
                                            const uint8_t* __restrict__ t1g, const uint8_t* __restrict__ accg,
                                            uint32_t win4, uint32_t start, uint32_t dead, Fn16 init,
-                                           uint8_t* __restrict__ out_state, uint8_t* __restrict__ out_accept)
+                                           uint32_t only_alike, uint8_t* __restrict__ out_state,
+                                           uint8_t* __restrict__ out_accept)
 {
     __shared__ __attribute__((aligned(16))) uint8_t f2[1024 * 8];
     __shared__ __attribute__((aligned(16))) uint8_t t2[1024 * 16];
     __shared__ __attribute__((aligned(16))) uint8_t t1[256 * 16];
     __shared__ __attribute__((aligned(16))) uint8_t acc[16];
+    if (only_alike && !strings_alike(reinterpret_cast<uint32_t*>(acc), begin, endp, n_strings)) return;
     stage_table(f2, f2g, 1024 * 8);
     stage_table(t2, t2g, 1024 * 16);
     stage_table(t1, t1g, 256 * 16);
@@ -364,10 +367,10 @@ dfa16_k2f_rot_pf8(const uint8_t* __restrict__ bytes, const int64_t* __restrict__
                   const int64_t* __restrict__ end, int64_t n_strings, const uint8_t* __restrict__ f2g,
                   const uint8_t* __restrict__ t2g, const uint8_t* __restrict__ t1g,
                   const uint8_t* __restrict__ accg, uint32_t win4, uint32_t start, uint32_t dead, uint32_t init0,
-                  uint32_t init1, uint32_t init2, uint32_t init3, uint8_t* __restrict__ out_state,
-                  uint8_t* __restrict__ out_accept) {
+                  uint32_t init1, uint32_t init2, uint32_t init3, uint32_t only_alike,
+                  uint8_t* __restrict__ out_state, uint8_t* __restrict__ out_accept) {
     rot_kernel<8>(bytes, begin, end, n_strings, f2g, t2g, t1g, accg, win4, start, dead,
-                  Fn16{{init0, init1, init2, init3}}, out_state, out_accept);
+                  Fn16{{init0, init1, init2, init3}}, only_alike, out_state, out_accept);
 }
 
 // ---------------------------------------------------------------------------

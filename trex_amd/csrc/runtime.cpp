@@ -127,6 +127,7 @@ int get_function(const char* name, hipFunction_t* out) {
             *out = f;
             return TREX_OK;
         }
+        (void)hipGetLastError();   // not in this code object: leave no error behind for the caller's next HIP call
     }
     return fail(TREX_ERR_HIP, "kernel %s not found in any loaded code object", name);
 }

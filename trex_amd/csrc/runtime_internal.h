@@ -73,9 +73,17 @@ struct trex_dfa {
     uint8_t* d_acc = nullptr; // [stride]
     uint8_t* d_t2 = nullptr;  // [1024][16] pair table t2[pair * 16 + s] (window variants only)
     uint8_t* d_f2 = nullptr;  // [1024] uint64 pair functions, nibble s = successor of s
+    // byte-class form (dfa_class_kernels.hip), null when the table has too many classes
+    uint8_t* d_cls = nullptr;
+    int cls_bytes = 0;        // bytes of d_cls
+    int n_classes = 0;        // classes of a form of at most 16 states, identity class included
+    const char* cls_kernel = nullptr;
+    uint32_t accept_bits = 0; // bit s: state s accepts (at most 16 states)
+    bool forced = false;      // a variant was chosen by trex_dfa_set_variant
     int prefetch = 8;         // 16-byte vectors in flight per lane (8 or 16)
     int rotation = -1;        // rotated read order of contiguous strings: -1 auto, 0 off, 1 on
     bool synchronizes = false;  // some window word sends every state that can occur to one state
+    bool rotate = false;      // launches that fill the chip leave alike strings to the rotated read order
     uint32_t rot_init[4] = {0, 0, 0, 0};  // starting function of the rotated kernel's composition
     // staging for trex_dfa_match_host
     trex::DevBuf in_bytes, in_offsets, out_state, out_accept;
