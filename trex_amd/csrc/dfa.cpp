@@ -7,7 +7,6 @@
 
 #include <algorithm>
 #include <cstdio>
-#include <map>
 #include <mutex>
 #include <vector>
 
@@ -106,42 +105,6 @@ void analyse_window(trex_dfa* h, const uint8_t* delta) {
     h->rotate = h->synchronizes && !sticky;
 }
 
-// Classes of bytes with equal columns of delta, numbered by first byte;
-// returns their count.
-int byte_classes(const uint8_t* delta, int n, uint8_t (&cls)[256]) {
-    std::map<std::vector<uint8_t>, int> seen;
-    std::vector<uint8_t> column((size_t)n);
-    for (int b = 0; b < 256; ++b) {
-        for (int s = 0; s < n; ++s) column[s] = delta[s * 256 + b];
-        cls[b] = (uint8_t)seen.emplace(column, (int)seen.size()).first->second;
-    }
-    return (int)seen.size();
-}
-
-// Largest pair table of a wide DFA's class form: with the map it leaves four
-// workgroups a CU.
-constexpr int kWidePairBytes = 36 << 10;
-
-// Arguments of the class kernels of at most 16 states (same layout in
-// dfa_class_kernels.hip).
-struct ClassArgs {
-    const uint8_t* bytes;
-    const int64_t* begin;
-    const int64_t* end;
-    int64_t n_strings;
-    const uint8_t* tab;
-    uint32_t tab_bytes;
-    uint32_t classes;
-    uint32_t accept;
-    uint32_t start;
-    uint8_t* out_state;
-    uint8_t* out_accept;
-};
-
-// Launch shape of the class kernels: from kClassBlockFrom strings on, 256
-// threads a workgroup, which orders its strings by length (kOrderBytes of LDS);
-// below, one wave a workgroup, so that the waves spread over the CUs.
-constexpr int64_t kClassBlockFrom = 65536;
 // From kRotateFrom strings on (eight waves a CU; below, the rotated order is no
 // faster), a table whose composed functions turn constant (trex_dfa::rotate)
 // gets a second launch for the workgroups of long strings that all start at
@@ -151,51 +114,6 @@ constexpr int64_t kClassBlockFrom = 65536;
 // launch costs 3 to 6 us (400,000 strings of 20 to 400 bytes: 21 us without,
 // 25 us with it; 41 us by the pair kernel).
 constexpr int64_t kRotateFrom = 131072;
-constexpr unsigned kOrderBytes = 64 * 4 + 256 * 2;
-
-// Byte-class tables of the class kernels (layouts in dfa_class_kernels.hip)
-// and the kernel they are for; an empty result when the table has too many
-// classes for either form.
-std::vector<uint8_t> class_tables(const uint8_t* delta, int n, int stride, const char** kernel, int* classes) {
-    uint8_t cls[256];
-    const int count = byte_classes(delta, n, cls);
-    std::vector<uint8_t> out;
-    std::vector<int> byte_of(count, 0);   // one byte of each class
-    for (int b = 255; b >= 0; --b) byte_of[cls[b]] = b;
-    auto next = [&](int s, int c) { return c == count ? s : (int)delta[s * 256 + byte_of[c]]; };
-    if (n <= 16) {
-        if (count > 31) return out;   // class * 8 fits a byte, the identity class included
-        const int all = count + 1, odd = all | 1;
-        // field width, what a field holds per successor state, first bit (Width in dfa_class_kernels.hip)
-        const int w = n <= 10 ? 6 : 4, mul = n <= 10 ? 6 : 1, first = n > 10 && n <= 15 ? 2 : 0;
-        *kernel = n <= 10 ? "dfa16_cls_n10" : n <= 15 ? "dfa16_cls_n15" : "dfa16_cls_n16";
-        std::vector<uint64_t> f2((size_t)(all * odd + 1) & ~(size_t)1, 0);
-        for (int c1 = 0; c1 < all; ++c1)
-            for (int c0 = 0; c0 < all; ++c0)
-                for (int s = 0; s < n; ++s)
-                    f2[c0 + c1 * odd] |= (uint64_t)(mul * next(next(s, c0), c1)) << (w * s + first);
-        out.resize(256 + f2.size() * 8);
-        for (int b = 0; b < 256; ++b) out[b] = (uint8_t)(8 * cls[b]);
-        memcpy(out.data() + 256, f2.data(), f2.size() * 8);
-        *classes = all;
-        return out;
-    }
-    const int all = count + 1;
-    const bool pair = all * all * stride <= kWidePairBytes;
-    const int rows = pair ? all * all : all;
-    if (rows * stride > 65536 - 1040) return out;
-    *kernel = pair ? "dfa_cls_pair" : "dfa_cls_single";
-    out.resize(1040 + (size_t)rows * stride, 0);
-    uint32_t* map = reinterpret_cast<uint32_t*>(out.data());
-    for (int b = 0; b < 257; ++b) {
-        const uint32_t c = b < 256 ? cls[b] : (uint32_t)count;
-        map[b] = pair ? (c * all * stride) | (c * stride) << 16 : c * stride;
-    }
-    for (int r = 0; r < rows; ++r)
-        for (int s = 0; s < n; ++s)
-            out[1040 + (size_t)r * stride + s] = (uint8_t)(pair ? next(next(s, r / all), r % all) : next(s, r));
-    return out;
-}
 
 bool variant_allowed(const trex_dfa* h, int v) {
     switch (v) {
@@ -234,7 +152,6 @@ int trex_dfa_create(const uint8_t* delta, const uint8_t* accept, int n_states, i
         for (int s = 0; s < stride; ++s)
             t1[(size_t)b * stride + s] = s < n_states ? delta[s * 256 + b] : (uint8_t)s;
     for (int s = 0; s < n_states; ++s) acc[s] = accept[s] ? 1 : 0;
-    for (int s = 0; s < std::min(n_states, 16); ++s) h->accept_bits |= acc[s] ? 1u << s : 0u;
 
     int rc = upload((void**)&h->d_t1, t1.data(), t1.size());
     if (!rc) rc = upload((void**)&h->d_acc, acc.data(), acc.size());
@@ -253,11 +170,7 @@ int trex_dfa_create(const uint8_t* delta, const uint8_t* accept, int n_states, i
         rc = upload((void**)&h->d_t2, t2.data(), t2.size());
         if (!rc) rc = upload((void**)&h->d_f2, f2.data(), f2.size() * sizeof(uint64_t));
     }
-    if (!rc) {
-        const std::vector<uint8_t> tab = class_tables(delta, n_states, stride, &h->cls_kernel, &h->n_classes);
-        h->cls_bytes = (int)tab.size();
-        if (!tab.empty()) rc = upload((void**)&h->d_cls, tab.data(), tab.size());
-    }
+    if (!rc) rc = make_class_form(delta, acc.data(), nullptr, n_states, start, &h->cls);
     if (rc) { trex_dfa_destroy(h); return rc; }
     if (h->window_base >= 0) analyse_window(h, delta);
     if (h->window_base >= 0) h->auto_variant = TREX_DFA_K2_WINDOW_F;
@@ -275,7 +188,7 @@ int trex_dfa_destroy(trex_dfa* h) {
     hipFree(h->d_acc);
     hipFree(h->d_t2);
     hipFree(h->d_f2);
-    hipFree(h->d_cls);
+    h->cls.release();
     h->in_bytes.release();
     h->in_offsets.release();
     h->out_state.release();
@@ -330,12 +243,13 @@ namespace {
 
 // The rotated read order over contiguous strings; only_alike: the workgroups
 // that the class kernel leaves to it.
-int launch_rotated(trex_dfa* h, ClassArgs& A, unsigned grid, hipStream_t s, uint32_t only_alike) {
-    uint32_t win4 = (uint32_t)h->window_base * 0x01010101u, dead = (uint32_t)h->dead;
-    void* args[] = {&A.bytes, &A.begin, &A.end, &A.n_strings, &h->d_f2, &h->d_t2, &h->d_t1, &h->d_acc, &win4,
-                    &A.start, &dead, &h->rot_init[0], &h->rot_init[1], &h->rot_init[2], &h->rot_init[3], &only_alike,
-                    &A.out_state, &A.out_accept};
-    return launch("dfa16_k2f_rot_pf8", grid, kBlock, 0, s, args);
+int launch_rotated(trex_dfa* h, const uint8_t* d_bytes, const int64_t* d_begin, const int64_t* d_end,
+                   int64_t n_strings, uint32_t only_alike, uint8_t* d_final_state, uint8_t* d_accept, hipStream_t s) {
+    uint32_t win4 = (uint32_t)h->window_base * 0x01010101u, dead = (uint32_t)h->dead, start = (uint32_t)h->start;
+    void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &h->d_f2, &h->d_t2, &h->d_t1, &h->d_acc, &win4, &start,
+                    &dead, &h->rot_init[0], &h->rot_init[1], &h->rot_init[2], &h->rot_init[3], &only_alike,
+                    &d_final_state, &d_accept};
+    return launch("dfa16_k2f_rot_pf8", (unsigned)((n_strings + kBlock - 1) / kBlock), kBlock, 0, s, args);
 }
 
 // One launch of the handle's variant over begin/end ranges; `il` selects the
@@ -353,23 +267,10 @@ int dfa_dispatch(trex_dfa* h, const uint8_t* d_bytes, const int64_t* d_begin, co
     uint32_t start = (uint32_t)h->start;
     const char* il_tag = il ? "_il" : "";
     char name[48];
-    if (!il && h->d_cls && !h->forced && h->rotation == -1 && h->prefetch == 8) {
-        uint32_t tab_bytes = (uint32_t)h->cls_bytes;
-        const unsigned block = n_strings >= kClassBlockFrom ? kBlock : 64u;
-        const int64_t blocks = (n_strings + block - 1) / block;
-        const unsigned lds = tab_bytes + (block == kBlock ? kOrderBytes : 0u);
-        if (h->n_states <= 16) {
-            const bool rot = h->rotate && n_strings >= kRotateFrom;
-            ClassArgs A = {d_bytes, d_begin, d_end, n_strings, h->d_cls, tab_bytes, (uint32_t)h->n_classes,
-                           h->accept_bits, start, d_final_state, d_accept};
-            void* args[] = {&A};
-            std::snprintf(name, sizeof(name), "%s%s", h->cls_kernel, rot ? "_left" : "");
-            TREX_TRY(launch(name, (unsigned)blocks, block, lds, s, args));
-            return rot ? launch_rotated(h, A, grid, s, 1u) : TREX_OK;
-        }
-        void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &h->d_cls, &tab_bytes, &h->d_acc, &start,
-                        &d_final_state, &d_accept};
-        return launch(h->cls_kernel, (unsigned)blocks, block, lds, s, args);
+    if (!il && h->cls.d_tab && !h->forced && h->rotation == -1 && h->prefetch == 8) {
+        const bool rot = h->rotate && n_strings >= kRotateFrom;
+        TREX_TRY(launch_class_form(h->cls, d_bytes, d_begin, d_end, n_strings, rot, d_final_state, nullptr, d_accept, s));
+        return rot ? launch_rotated(h, d_bytes, d_begin, d_end, n_strings, 1u, d_final_state, d_accept, s) : TREX_OK;
     }
     if (h->variant == TREX_DFA_K2_WINDOW || h->variant == TREX_DFA_K2_WINDOW_F ||
         h->variant == TREX_DFA_K2_WINDOW_FR) {
@@ -381,8 +282,7 @@ int dfa_dispatch(trex_dfa* h, const uint8_t* d_bytes, const int64_t* d_begin, co
         trex_dfa_rotation(h, &rot, nullptr);
         if (!il && rot && h->variant == TREX_DFA_K2_WINDOW_F && h->prefetch == 8) {
             // contiguous strings, read order rotated per wave (spreads HBM channels)
-            ClassArgs A = {d_bytes, d_begin, d_end, n_strings, nullptr, 0, 0, 0, start, d_final_state, d_accept};
-            return launch_rotated(h, A, grid, s, 0u);
+            return launch_rotated(h, d_bytes, d_begin, d_end, n_strings, 0u, d_final_state, d_accept, s);
         }
         std::snprintf(name, sizeof(name), "dfa16_%s%s_pf%d", form, il_tag, h->prefetch == 16 ? 16 : 8);
         void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &table, &h->d_t1, &h->d_acc,

@@ -23,7 +23,7 @@
 
 #include "device_common.h"
 
-// Arguments of the kernels of at most 16 states (same layout in dfa.cpp).
+// Arguments of every kernel (same layout in dfa_class.cpp).
 struct ClassArgs {
     const uint8_t* bytes;
     const int64_t* begin;
@@ -31,10 +31,13 @@ struct ClassArgs {
     int64_t n_strings;
     const uint8_t* tab;
     uint32_t tab_bytes;
-    uint32_t classes;     // identity class included
-    uint32_t accept;      // bit s: state s accepts
+    uint32_t classes;        // identity class included (at most 16 states)
+    uint32_t accept;         // bit s: state s accepts (at most 16 states)
     uint32_t start;
+    const uint8_t* acc;      // accept byte of every state
+    const uint64_t* masks;   // _mask: what each state stands for
     uint8_t* out_state;
+    uint64_t* out_mask;      // _mask
     uint8_t* out_accept;
 };
 
@@ -46,53 +49,9 @@ constexpr int kClsBytes = 256;    // byte -> class * 8
 constexpr int kMapBytes = 1040;   // map[257] of the wide form, padded
 constexpr int kPF = 4;            // vectors in flight ahead of the block being walked
 
-// The string each thread of a 256-thread workgroup walks: the workgroup's
-// strings in order of length, so that the lanes of a wave end together (a wave
-// lasts as long as its longest string). Lengths go to 64 buckets, exact below
-// 16 vectors and eight to the octave above. Strings of nearly equal length, or
-// of under kSortFrom vectors, stay as they are: ordering costs a pass through
-// LDS (2 us of 15 us for a million strings of 16 to 64 bytes), and gains as
-// much as the lengths differ (400,000 strings of 20 to 400 bytes: 30 us as
-// they lie, 23 us in order).
-constexpr uint32_t kOrderBytes = 64 * 4 + 256 * 2;
-constexpr uint32_t kSortFrom = 8;
-
-__device__ __forceinline__ uint32_t length_bucket(int64_t len) {
-    const uint32_t v = (uint32_t)min<int64_t>((len + 15) >> 4, 1023);
-    if (v < 16u) return v;
-    const uint32_t e = 31u - (uint32_t)__clz((int)v);   // 4 .. 9
-    return 16u + (e - 4u) * 8u + ((v >> (e - 3u)) & 7u);
-}
-
-// Called by every thread of the workgroup, after `count` was cleared and a
-// barrier: the offset of the thread's string in the workgroup's run of n_here
-// strings (>= n_here: none).
-__device__ __forceinline__ uint32_t order_by_length(uint32_t* count, uint32_t n_here, int64_t len) {
-    const uint32_t t = threadIdx.x, lane = t & 63u;
-    uint16_t* item = reinterpret_cast<uint16_t*>(count + 64);
-    const uint32_t b = length_bucket(len);
-    uint32_t rank = 0;
-    if (t < n_here) rank = atomicAdd(&count[b], 1u);
-    __syncthreads();
-    const uint32_t own = count[63u - lane];   // longest bucket first; the same in every wave
-    const uint64_t used = __ballot(own != 0u);
-    const int longest = 63 - (int)__builtin_ctzll(used), shortest = (int)__builtin_clzll(used);
-    if (longest < (int)kSortFrom || longest - shortest < 3) return t;
-    uint32_t x = own;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
-        if ((int)lane >= d) x += y;
-    }
-    const uint32_t at = (uint32_t)__shfl((int)(x - own), (int)(63u - b), 64) + rank;
-    if (t < n_here) item[at] = (uint16_t)t;
-    __syncthreads();
-    return t < n_here ? item[t] : t;
-}
-
 // Stages the table (its copy in LDS starts at byte 0, so that table offsets
 // are immediates) and finds the thread's string, -1 for none. Dynamic LDS:
-// tab_bytes, and kOrderBytes more in workgroups of 256 threads.
+// tab_bytes, and order_bytes(256) more in workgroups of 256 threads.
 __device__ __forceinline__ int64_t stage_and_pick(uint8_t* lds, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
                                                   const int64_t* __restrict__ begin,
                                                   const int64_t* __restrict__ endp, int64_t n_strings) {
@@ -198,7 +157,8 @@ struct ClassWalk {
 };
 
 // LEAVE: workgroups whose strings are alike are left to the rotated kernel.
-template <Width W, bool LEAVE>
+// MASK: results are the states' masks.
+template <Width W, bool LEAVE, bool MASK>
 __device__ __forceinline__ void class_kernel(const ClassArgs& A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -220,7 +180,8 @@ __device__ __forceinline__ void class_kernel(const ClassArgs& A)
     stream_span<PF>(sp.body, sp.full, [&](const uint4 (&a)[PF]) { w.block(a); }, [&](const uint4& v) { w.vector(v); });
     if (sp.n_last) w.masked(last, 0u, sp.n_last);
     const uint32_t s = w.state();
-    A.out_state[sid] = (uint8_t)s;
+    if constexpr (MASK) A.out_mask[sid] = A.masks[s];
+    else A.out_state[sid] = (uint8_t)s;
     A.out_accept[sid] = (uint8_t)((A.accept >> s) & 1u);
 }
 
@@ -285,24 +246,21 @@ struct WideWalk {
     }
 };
 
-template <bool PAIR>
-__device__ __forceinline__ void wide_kernel(const uint8_t* __restrict__ bytes, const int64_t* __restrict__ begin,
-                                            const int64_t* __restrict__ endp, int64_t n_strings,
-                                            const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
-                                            const uint8_t* __restrict__ accg, uint32_t start,
-                                            uint8_t* __restrict__ out_state, uint8_t* __restrict__ out_accept)
+template <bool PAIR, bool MASK>
+__device__ __forceinline__ void wide_kernel(const ClassArgs& A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // map (1,040 bytes), succ
-    const int64_t sid = stage_and_pick(lds, tabg, tab_bytes, begin, endp, n_strings);
+    const int64_t sid = stage_and_pick(lds, A.tab, A.tab_bytes, A.begin, A.end, A.n_strings);
     if (sid < 0) return;
-    const Span sp(bytes, begin[sid], endp[sid]);
+    const Span sp(A.bytes, A.begin[sid], A.end[sid]);
     const uint4 first = sp.first(), last = sp.last();
-    WideWalk<PAIR> w{reinterpret_cast<const uint32_t*>(lds), lds + kMapBytes, start};
+    WideWalk<PAIR> w{reinterpret_cast<const uint32_t*>(lds), lds + kMapBytes, A.start};
     if (sp.n_first) w.masked(first, sp.lo, sp.n_first);
     stream_span<kPF>(sp.body, sp.full, [&](const uint4 (&a)[kPF]) { w.block(a); }, [&](const uint4& v) { w.vector(v); });
     if (sp.n_last) w.masked(last, 0u, sp.n_last);
-    out_state[sid] = (uint8_t)w.s;
-    out_accept[sid] = accg[w.s];
+    if constexpr (MASK) A.out_mask[sid] = A.masks[w.s];
+    else A.out_state[sid] = (uint8_t)w.s;
+    A.out_accept[sid] = A.acc[w.s];
 }
 
 }  // namespace
@@ -315,25 +273,26 @@ __device__ __forceinline__ void wide_kernel(const uint8_t* __restrict__ bytes, c
 // No kernel here has LDS of fixed size: the tables' copies then start at byte 0
 // and every offset into them is an immediate (behind 256 bytes of it, 250 us
 // of 262,144 x 4 KiB became 300 us).
-#define TREX_CLASS_KERNELS(W, TAG)                                                                            \
-    extern "C" __global__ void __launch_bounds__(256) dfa16_cls_##TAG(ClassArgs A) { class_kernel<W, false>(A); } \
-    extern "C" __global__ void __launch_bounds__(256) dfa16_cls_##TAG##_left(ClassArgs A) { class_kernel<W, true>(A); }
+// _left: workgroups of alike strings are left to the rotated kernel; _mask: the
+// results are the states' masks.
+#define TREX_CLASS_KERNEL(NAME, ...) \
+    extern "C" __global__ void __launch_bounds__(256) NAME(ClassArgs A) { class_kernel<__VA_ARGS__>(A); }
+#define TREX_CLASS_KERNELS(W, TAG)                               \
+    TREX_CLASS_KERNEL(dfa16_cls_##TAG, W, false, false)          \
+    TREX_CLASS_KERNEL(dfa16_cls_##TAG##_left, W, true, false)    \
+    TREX_CLASS_KERNEL(dfa16_cls_##TAG##_mask, W, false, true)
 
 TREX_CLASS_KERNELS(W10, n10)
 TREX_CLASS_KERNELS(W15, n15)
 TREX_CLASS_KERNELS(W16, n16)
 
-// tabg: map[257] (uint32, padded to 1,040 bytes), then the successor rows of
-// the class pairs (pair) or classes (single); accg [stride]. Dynamic LDS as
-// above.
-#define TREX_WIDE_KERNEL(NAME, PAIR)                                                                          \
-    extern "C" __global__ void __launch_bounds__(256)                                                         \
-    NAME(const uint8_t* __restrict__ bytes, const int64_t* __restrict__ begin, const int64_t* __restrict__ end, \
-         int64_t n_strings, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,                             \
-         const uint8_t* __restrict__ accg, uint32_t start, uint8_t* __restrict__ out_state,                   \
-         uint8_t* __restrict__ out_accept) {                                                                  \
-        wide_kernel<PAIR>(bytes, begin, end, n_strings, tabg, tab_bytes, accg, start, out_state, out_accept); \
-    }
+// tab: map[257] (uint32, padded to 1,040 bytes), then the successor rows of
+// the class pairs (pair) or classes (single), padded to 16 states. Dynamic LDS
+// as above.
+#define TREX_WIDE_KERNEL(NAME, ...) \
+    extern "C" __global__ void __launch_bounds__(256) NAME(ClassArgs A) { wide_kernel<__VA_ARGS__>(A); }
 
-TREX_WIDE_KERNEL(dfa_cls_pair, true)
-TREX_WIDE_KERNEL(dfa_cls_single, false)
+TREX_WIDE_KERNEL(dfa_cls_pair, true, false)
+TREX_WIDE_KERNEL(dfa_cls_pair_mask, true, true)
+TREX_WIDE_KERNEL(dfa_cls_single, false, false)
+TREX_WIDE_KERNEL(dfa_cls_single_mask, false, true)

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <unordered_map>
 #include <vector>
 
 #include "runtime_internal.h"
@@ -16,6 +17,7 @@ using namespace trex;
 namespace {
 constexpr int kNfaBlock = 512;
 constexpr int kNfa5Block = 1024;   // nfa64_window5: one 1024-thread workgroup per CU holds the 104 KB of tables
+constexpr int64_t kOneLaneFrom = 160, kTwoLanesFrom = 64;   // strings per CU
 constexpr int kMaxSymbols = 62;   // (62 + 2) classes x 2 KB of nibble tables fit one workgroup's LDS
 }
 
@@ -68,14 +70,14 @@ std::vector<uint8_t> slice5_tables(const std::vector<const uint64_t*>& succ_of_c
     return out;
 }
 
-// 6/5-bit slice tables (layout of nfa64_window6): each 32-bit half of the
-// state cut into fields of 6, 6, 5, 5, 5, 5 bits; class k at byte k * kClass6,
+// 6/5-bit slice tables (layout of nfa64_window6): each 16-bit quarter of the
+// state cut into fields of 6, 5 and 5 bits; class k at byte k * kClass6,
 // field r's row at byte kRow6[r] of it, entry v = union of succ[b_r + i] over
 // the bits i of v.
 constexpr size_t kClass6 = 4096 + 8;
-constexpr int kBits6[12] = {6, 6, 5, 5, 5, 5, 6, 6, 5, 5, 5, 5};
-constexpr int kFirst6[12] = {0, 6, 12, 17, 22, 27, 32, 38, 44, 49, 54, 59};
-constexpr size_t kRow6[12] = {0, 512, 1024, 1280, 1536, 1792, 2048, 2560, 3072, 3328, 3584, 3840};
+constexpr int kBits6[12] = {6, 5, 5, 6, 5, 5, 6, 5, 5, 6, 5, 5};
+constexpr int kFirst6[12] = {0, 6, 11, 16, 22, 27, 32, 38, 43, 48, 54, 59};
+constexpr size_t kRow6[12] = {0, 512, 768, 1024, 1536, 1792, 2048, 2560, 2816, 3072, 3584, 3840};
 
 std::vector<uint8_t> slice6_tables(const std::vector<const uint64_t*>& succ_of_class) {
     std::vector<uint8_t> out(32 * kClass6, 0);
@@ -90,6 +92,41 @@ std::vector<uint8_t> slice6_tables(const std::vector<const uint64_t*>& succ_of_c
             }
     }
     return out;
+}
+
+// The automaton as a DFA over the sets it reaches, when there are at most 256
+// (state 0 is the start set): delta[n][256] and the sets. Regex automata mostly
+// are; dense random ones are given up after a few sets.
+constexpr size_t kMaxSets = 256;
+
+bool determinise(const uint64_t* succ, const int16_t* byte_to_sym, uint64_t start, std::vector<uint8_t>& delta,
+                 std::vector<uint64_t>& sets) {
+    std::unordered_map<uint64_t, int> id;
+    auto number = [&](uint64_t set) {
+        const auto it = id.emplace(set, (int)sets.size());
+        if (it.second) sets.push_back(set);
+        return it.first->second;
+    };
+    number(start);
+    for (size_t k = 0; k < sets.size(); ++k) {
+        int to[kMaxSymbols + 2];   // by symbol + 2: skip, reject, symbols
+        std::fill(to, to + kMaxSymbols + 2, -1);
+        delta.resize((k + 1) * 256);
+        for (int b = 0; b < 256; ++b) {
+            const int c = byte_to_sym[b];
+            int& t = to[c + 2];
+            if (t < 0) {
+                uint64_t next = c == -2 ? sets[k] : 0;
+                if (c >= 0)
+                    for (uint64_t rest = sets[k]; rest; rest &= rest - 1)
+                        next |= succ[(size_t)c * 64 + __builtin_ctzll(rest)];
+                t = number(next);
+                if (sets.size() > kMaxSets) return false;
+            }
+            delta[k * 256 + b] = (uint8_t)t;
+        }
+    }
+    return true;
 }
 
 }  // namespace
@@ -165,6 +202,14 @@ int trex_nfa_create(const uint64_t* succ, int n_symbols, const int16_t* byte_to_
             }
         }
     }
+    if (!rc) {
+        std::vector<uint8_t> delta, acc;
+        std::vector<uint64_t> sets;
+        if (determinise(succ, byte_to_sym, start, delta, sets)) {
+            for (uint64_t m : sets) acc.push_back((m & accept) != 0);
+            rc = make_class_form(delta.data(), acc.data(), sets.data(), (int)sets.size(), 0, &h->det);
+        }
+    }
     if (rc) { trex_nfa_destroy(h); return rc; }
     h->variant = h->d_tab6 ? TREX_NFA_WINDOW6 : h->window_base >= 0 ? TREX_NFA_WINDOW : TREX_NFA_BYTES;
     *out = h;
@@ -180,6 +225,7 @@ int trex_nfa_destroy(trex_nfa* h) {
     hipFree(h->d_cls_win);
     hipFree(h->d_tab5);
     hipFree(h->d_tab6);
+    h->det.release();
     h->in_bytes.release();
     h->in_offsets.release();
     h->out_mask.release();
@@ -202,6 +248,7 @@ int trex_nfa_set_variant(trex_nfa* h, int variant) {
     if (variant == TREX_NFA_BYTES || (variant == TREX_NFA_WINDOW && h->window_base >= 0) ||
         (variant == TREX_NFA_WINDOW5 && h->d_tab5) || (variant == TREX_NFA_WINDOW6 && h->d_tab6)) {
         h->variant = variant;
+        h->forced = true;
         return TREX_OK;
     }
     return fail(TREX_ERR_INVALID, "variant %d not usable for this automaton", variant);
@@ -213,16 +260,26 @@ int trex_nfa_match_ranges(trex_nfa* h, const uint8_t* d_bytes, const int64_t* d_
     if (n_strings < 0) return fail(TREX_ERR_INVALID, "n_strings < 0");
     if (n_strings == 0) return TREX_OK;
     if (!d_bytes || !d_begin || !d_end || !d_final_mask || !d_accept) return fail(TREX_ERR_INVALID, "null buffer");
+    if (h->det.d_tab && !h->forced)
+        return launch_class_form(h->det, d_bytes, d_begin, d_end, n_strings, false, nullptr, d_final_mask, d_accept,
+                                 (hipStream_t)stream);
     if (h->variant == TREX_NFA_WINDOW5 || h->variant == TREX_NFA_WINDOW6) {
         const bool six = h->variant == TREX_NFA_WINDOW6;
-        const int64_t grid5 = (n_strings + kNfa5Block - 1) / kNfa5Block;
-        if (grid5 > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");
         uint8_t* tab5 = six ? h->d_tab6 : h->d_tab5;
         uint32_t win4 = (uint32_t)h->window_base * 0x01010101u;
         uint64_t start = h->start, accept = h->accept;
         void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &tab5, &win4, &start, &accept, &d_final_mask, &d_accept};
-        return launch(six ? "nfa64_window6" : "nfa64_window5", (unsigned)grid5, kNfa5Block, 0, (hipStream_t)stream,
-                      args);
+        // one workgroup a CU (the tables fill its LDS), as many threads as
+        // spread the batch over all CUs; several lanes a string while that
+        // leaves a wave or so on each SIMD (measured in nfa_kernels.hip)
+        const int64_t cus = device_cu_count();
+        const int64_t lanes = !six || n_strings > cus * kOneLaneFrom ? 1 : n_strings > cus * kTwoLanesFrom ? 2 : 4;
+        const int64_t threads = (n_strings * lanes + cus - 1) / cus;
+        const unsigned block = (unsigned)std::min<int64_t>(kNfa5Block, std::max<int64_t>((threads + 63) / 64 * 64, 256));
+        const int64_t grid5 = (n_strings * lanes + block - 1) / block;
+        if (grid5 > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");
+        return launch(!six ? "nfa64_window5" : lanes == 1 ? "nfa64_window6" : lanes == 2 ? "nfa64_window6_x2" : "nfa64_window6_x4",
+                      (unsigned)grid5, block, 0, (hipStream_t)stream, args);
     }
     const int64_t grid64 = (n_strings + kNfaBlock - 1) / kNfaBlock;
     if (grid64 > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");

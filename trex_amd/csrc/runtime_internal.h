@@ -58,6 +58,28 @@ constexpr uint32_t kWaitBoundUs = 100000;
 // (each chunk walked front to back) or 2 (its two halves side by side).
 constexpr int kScanChains = 1;
 
+// Byte-class form of a byte table (dfa_class_kernels.hip); d_tab is null when
+// the table has too many classes for it.
+struct ClassForm {
+    uint8_t* d_tab = nullptr;      // tables, accept bytes, masks
+    size_t acc_at = 0, masks_at = 0;
+    int tab_bytes = 0;             // of the tables, a multiple of 16
+    int classes = 0;               // identity class included (at most 16 states)
+    int start = 0;
+    uint32_t accept = 0;           // bit s: state s accepts
+    const char* kernel = nullptr;
+    void release() { (void)hipFree(d_tab); d_tab = nullptr; }
+};
+// delta[n][256], accept[n]; masks[n] (or null): what each final state stands for.
+int make_class_form(const uint8_t* delta, const uint8_t* accept, const uint64_t* masks, int n, int start,
+                    ClassForm* out);
+// One launch over contiguous strings. Final states go to d_state, or their
+// masks to d_mask; leave_alike (at most 16 states): workgroups of alike strings
+// are left to a second launch.
+int launch_class_form(const ClassForm& f, const uint8_t* d_bytes, const int64_t* d_begin, const int64_t* d_end,
+                      int64_t n_strings, bool leave_alike, uint8_t* d_state, uint64_t* d_mask, uint8_t* d_accept,
+                      hipStream_t stream);
+
 }  // namespace trex
 
 // A resident DFA byte table (the handle behind trex_dfa_*).
@@ -73,12 +95,7 @@ struct trex_dfa {
     uint8_t* d_acc = nullptr; // [stride]
     uint8_t* d_t2 = nullptr;  // [1024][16] pair table t2[pair * 16 + s] (window variants only)
     uint8_t* d_f2 = nullptr;  // [1024] uint64 pair functions, nibble s = successor of s
-    // byte-class form (dfa_class_kernels.hip), null when the table has too many classes
-    uint8_t* d_cls = nullptr;
-    int cls_bytes = 0;        // bytes of d_cls
-    int n_classes = 0;        // classes of a form of at most 16 states, identity class included
-    const char* cls_kernel = nullptr;
-    uint32_t accept_bits = 0; // bit s: state s accepts (at most 16 states)
+    trex::ClassForm cls;      // byte-class form for contiguous strings
     bool forced = false;      // a variant was chosen by trex_dfa_set_variant
     int prefetch = 8;         // 16-byte vectors in flight per lane (8 or 16)
     int rotation = -1;        // rotated read order of contiguous strings: -1 auto, 0 off, 1 on
@@ -105,6 +122,8 @@ struct trex_nfa {
     uint8_t* d_cls_win = nullptr;   // [256]
     uint8_t* d_tab5 = nullptr;      // 32 window classes of 5-bit slice tables, class k at byte k * 3336
     uint8_t* d_tab6 = nullptr;      // 32 window classes of 6/5-bit slice tables, class k at byte k * 4104
+    trex::ClassForm det;            // the automaton as a DFA, when it reaches at most 256 sets
+    bool forced = false;            // a variant was chosen by trex_nfa_set_variant
     trex::DevBuf in_bytes, in_offsets, out_mask, out_accept;
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
