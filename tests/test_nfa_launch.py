@@ -73,3 +73,26 @@ def test_automata_of_few_sets(gpu_lib, make):
     got = _check(eng, data, offsets)
     eng.set_variant("window6")   # the bit-parallel kernels give the same sets
     assert np.array_equal(_check(eng, data, offsets), got)
+
+
+@pytest.mark.parametrize("pattern,found", [("[A-Z]*(ERROR|WARN)[A-Z]*", False), ("[A-Z]*(ERROR|WARN)[A-Z]*", True),
+                                           ("[A-Z]*A[A-Z][A-Z][A-Z][A-Z][A-Z]", True), ("([A-Z][A-Z][A-Z])*", True)],
+                         ids=["not found", "found", "last letters", "length"])
+def test_long_strings_in_short_chunks(gpu_lib, pattern, found):
+    """Few long strings are cut into chunks far below the given lengths; their
+    guesses hold always, until a word is found, or never."""
+    from trex_amd.mix import MixParams
+    from trex_amd.nfa_matrices import compile_nfa_matrices
+    rng = np.random.default_rng(8)
+    eng = NfaEngine.from_matrices(compile_nfa_matrices(pattern))
+    lengths = np.array([300_000, 0, 5, 33_000, 70_001, 512, 513])
+    offsets = np.zeros(len(lengths) + 1, np.int64)
+    np.cumsum(lengths, out=offsets[1:])
+    data = rng.choice(np.frombuffer(b"BCDFGHIJKLMPQSTUVXYZA", np.uint8), int(offsets[-1]))
+    if found:
+        for at in (150_003, 310_000):
+            data[at:at + 5] = np.frombuffer(b"ERROR", np.uint8)
+    want, _ = oracle_cpu.nfa_walk(eng.succ, eng.byte_to_sym, eng.start, eng.accept, data, offsets)
+    for params in (MixParams(), MixParams(form="slice"), MixParams(nfa_split=1 << 14, nfa_chunk=1 << 13, ck=256)):
+        mask, _, _, _ = eng.match_split(data, offsets, params)
+        assert np.array_equal(mask, want)

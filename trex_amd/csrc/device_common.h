@@ -158,6 +158,27 @@ struct Span {
     __device__ __forceinline__ uint4 last() const { return n_last ? body[full] : make_uint4(0u, 0u, 0u, 0u); }
 };
 
+// f(byte) for bytes lo .. lo + n - 1 of a vector, in order (shifted out of two
+// 64-bit words: indexing the vector would put it into scratch memory).
+template <class F>
+__device__ __forceinline__ void each_byte(const uint4& v, uint32_t lo, uint32_t n, F&& f) {
+    uint64_t a = (uint64_t)v.x | ((uint64_t)v.y << 32), b = (uint64_t)v.z | ((uint64_t)v.w << 32);
+    if (lo & 8u) {
+        a = b;
+        b = 0;
+    }
+    const uint32_t sh = 8u * (lo & 7u);
+    if (sh) {
+        a = (a >> sh) | (b << (64u - sh));
+        b >>= sh;
+    }
+    for (uint32_t i = 0; i < n; ++i) {
+        f((uint32_t)a & 255u);
+        a = (a >> 8) | (b << 56);
+        b >>= 8;
+    }
+}
+
 // As stream_blocks for contiguous strings: vectors up to the first 16 * PF
 // byte boundary (long strings only), whole blocks, the rest; the loads of each
 // go out together. Blocks that start on such a boundary touch as few cache
@@ -436,6 +457,19 @@ __device__ __forceinline__ void store_release(uint32_t* p, uint32_t v) {
 __device__ __forceinline__ void store_relaxed(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// 64-bit values written through to where every XCD reads them, and read from
+// there: with wait_stores() between them and a flag's store they are published
+// without a release (which writes back the whole L2: at a wave's rate of one a
+// microsecond that bounds launches of short chunks).
+__device__ __forceinline__ void store_through(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t load_through(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits until this wave's stores and atomics are done.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // A wait bounded twice: by a count of unsuccessful polls (max_spins, 0 = no
 // count limit) and by elapsed time on the device's constant-rate wall clock

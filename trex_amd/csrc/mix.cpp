@@ -31,6 +31,12 @@ constexpr int kMixBlockSlice = 1024;   // workgroup of mix_persistent_slice (6/5
 constexpr int kNfaClasses = 34;
 constexpr unsigned kTabSliceBytes = 32u * (4096u + 8u);   // 6/5-bit slice tables of the 32 window classes
 constexpr uint32_t kRoleDfaWhole = 0, kRoleDfaChunk = 1, kRoleNfaWhole = 2, kRoleNfaSpec = 3, kRoleNfaFixup = 4;
+// Length from which NFA chunks record checkpoints (a release per wave then costs
+// little; a chunk whose guess is wrong and that has none is walked again whole).
+constexpr int64_t kRecordFrom = 8192;
+// Bytes walked ahead of an NFA chunk for the guess of its entry set (random
+// 64-state sets coincide within some 64 bytes).
+int64_t warm_of(int64_t chunk) { return chunk >= kRecordFrom ? 256 : std::min<int64_t>(chunk, std::max<int64_t>(64, chunk / 8)); }
 constexpr int64_t kNfaWeight = 10;   // NFA-64 bytes cost about ten DFA-16 bytes (LDS lookups per byte)
 
 // Same layout as MixPattern / MixArgs in mix_kernels.hip.
@@ -43,6 +49,7 @@ struct MixPattern {
     uint32_t reserved;
     uint64_t nstart;
     uint64_t naccept;
+    uint64_t nguess;
     const uint8_t* t1;
     const uint8_t* t2;
     const uint8_t* f2;
@@ -67,10 +74,12 @@ struct MixArgs {
     const int32_t* ic;
     const uint32_t* iflags;
     int32_t n_ck;
+    int32_t warm;
     uint32_t* ticket;
     uint32_t* status;
     uint64_t* agg;
     uint32_t* done;
+    uint32_t* unmet;
     uint64_t* ckpt;
     uint64_t* spec_exit;
     uint32_t* error;
@@ -88,7 +97,7 @@ struct Plan {
     std::vector<uint32_t> iflags;
     std::vector<int32_t> bfirst, bcount, bpattern, brole;
     int64_t n_spec = 0, n_slots = 0, n_chunks = 0, n_strings = 0;
-    int32_t ck = 64, n_ck = 0;
+    int32_t ck = 64, n_ck = 0, warm = 0;
     int32_t block = kMixBlock;   // lane items per batch = workgroup size of the form planned for
 
     int32_t add(int64_t b, int64_t e, int32_t a, int32_t out, int32_t c, uint32_t flags) {
@@ -99,6 +108,14 @@ struct Plan {
         ic.push_back(c);
         iflags.push_back(flags);
         return (int32_t)(ibeg.size() - 1);
+    }
+    void reserve(size_t n) {
+        ibeg.reserve(n);
+        iend.reserve(n);
+        ia.reserve(n);
+        ib.reserve(n);
+        ic.reserve(n);
+        iflags.reserve(n);
     }
     size_t items() const { return ibeg.size(); }
 };
@@ -133,7 +150,7 @@ struct trex_mix {
     hipEvent_t staged = nullptr;   // recorded behind the last upload from h_stage
     bool staged_pending = false;
     DevBuf d_plan;
-    DevBuf d_words;   // ticket, error, converged, done[n_slots], status[n_items]
+    DevBuf d_words;   // ticket, error, converged, done[n_slots], unmet[n_slots], status[n_items]
     DevBuf d_agg, d_ckpt, d_exit;
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -199,8 +216,8 @@ int stage_plan(trex_mix* m) {
         if (sizes[i]) std::memcpy(m->h_stage + m->off[i], srcs[i], sizes[i]);
     m->plan_bytes = total;
     m->need[0] = total;
-    m->need[1] = 4 * (3 + (size_t)Q.n_slots + Q.items());
-    m->need[2] = 8 * std::max<size_t>(Q.items(), 1);
+    m->need[1] = 4 * (3 + 2 * (size_t)Q.n_slots + Q.items());
+    m->need[2] = 16 * std::max<size_t>(Q.items(), 1);
     m->need[3] = 8 * std::max<size_t>((size_t)Q.n_spec * Q.n_ck, 1);
     m->need[4] = 8 * std::max<size_t>((size_t)Q.n_spec, 1);
     m->dirty = true;
@@ -218,6 +235,46 @@ int upload_plan(trex_mix* m, hipStream_t s) {
     m->staged_pending = true;
     m->dirty = false;
     return TREX_OK;
+}
+
+}  // namespace
+
+namespace {
+
+// Split and chunk lengths of a batch too small to fill the chip at the given
+// ones: every lane walks its string or chunk alone, so a batch lasts at least
+// as long as one chunk (a 32 KiB NFA chunk: 3 to 7 ms), however little there is
+// of it. Chunks become as short as gives every CU kLanesPerCu lanes of either
+// kind, within the lengths below and the given ones; a batch that fills the
+// chip keeps the given ones, and so do callers that ask for short ones
+// themselves (kTakenAsGiven). True when something became shorter. 16 patterns,
+// 1,024 strings of 32 B to 1 MiB (101 MB): 8.3 ms at 32 / 64 KiB, 345 us at
+// 1 KiB NFA chunks, 278 us at 512 B, 296 us at 256 B.
+constexpr int64_t kLanesPerCu = 512;
+constexpr int64_t kBatchesPerCu = 2;
+constexpr int64_t kTakenAsGiven = 4096;
+constexpr int64_t kLeastNfaChunk = 512, kLeastDfaChunk = 1024;
+
+bool refine(const trex_mix* m, const int64_t* begin, const int64_t* end, const int32_t* pattern_of, int64_t n_strings,
+            int32_t ck, int64_t& dfa_split, int64_t& dfa_chunk, int64_t& nfa_split, int64_t& nfa_chunk) {
+    int64_t bytes[2] = {0, 0};
+    for (int64_t i = 0; i < n_strings; ++i)
+        bytes[m->kinds[pattern_of[i]] == TREX_MIX_NFA ? 1 : 0] += end[i] - begin[i];
+    const int64_t lanes = kLanesPerCu * device_cu_count();
+    auto up = [](int64_t x, int64_t step) { return (x + step - 1) / step * step; };
+    const int64_t dfa = up(std::max(bytes[0] / lanes, kLeastDfaChunk), 16);
+    const int64_t nfa = up(std::max(bytes[1] / lanes, kLeastNfaChunk), ck);
+    bool finer = false;
+    auto cut = [&](int64_t& length, int64_t to) {
+        if (length <= kTakenAsGiven || length <= to) return;
+        length = to;
+        finer = true;
+    };
+    cut(dfa_chunk, dfa);
+    cut(dfa_split, std::max(dfa, std::min(dfa_chunk, dfa_split)));
+    cut(nfa_chunk, nfa);
+    cut(nfa_split, std::max(nfa, std::min(nfa_chunk, nfa_split)));
+    return finer;
 }
 
 }  // namespace
@@ -261,6 +318,7 @@ int trex_mix_create(const int32_t* kinds, const void* const* handles, int32_t n_
                 P.win4 = (uint32_t)f->window_base * 0x01010101u;
                 P.nstart = f->start;
                 P.naccept = f->accept;
+                P.nguess = f->guess;
                 P.ntab = reinterpret_cast<const uint8_t*>(f->d_tab_win);
                 P.ncls = f->d_cls_win;
             }
@@ -323,10 +381,13 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
     drop_graph(m);
     Plan P;
     P.block = m->form == TREX_MIX_FORM_SLICE ? kMixBlockSlice : kMixBlock;
-    P.ck = ck;
-    P.n_ck = (int32_t)(nfa_chunk / ck);
-    P.n_strings = n_strings;
     const int32_t np = m->n_patterns;
+    const bool finer = m->has_device && refine(m, begin, end, pattern_of, n_strings, ck, dfa_split, dfa_chunk,
+                                               nfa_split, nfa_chunk);
+    P.ck = ck;
+    P.n_ck = nfa_chunk >= kRecordFrom ? (int32_t)(nfa_chunk / ck) : 0;
+    P.warm = (int32_t)warm_of(nfa_chunk);
+    P.n_strings = n_strings;
 
     // strings per pattern, split into whole and long
     std::vector<std::vector<int32_t>> whole(np), longs(np);
@@ -336,11 +397,26 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
         const int64_t split = m->kinds[p] == TREX_MIX_DFA ? dfa_split : nfa_split;
         (len > split ? longs : whole)[p].push_back((int32_t)i);
     }
+    int64_t lanes = 0, fixups = 0;   // whole strings and chunks; strings with a fix-up
+    for (int32_t p = 0; p < np; ++p) {
+        const bool dfa = m->kinds[p] == TREX_MIX_DFA;
+        const int64_t chunk = dfa ? dfa_chunk : nfa_chunk;
+        lanes += (int64_t)whole[p].size();
+        for (int32_t sid : longs[p]) lanes += (end[sid] - begin[sid] + chunk - 1) / chunk;
+        if (!dfa) fixups += (int64_t)longs[p].size();
+    }
+    P.reserve((size_t)(lanes + fixups));
+    // lanes per batch: a workgroup's, or fewer when that would leave CUs without a batch
+    int32_t most = P.block;
+    if (m->has_device) {
+        const int64_t share = lanes / (kBatchesPerCu * device_cu_count());
+        most = (int32_t)std::min<int64_t>(P.block, std::max<int64_t>((share + 63) / 64 * 64, 64));
+    }
     std::vector<BatchRef> spec_b, chunk_b, fix_b, whole_b;
     auto cut = [&](int32_t first, int32_t n, int32_t pat, int32_t role, std::vector<BatchRef>& out,
                    const std::vector<int64_t>& keys) {
-        for (int32_t o = 0; o < n; o += P.block)
-            out.push_back({first + o, std::min(P.block, n - o), pat, role, keys.empty() ? 0 : keys[o]});
+        for (int32_t o = 0; o < n; o += most)
+            out.push_back({first + o, std::min(most, n - o), pat, role, keys.empty() ? 0 : keys[o]});
     };
 
     // 1. NFA speculative chunks: each long string's chunks contiguous
@@ -376,7 +452,10 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
             const int64_t n = (end[sid] - begin[sid] + dfa_chunk - 1) / dfa_chunk;
             for (int64_t k = 0; k < n; ++k) cs.push_back({sid, k});
         }
-        std::stable_sort(cs.begin(), cs.end(), [](const C& a, const C& b) { return a.k < b.k; });
+        // in chunk-position order, so that a chunk's predecessor is long done; a
+        // batch of short chunks keeps each string's chunks together instead:
+        // they all run at once, and a wave resolves its own in registers
+        if (!finer) std::stable_sort(cs.begin(), cs.end(), [](const C& a, const C& b) { return a.k < b.k; });
         const int32_t first = (int32_t)P.items();
         std::vector<int64_t> keys;
         // the predecessor of chunk k is the item of chunk k - 1, placed earlier
@@ -387,7 +466,7 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
             const bool last = e == end[c.sid];
             const int32_t it = P.add(b, e, c.k == 0 ? -1 : latest[c.sid], last ? c.sid : -1, 0, c.k == 0 ? 1u : 0u);
             latest[c.sid] = it;
-            keys.push_back(c.k);
+            keys.push_back(finer ? 0 : c.k);
         }
         P.n_chunks += (int32_t)P.items() - first;
         cut(first, (int32_t)P.items() - first, p, kRoleDfaChunk, chunk_b, keys);
@@ -473,7 +552,7 @@ int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint
     hipStream_t s = (hipStream_t)stream;
     TREX_TRY(upload_plan(m, s));
     uint32_t* words = m->d_words.as<uint32_t>();
-    int64_t n_words = 3 + Q.n_slots + (int64_t)Q.items();
+    int64_t n_words = 3 + 2 * Q.n_slots + (int64_t)Q.items();
     uint32_t zero = 0;
     {
         const unsigned grid = (unsigned)std::min<int64_t>((n_words + kBlock - 1) / kBlock, 4096);
@@ -498,11 +577,13 @@ int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint
     a.n_batches = (int32_t)Q.bfirst.size();
     a.ck = Q.ck;
     a.n_ck = Q.n_ck;
+    a.warm = Q.warm;
     a.ticket = words;
     a.error = words + 1;
     a.converged = words + 2;
     a.done = words + 3;
-    a.status = words + 3 + Q.n_slots;
+    a.unmet = a.done + Q.n_slots;
+    a.status = a.unmet + Q.n_slots;
     a.agg = m->d_agg.as<uint64_t>();
     a.ckpt = m->d_ckpt.as<uint64_t>();
     a.spec_exit = m->d_exit.as<uint64_t>();

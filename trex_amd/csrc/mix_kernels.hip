@@ -14,15 +14,20 @@
 //   NFA_WHOLE  a string walked by the bit-parallel NFA-64 step
 //   NFA_SPEC   one chunk of a long string: the first chunk of the string is
 //              walked from the start set; every other chunk is walked from
-//              the set of all states (a guess) and records its state set
-//              every kCk bytes (checkpoints) and at its end
+//              the pattern's guess set `warm` bytes ahead of it, which makes a
+//              guess of the set it is entered with, and on to its end. The
+//              guess is right when the chunk before it ends in that set (taken
+//              from the neighbouring lane, or published by the wave before)
+//              and was entered with the right set itself. Long chunks also
+//              record their set every kCk bytes (checkpoints)
 //   NFA_FIXUP  one lane per long string, after all its NFA_SPEC chunks are
-//              done: walks each chunk again from the true entry set until the
-//              set equals the chunk's checkpoint at the same position, after
-//              which both walks coincide, so the chunk's exit is the recorded
-//              one. A chunk that never meets its checkpoints is walked to its
-//              end, and an empty set ends the fix-up (the empty set is
-//              absorbing). The result is exact either way.
+//              done: when every guess was its predecessor's end, the last end
+//              is the string's. Otherwise it goes from chunk to chunk: where
+//              the true set is the guess, the chunk's end is known; any other
+//              chunk is walked again from the true set, with checkpoints only
+//              until the set equals the one recorded at the same position,
+//              after which both walks coincide. An empty set ends it (the
+//              empty set is absorbing). The result is exact either way.
 //
 // Forward progress: the queue puts every batch that is waited on before the
 // batches that wait on it (DFA chunks after their predecessors, fix-ups after
@@ -30,7 +35,8 @@
 // workgroup, and no waited-on work waits itself. A DFA chunk never waits on
 // a chunk of its own wave (those come by shuffle). Waits are bounded by a
 // poll count (max_spins) and by wall-clock ticks (max_ticks); on expiry the
-// error word is set and the wave moves on.
+// error word is set and the wave moves on (a NFA_SPEC lane that does not see
+// the end set before it in time leaves its chunk to the fix-up, no error).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -47,6 +53,7 @@ using namespace trexdev;
 constexpr uint32_t kRoleDfaWhole = 0, kRoleDfaChunk = 1, kRoleNfaWhole = 2, kRoleNfaSpec = 3, kRoleNfaFixup = 4;
 constexpr uint32_t kStatusAggregate = 1u, kStatusPrefix = 2u;
 constexpr int kNfaClasses = 34;   // window bytes 0..31, reject, skip
+constexpr int kFixupBlock = 4;    // chunks a fix-up reads at once
 
 // Pattern descriptor (host layout in mix.cpp).
 struct MixPattern {
@@ -58,6 +65,7 @@ struct MixPattern {
     uint32_t reserved;
     uint64_t nstart;      // NFA start set
     uint64_t naccept;     // NFA accept set
+    uint64_t nguess;      // NFA set a chunk's guess is walked from
     const uint8_t* t1;    // DFA byte table [256][16]
     const uint8_t* t2;    // DFA pair rows [1024][16]
     const uint8_t* f2;    // DFA pair functions [1024] x uint64
@@ -81,15 +89,17 @@ struct MixArgs {
     const int32_t* ib;        // item: output string, -1 if none
     const int32_t* ic;        // item: NFA_SPEC checkpoint ordinal
     const uint32_t* iflags;   // item: bit 0 first chunk of its string
-    int32_t n_ck;             // checkpoints per NFA_SPEC item
+    int32_t n_ck;             // checkpoints per NFA_SPEC item, 0: none recorded
+    int32_t warm;             // bytes walked ahead of a NFA_SPEC chunk for its guess (at most a chunk)
     uint32_t* ticket;
-    uint32_t* status;         // per item (DFA_CHUNK)
-    uint64_t* agg;            // per item (DFA_CHUNK)
+    uint32_t* status;         // per item (DFA_CHUNK; NFA_SPEC: 1 once its end is published)
+    uint64_t* agg;            // two words per item (DFA_CHUNK: function, item to go on from; NFA_SPEC: guess)
     uint32_t* done;           // per NFA string slot: finished NFA_SPEC chunks
+    uint32_t* unmet;          // per NFA string slot: chunks whose guess is not their predecessor's end
     uint64_t* ckpt;           // [n_spec][n_ck]
     uint64_t* spec_exit;      // [n_spec]
     uint32_t* error;
-    uint32_t* converged;      // fix-up chunks that met a checkpoint
+    uint32_t* converged;      // chunks whose end the fix-ups took as recorded
     uint32_t max_spins;       // wait bound in polls (0: none)
     uint32_t reserved;
     uint64_t max_ticks;       // wait bound in wall-clock ticks
@@ -118,20 +128,20 @@ __device__ __forceinline__ uint32_t k2f_word(const uint64_t* __restrict__ f2, ui
 __device__ uint32_t dfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, const DfaLds& L,
                              const MixPattern& P) {
     uint32_t s = P.start;
-    const int64_t head_end = min(end, p + head_len(bytes, p));
-    for (; p < head_end; ++p) s = L.t1[((uint32_t)bytes[p] << 4) | s];
+    const Span sp(bytes, p, end);
+    const uint4 first = sp.first(), last = sp.last();
+    auto byte = [&](uint32_t b) { s = L.t1[(b << 4) | s]; };
+    each_byte(first, sp.lo, sp.n_first, byte);
     WinCheck w;
     w.init();
-    const int64_t nvec = (end - p) >> 4;
-    stream_body<8>(reinterpret_cast<const uint4*>(bytes + p), nvec, [&](uint4 v) {
+    stream_body<8>(sp.body, sp.full, [&](uint4 v) {
         w.add(v.x); w.add(v.y); w.add(v.z); w.add(v.w);
         s = k2f_word(L.f2, s, v.x);
         s = k2f_word(L.f2, s, v.y);
         s = k2f_word(L.f2, s, v.z);
         s = k2f_word(L.f2, s, v.w);
     });
-    p += nvec << 4;
-    for (; p < end; ++p) s = L.t1[((uint32_t)bytes[p] << 4) | s];
+    each_byte(last, 0u, sp.n_last, byte);
     if (w.outside(P.win4)) s = P.dead;
     return s;
 }
@@ -197,13 +207,12 @@ __device__ __forceinline__ void dfa_chunk(const MixArgs& A, const MixPattern& P,
     sc.walking = pred < 0;
     sc.s = P.start;
     sc.f = fn_identity_on(P.nstates);
-    const uint8_t* bytes = A.bytes;
-    const int64_t head_end = min(end, p + head_len(bytes, p));
-    for (; p < head_end; ++p) sc.byte(bytes[p]);
-    const int64_t nvec = (end - p) >> 4;
-    stream_body<4>(reinterpret_cast<const uint4*>(bytes + p), nvec, [&](const uint4& a) { sc.vector(a); });
-    p += nvec << 4;
-    for (; p < end; ++p) sc.byte(bytes[p]);
+    const Span sp(A.bytes, p, end);
+    const uint4 first = sp.first(), last = sp.last();
+    auto byte = [&](uint32_t b) { sc.byte(b); };
+    each_byte(first, sp.lo, sp.n_first, byte);
+    stream_body<4>(sp.body, sp.full, [&](const uint4& a) { sc.vector(a); });
+    each_byte(last, 0u, sp.n_last, byte);
     sc.settle();
     if (sc.w.outside(P.win4)) { sc.walking = true; sc.s = P.dead; }
 
@@ -216,8 +225,7 @@ __device__ __forceinline__ void dfa_chunk(const MixArgs& A, const MixPattern& P,
     const uint32_t lane = threadIdx.x & 63u;
     const int64_t wave_first = item - (int64_t)lane;
     const bool own_known = pred < 0 || sc.walking;
-    const Fn16 own = own_known ? fn_const(sc.s) : sc.f;
-    Fn16 g = own;
+    Fn16 g = own_known ? fn_const(sc.s) : sc.f;
     const bool inwave = active && (int64_t)pred >= wave_first;
     uint32_t root = inwave ? (uint32_t)((int64_t)pred - wave_first) : lane;
     bool closed = !inwave;
@@ -238,15 +246,18 @@ __device__ __forceinline__ void dfa_chunk(const MixArgs& A, const MixPattern& P,
     }
 
     // A chunk whose chain function is constant knows its final state and
-    // publishes PREFIX at once; any other publishes its own chunk's function
-    // (a look-back from another wave steps chunk by chunk over A.ia).
+    // publishes PREFIX at once; any other publishes the function of its chain
+    // up to here and the predecessor of the chain's root, where a look-back
+    // that meets it goes on (one step per wave of a string's chunks).
+    const int32_t root_pred = __shfl(pred, (int)root, 64);
     const bool known = fn_is_const(g);
     const uint32_t kstate = g.d[0] & 0xffu;
     if (active) {
         if (known) {
             store_relaxed(&A.status[item], kStatusPrefix | (kstate << 8));   // the word says it all
         } else {
-            A.agg[item] = fn_pack(own);
+            A.agg[2 * item] = fn_pack(g);
+            A.agg[2 * item + 1] = (uint64_t)(int64_t)root_pred;
             store_release(&A.status[item], kStatusAggregate);   // agg first
         }
     }
@@ -271,8 +282,8 @@ __device__ __forceinline__ void dfa_chunk(const MixArgs& A, const MixPattern& P,
                 break;
             }
             fence_acquire();   // agg[j] was written before status[j] was released
-            acc_fn = nib_then(A.agg[j], acc_fn);   // the earlier chunk applies first
-            j = (A.iflags[j] & 1u) ? -1 : A.ia[j];
+            acc_fn = nib_then(A.agg[2 * (int64_t)j], acc_fn);   // the earlier chunks apply first
+            j = (int32_t)(int64_t)A.agg[2 * (int64_t)j + 1];
             if (j < 0) {   // cannot happen: a string's first chunk publishes a prefix
                 atomicOr(A.error, 2u);
                 incoming = P.dead;
@@ -337,42 +348,74 @@ __device__ uint64_t nfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64
                              const void* tab, const uint8_t* cls, uint32_t win4) {
     NfaWalker<SLICE> nw{tab, cls, s, {}};
     nw.w.init();
-    const int64_t head_end = min(end, p + head_len(bytes, p));
-    for (; p < head_end; ++p) nw.byte(bytes[p]);
-    const int64_t nvec = (end - p) >> 4;
-    stream_body<2>(reinterpret_cast<const uint4*>(bytes + p), nvec, [&](uint4 x) { nw.vec(x); });
+    const Span sp(bytes, p, end);
+    const uint4 first = sp.first(), last = sp.last();
+    auto byte = [&](uint32_t b) { nw.byte(b); };
+    each_byte(first, sp.lo, sp.n_first, byte);
+    stream_body<2>(sp.body, sp.full, [&](uint4 x) { nw.vec(x); });
     nw.settle(win4);
-    p += nvec << 4;
-    for (; p < end; ++p) nw.byte(bytes[p]);
+    each_byte(last, 0u, sp.n_last, byte);
     nw.settle(win4);
     return nw.s;
 }
 
-// Walks [p, end) from set s. When `record`, stores the set at every absolute
-// position that is a multiple of ck (ck a multiple of 16) into ck_out[0..n_ck).
-// When `compare`, stops at the first such position whose set equals
-// ck_in[idx] and reports it through `met`.
-template <bool SLICE, bool RECORD, bool COMPARE>
-__device__ uint64_t nfa_walk_ck(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
-                                const void* tab, const uint8_t* cls, uint32_t win4, int32_t ck,
-                                uint64_t* __restrict__ ck_out, const uint64_t* __restrict__ ck_in, int32_t n_ck,
-                                bool& met) {
+// Walks [p, end) from set s and stores the set at every absolute position that
+// is a multiple of ck (ck a multiple of 16) into ck_out[0..n_ck); n_ck = 0
+// stores none.
+template <bool SLICE>
+__device__ uint64_t nfa_walk_record(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
+                                    const void* tab, const uint8_t* cls, uint32_t win4, int32_t ck,
+                                    uint64_t* __restrict__ ck_out, int32_t n_ck) {
+    NfaWalker<SLICE> nw{tab, cls, s, {}};
+    nw.w.init();
+    const Span sp(bytes, p, end);
+    const uint4 first = sp.first(), last = sp.last();
+    auto byte = [&](uint32_t b) { nw.byte(b); };
+    each_byte(first, sp.lo, sp.n_first, byte);
+    p += sp.n_first;
+    // vectors to the first multiple of ck after p (positions off the vectors'
+    // grid meet none), then ck / 16 at a time; no division per vector
+    const int64_t to_ck = (p + 16 + ck - 1) / ck * ck - p;
+    int32_t left = n_ck > 0 && (to_ck & 15) == 0 ? (int32_t)(to_ck >> 4) : 0;
+    int32_t idx = 0;
+    stream_body<2>(sp.body, sp.full, [&](const uint4& x) {
+        nw.vec(x);
+        if (--left == 0) {
+            left = ck >> 4;
+            if (idx < n_ck) {
+                nw.settle(win4);
+                ck_out[idx++] = nw.s;
+            }
+        }
+    });
+    nw.settle(win4);
+    each_byte(last, 0u, sp.n_last, byte);
+    nw.settle(win4);
+    return nw.s;
+}
+
+// Walks [p, end) from set s and stops at the first multiple of ck whose set
+// equals ck_in[idx] (as nfa_walk_record stored them), reported through `met`.
+template <bool SLICE>
+__device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
+                                  const void* tab, const uint8_t* cls, uint32_t win4, int32_t ck,
+                                  const uint64_t* __restrict__ ck_in, int32_t n_ck, bool& met) {
     NfaWalker<SLICE> nw{tab, cls, s, {}};
     nw.w.init();
     met = false;
-    const int64_t head_end = min(end, p + head_len(bytes, p));
-    for (; p < head_end; ++p) nw.byte(bytes[p]);
+    const Span sp(bytes, p, end);
+    const uint4 first = sp.first(), last = sp.last();
+    auto byte = [&](uint32_t b) { nw.byte(b); };
+    each_byte(first, sp.lo, sp.n_first, byte);
+    p += sp.n_first;
     int32_t idx = 0;
-    const uint4* v = reinterpret_cast<const uint4*>(bytes + p);
-    const int64_t nvec = (end - p) >> 4;
+    const uint4* v = sp.body;
+    const int64_t nvec = sp.full;
     // two vectors in flight ahead of the one being walked (a walk that stops
     // at a checkpoint drops them)
     uint4 n0 = make_uint4(0u, 0u, 0u, 0u), n1 = n0;
     if (nvec > 0) n0 = v[0];
     if (nvec > 1) n1 = v[1];
-    // the first multiple of ck after p; positions advance by 16 and ck is a
-    // multiple of 16, so pos meets every later one exactly (no division per
-    // vector)
     int64_t next_ck = (p + 16 + ck - 1) / ck * ck;
     for (int64_t i = 0; i < nvec; ++i) {
         const uint4 cur = n0;
@@ -384,19 +427,15 @@ __device__ uint64_t nfa_walk_ck(const uint8_t* __restrict__ bytes, int64_t p, in
         next_ck += ck;
         if (idx < n_ck) {
             nw.settle(win4);
-            if constexpr (RECORD) ck_out[idx] = nw.s;
-            if constexpr (COMPARE) {
-                if (nw.s == ck_in[idx]) {
-                    met = true;
-                    return nw.s;
-                }
+            if (nw.s == ck_in[idx]) {
+                met = true;
+                return nw.s;
             }
             ++idx;
         }
     }
     nw.settle(win4);
-    p += nvec << 4;
-    for (; p < end; ++p) nw.byte(bytes[p]);
+    each_byte(last, 0u, sp.n_last, byte);
     nw.settle(win4);
     return nw.s;
 }
@@ -465,13 +504,55 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
         } else if (role == kRoleNfaSpec) {
             const bool first = (A.iflags[item] & 1u) != 0;
             const int32_t o = A.ic[item];
+            const int64_t p = A.ibeg[item], end = A.iend[item];
             bool met;
-            const uint64_t s = nfa_walk_ck<SLICE, true, false>(A.bytes, A.ibeg[item], A.iend[item],
-                                                            first ? P.nstart : ~0ull, ntab, ncls, P.win4, A.ck,
-                                                            A.ckpt + (int64_t)o * A.n_ck, nullptr, A.n_ck, met);
-            A.spec_exit[o] = s;
-            __threadfence();
-            atomicAdd(&A.done[A.ia[item]], 1u);
+            uint64_t guess = 0, s = first ? P.nstart : P.nguess;
+#pragma unroll 1
+            for (int part = 0; part < 2; ++part) {   // the bytes ahead, then the chunk: one copy of the walk
+                const int64_t from = part == 0 && !first ? p - A.warm : p;
+                if (part == 1) guess = s;
+                s = nfa_walk_record<SLICE>(A.bytes, from, part ? end : p, s, ntab, ncls, P.win4, A.ck,
+                                           A.ckpt + (int64_t)o * A.n_ck, part ? A.n_ck : 0);
+            }
+            store_through(&A.spec_exit[o], s);
+            store_through(&A.agg[2 * item], guess);
+            // the chunk before this one is the item before it: the lane below,
+            // or the last lane of the wave before (of this batch or an earlier
+            // one), which publishes before it waits itself
+            const uint32_t lane = threadIdx.x & 63u;
+            if (A.n_ck) __threadfence();   // checkpoints are ordinary stores
+            wait_stores();
+            if (lane == 63u || (int32_t)threadIdx.x == count - 1) store_relaxed(&A.status[item], 1u);
+            uint64_t before = (uint64_t)(uint32_t)__shfl_up((int)(uint32_t)s, 1, 64) |
+                              ((uint64_t)(uint32_t)__shfl_up((int)(uint32_t)(s >> 32), 1, 64) << 32);
+            met = first || lane > 0u;
+            if (!met) {
+                BoundedWait wait(A.max_spins, A.max_ticks);
+                while (!(met = load_relaxed(&A.status[item - 1]) != 0u) && !wait.expired())
+                    __builtin_amdgcn_s_sleep(2);
+                before = load_through(&A.spec_exit[o - 1]);
+                if (!met) atomicOr(A.error, 4u);
+            }
+            met = met && (first || before == guess);
+            // one atomic per string and wave (they are served one after another,
+            // about 70 ns each: one per chunk of a long string adds up)
+            wait_stores();
+            const int32_t slot = A.ia[item];
+            bool left = true;
+            for (uint64_t todo; (todo = __ballot(left)) != 0ull;) {
+                const int32_t of = __shfl(slot, (int)__builtin_ctzll(todo), 64);
+                const uint64_t mine = __ballot(left && slot == of), un = __ballot(left && slot == of && !met);
+                if (left && slot == of) {
+                    if (lane == (uint32_t)__builtin_ctzll(mine)) {
+                        if (un) {
+                            atomicAdd(&A.unmet[of], (uint32_t)__popcll(un));
+                            wait_stores();
+                        }
+                        atomicAdd(&A.done[of], (uint32_t)__popcll(mine));
+                    }
+                    left = false;
+                }
+            }
         } else if (role == kRoleNfaFixup) {
             const int64_t c0 = A.ibeg[item], c1 = A.iend[item];
             const uint32_t need = (uint32_t)(c1 - c0);
@@ -485,20 +566,53 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
                 }
                 __builtin_amdgcn_s_sleep(8);
             }
-            fence_acquire();   // checkpoints and exits were written before each chunk counted itself
             uint64_t s = 0;
-            if (ok) {
-                s = A.spec_exit[A.ic[c0]];   // the first chunk was walked from the start set
-                // the empty set is absorbing: once the true set is empty, so are all later exits
-                for (int64_t c = c0 + 1; c < c1 && s != 0; ++c) {
-                    const int32_t o = A.ic[c];
-                    bool met;
-                    const uint64_t t = nfa_walk_ck<SLICE, false, true>(A.bytes, A.ibeg[c], A.iend[c], s, ntab, ncls,
-                                                                    P.win4, A.ck, nullptr,
-                                                                    A.ckpt + (int64_t)o * A.n_ck, A.n_ck, met);
-                    s = met ? A.spec_exit[o] : t;
-                    if (met) atomicAdd(A.converged, 1u);
+            uint32_t converged = 0;
+            if (ok) {   // guesses and ends were written through before each chunk counted itself
+                if (A.n_ck) fence_acquire();
+                const int32_t o0 = A.ic[c0];
+                s = load_through(&A.spec_exit[o0]);   // the first chunk was walked from the start set
+                int64_t from = c0 + 1;
+                if (load_relaxed(&A.unmet[A.ia[item]]) == 0u) {
+                    converged = (uint32_t)(c1 - from);
+                    s = load_through(&A.spec_exit[o0 + (c1 - 1 - c0)]);
+                    from = c1;
                 }
+                // the empty set is absorbing: once the true set is empty, so are all later exits
+                for (int64_t c = from; c < c1 && s != 0; c += kFixupBlock) {
+                    // guesses and ends of the next chunks (items and ordinals of a string are
+                    // consecutive), read together
+                    uint64_t ends[kFixupBlock], guesses[kFixupBlock];
+#pragma unroll
+                    for (int k = 0; k < kFixupBlock; ++k) {
+                        const int64_t j = min(c + k, c1 - 1);
+                        ends[k] = load_through(&A.spec_exit[o0 + (j - c0)]);
+                        guesses[k] = load_through(&A.agg[2 * j]);
+                    }
+                    bool known = true;   // all of them entered as guessed
+                    uint64_t t = s;
+#pragma unroll
+                    for (int k = 0; k < kFixupBlock; ++k) {
+                        known = known && (c + k >= c1 || t == guesses[k]);
+                        if (c + k < c1) t = ends[k];
+                    }
+                    if (known) {
+                        s = t;
+                        converged += (uint32_t)min<int64_t>(kFixupBlock, c1 - c);
+                        continue;
+                    }
+                    for (int64_t j = c; j < min(c + kFixupBlock, c1) && s != 0; ++j) {
+                        const int64_t o = o0 + (j - c0);
+                        const uint64_t stop = load_through(&A.spec_exit[o]);
+                        bool met = s == load_through(&A.agg[2 * j]);
+                        if (!met)
+                            s = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], s, ntab, ncls, P.win4, A.ck,
+                                                     A.ckpt + o * A.n_ck, A.n_ck, met);
+                        if (met) s = stop;
+                        converged += met ? 1u : 0u;
+                    }
+                }
+                atomicAdd(A.converged, converged);
             }
             A.out_mask[A.ib[item]] = s;
             A.out_accept[A.ib[item]] = (s & P.naccept) != 0 ? 1 : 0;

@@ -148,6 +148,11 @@ int trex_nfa_create(const uint64_t* succ, int n_symbols, const int16_t* byte_to_
     h->n_symbols = n_symbols;
     h->start = start;
     h->accept = accept;
+    for (int s = 0; s < 64 && n_symbols > 0; ++s) {
+        bool kept = ((start >> s) & 1u) == 0;
+        for (int c = 0; c < n_symbols && kept; ++c) kept = (succ[(size_t)c * 64 + s] >> s) & 1u;
+        if (kept) h->guess = start;
+    }
     const int reject = n_symbols, skip = n_symbols + 1;
     h->n_classes = n_symbols + 2;
     std::vector<uint64_t> ident(64), none(64, 0);

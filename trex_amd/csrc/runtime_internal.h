@@ -113,6 +113,10 @@ struct trex_dfa {
 struct trex_nfa {
     int n_symbols = 0;
     uint64_t start = 0, accept = 0;
+    // what walks of later chunks of a string start from: all states, or the start
+    // set for automata that keep a state outside it once it is reached (a text
+    // found stays found): from all states such a state is never lost again
+    uint64_t guess = ~0ull;
     int window_base = -1;
     int variant = TREX_NFA_BYTES;
     int n_classes = 0, n_classes_win = 0;
