@@ -8,7 +8,7 @@ from oracle import cpu as ocpu
 from oracle.dfa import table_walk_one
 from oracle.scan import lookback_final_state, plan_chunks, wave_protocol
 from trex_amd.regex_to_dfa import compile_regex
-from trex_amd.tables import dfa_byte_table
+from trex_amd.tables import DfaByteTable, dfa_byte_table
 from trex_amd.workloads import ALPHABET_32, random_dfa_pattern, ragged_batch
 
 EVEN_A = "(b*ab*ab*)*b*"
@@ -458,3 +458,65 @@ def test_synchronizes_and_chunk_target():
                     img.add(s)
                 found |= len(img) == 1
         assert found == sync, rx
+
+
+def _table(rng, n_states, byte_lo, n_bytes, dead, pure=False):
+    """A random byte table of n_states states over n_bytes byte values from
+    byte_lo; with `dead`, the last state is dead and every other byte leads
+    there, else every other byte leaves the state as it is. `pure`: each byte
+    permutes the live states, so no run of bytes makes a chunk constant."""
+    live = n_states - 1 if dead else n_states
+    delta = np.tile(np.arange(n_states, dtype=np.uint8), (256, 1)).T.copy()
+    if dead:
+        delta[:live] = live
+    for b in range(byte_lo, byte_lo + n_bytes):
+        delta[:live, b] = rng.permutation(live) if pure else rng.integers(0, live, live)
+    accept = rng.integers(0, 2, n_states).astype(np.uint8)
+    if dead:
+        accept[live] = 0
+    return delta, accept
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_bytes", [26, 60], ids=["window", "bytes"])
+@pytest.mark.parametrize("n_states,dead,pure", [(2, True, False), (8, True, False), (8, False, True), (9, True, False),
+                                                (9, True, True), (16, True, False), (16, False, False)])
+def test_plan_dead_strings(gpu_lib, n_states, dead, pure, n_bytes):
+    """Strings that die in their first, a middle or their last chunk, at either
+    end of it, next to ones that do not, with at most eight states and with
+    more, with a dead state and without one: a plan run twice and from begin
+    offsets of every alignment, both engines on the one plan, gives the walk."""
+    from trex_amd.device import DeviceBuffer
+    from trex_amd.engine import ChunkPlan, DfaEngine
+    rng = np.random.default_rng(n_states * 8 + dead * 4 + pure * 2 + (n_bytes > 32))
+    chunk = 256
+    tabs = [_table(rng, n_states, 0x41, n_bytes, dead, pure), _table(rng, 5, 0x41, 26, True)]
+    lengths = [0, 1, 15, 16, 17, chunk - 1, chunk, chunk + 1] + [5 * chunk + r for r in range(24)]
+    begin, end, at = [], [], 0
+    for k, n in enumerate(lengths * 2):
+        at += k % 17
+        begin.append(at)
+        at += n
+        end.append(at)
+    begin, end = np.array(begin, np.int64), np.array(end, np.int64)
+    data = rng.integers(0x41, 0x41 + 26, at + 16).astype(np.uint8)
+    for k in range(0, len(begin), 2):
+        n = end[k] - begin[k]
+        if n:
+            where = [0, n - 1, n // 2, min(chunk, n - 1), min(chunk, n) - 1][(k // 2) % 5]
+            data[begin[k] + where] = 0x7e
+    d = DeviceBuffer(data.nbytes)
+    d.upload(data)
+    plan = ChunkPlan(begin, end, chunk)
+    out = DeviceBuffer(len(begin)), DeviceBuffer(len(begin))
+    engines = [DfaEngine(DfaByteTable(t, a, 0, -1, len(a))) for t, a in tabs]
+    for _ in range(2):
+        for eng, (delta, accept) in zip(engines, tabs):
+            eng.match_plan(plan, d.ptr, out[0].ptr, out[1].ptr)
+            assert plan.error() == 0
+            f, a = (o.download(np.uint8, len(begin)) for o in out)
+            for k in range(len(begin)):
+                s = 0
+                for b in data[begin[k]:end[k]]:
+                    s = delta[s, b]
+                assert (f[k], a[k]) == (s, accept[s]), (k, int(end[k] - begin[k]))

@@ -402,6 +402,75 @@ __device__ __forceinline__ uint64_t fn_pack(const Fn16& f) {
     return out;
 }
 
+__device__ __forceinline__ Fn16 load_row(const uint8_t* __restrict__ table, uint32_t row) {
+    const uint4 v = *reinterpret_cast<const uint4*>(table + row * 16u);
+    return Fn16{{v.x, v.y, v.z, v.w}};
+}
+
+// Functions of at most eight states: two words, one byte permute per word and
+// composition (a selector byte below 8 picks among the two), where sixteen
+// slots take three permutes and three other instructions in each of four words.
+struct Fn8 {
+    uint32_t d[2];
+};
+
+__device__ __forceinline__ Fn8 fn_then(const Fn8& f, const Fn8& g) {
+    return Fn8{{__builtin_amdgcn_perm(g.d[1], g.d[0], f.d[0]), __builtin_amdgcn_perm(g.d[1], g.d[0], f.d[1])}};
+}
+__device__ __forceinline__ bool fn_is_const(const Fn8& f) {
+    const uint32_t c = (f.d[0] & 0xffu) * 0x01010101u;
+    return (f.d[0] == c) & (f.d[1] == c);
+}
+__device__ __forceinline__ uint32_t fn_apply(const Fn8& f, uint32_t s) {
+    return __builtin_amdgcn_perm(f.d[1], f.d[0], 0x0c0c0c00u | s);
+}
+__device__ __forceinline__ uint64_t fn_pack(const Fn8& f) {
+    uint64_t out = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < 8; ++s) out |= (uint64_t)((f.d[s >> 2] >> (8 * (s & 3))) & 15u) << (4 * s);
+    return out;
+}
+
+// The same by function type: the constant, the identity on states 0 .. n-1
+// whose other slots hold state `fill`, as does the slot of state `without` (16:
+// none), and a table row (16 bytes apart).
+template <class F>
+struct FnOf;
+template <>
+struct FnOf<Fn16> {
+    static constexpr int kWords = 4;
+    __device__ __forceinline__ static Fn16 row(const uint8_t* __restrict__ t, uint32_t r) { return load_row(t, r); }
+};
+template <>
+struct FnOf<Fn8> {
+    static constexpr int kWords = 2;
+    __device__ __forceinline__ static Fn8 row(const uint8_t* __restrict__ t, uint32_t r) {
+        const uint2 v = *reinterpret_cast<const uint2*>(t + r * 16u);
+        return Fn8{{v.x, v.y}};
+    }
+};
+template <class F>
+__device__ __forceinline__ F fn_const_of(uint32_t s) {
+    F f;
+#pragma unroll
+    for (int i = 0; i < FnOf<F>::kWords; ++i) f.d[i] = s * 0x01010101u;
+    return f;
+}
+template <class F>
+__device__ __forceinline__ F fn_start_of(uint32_t n, uint32_t without, uint32_t fill) {
+    F f;
+#pragma unroll
+    for (int i = 0; i < FnOf<F>::kWords; ++i) {
+        f.d[i] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t s = 4 * i + k;
+            f.d[i] |= (s < n && s != without ? s : fill) << (8 * k);
+        }
+    }
+    return f;
+}
+
 __device__ __forceinline__ uint32_t nib(uint64_t f, uint32_t s) { return (uint32_t)(f >> (4 * s)) & 15u; }
 
 // (g o f) on 64-bit nibble functions.
@@ -412,10 +481,6 @@ __device__ __forceinline__ uint64_t nib_then(uint64_t f, uint64_t g) {
     return out;
 }
 
-__device__ __forceinline__ Fn16 load_row(const uint8_t* __restrict__ table, uint32_t row) {
-    const uint4 v = *reinterpret_cast<const uint4*>(table + row * 16u);
-    return Fn16{{v.x, v.y, v.z, v.w}};
-}
 
 // Whether the strings of this workgroup are all long and start at one offset
 // modulo 4 KiB, as in a packed batch of equal strings. `vote` is one word of

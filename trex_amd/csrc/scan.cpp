@@ -24,7 +24,7 @@ struct trex_plan {
     int64_t n_chunks = 0;
     int64_t chunk_len = 0;
     DevBuf begin, end, sid, pred, flags;   // per chunk, in processing order
-    DevBuf status, agg, jump, control;     // look-back state; control = {ticket, error}
+    DevBuf words, agg, jump;               // look-back state; words = {ticket, error}, status[n_chunks], dead[n_strings]
     // chunk-interleaved image (see trex_plan_build_image): tile t = chunks
     // 64t .. 64t+63 in processing order, tile_vecs[t] 16-byte vectors per lane
     std::vector<int64_t> h_begin, h_end;   // chunk ranges in processing order (host copy)
@@ -123,10 +123,9 @@ int trex_plan_create(const int64_t* begin, const int64_t* end, int64_t n_strings
     if (!rc) rc = p->sid.reserve(m * 4);
     if (!rc) rc = p->pred.reserve(m * 4);
     if (!rc) rc = p->flags.reserve(m * 4);
-    if (!rc) rc = p->status.reserve(m * 4);
+    if (!rc) rc = p->words.reserve((2 + m + (size_t)n_strings) * 4);
     if (!rc) rc = p->agg.reserve(m * 8);
     if (!rc) rc = p->jump.reserve(m * 4);
-    if (!rc) rc = p->control.reserve(16);
     p->h_begin = ob;
     p->h_end = oe;
     if (!rc) rc = p->tile_off.reserve(((n + 63) / 64 + 1) * 8);
@@ -146,7 +145,7 @@ int trex_plan_create(const int64_t* begin, const int64_t* end, int64_t n_strings
 
 int trex_plan_destroy(trex_plan* p) {
     if (!p) return TREX_OK;
-    for (DevBuf* b : {&p->begin, &p->end, &p->sid, &p->pred, &p->flags, &p->status, &p->agg, &p->jump, &p->control,
+    for (DevBuf* b : {&p->begin, &p->end, &p->sid, &p->pred, &p->flags, &p->words, &p->agg, &p->jump,
                       &p->tile_off})
         b->release();
     delete p;
@@ -178,17 +177,18 @@ int match_plan(trex_dfa* h, trex_plan* p, const uint8_t* d_bytes, bool image, ui
     hipStream_t s = (hipStream_t)stream;
     std::lock_guard<std::mutex> lock(p->mu);
 
-    // clear look-back status, ticket and error word with the fill kernel
+    // clear ticket, error word, look-back status and dead flags with the fill kernel
+    uint32_t* ticket = p->words.as<uint32_t>();
+    uint32_t* error = ticket + 1;
+    uint32_t* status = ticket + 2;
+    // (no flags with two chains per lane: joined, the second half's constant
+    // hides a first half that died)
+    uint32_t* dead_flag = h->dead >= 0 && p->chains == 1 ? status + p->n_chunks : nullptr;
     {
-        uint32_t* st = p->status.as<uint32_t>();
-        int64_t n = p->n_chunks;
+        int64_t n = 2 + p->n_chunks + p->n_strings;
         uint32_t zero = 0;
-        void* a1[] = {&st, &n, &zero};
-        TREX_TRY(launch("fill_u32", (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 4096), kBlock, 0, s, a1));
-        uint32_t* ctl = p->control.as<uint32_t>();
-        int64_t two = 2;
-        void* a2[] = {&ctl, &two, &zero};
-        TREX_TRY(launch("fill_u32", 1, kBlock, 0, s, a2));
+        void* a[] = {&ticket, &n, &zero};
+        TREX_TRY(launch("fill_u32", (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 4096), kBlock, 0, s, a));
     }
     const bool window = h->window_base >= 0;
     uint32_t win4 = window ? (uint32_t)h->window_base * 0x01010101u : 0u;
@@ -198,19 +198,22 @@ int match_plan(trex_dfa* h, trex_plan* p, const uint8_t* d_bytes, bool image, ui
     uint8_t* t2 = window ? h->d_t2 : h->d_t1;
     uint8_t* f2 = window ? h->d_f2 : h->d_t1;   // the byte kernel builds its own functions
     int64_t n_chunks = p->n_chunks;
-    uint32_t* ticket = p->control.as<uint32_t>();
-    uint32_t* error = ticket + 1;
     void* args[] = {&d_bytes, &p->tile_off.ptr, &p->begin.ptr, &p->end.ptr, &p->sid.ptr, &p->pred.ptr,
                     &p->flags.ptr, &n_chunks, &t2, &h->d_t1, &f2, &h->d_acc, &win4, &start, &dead, &n_states,
-                    &p->status.ptr, &p->agg.ptr, &p->jump.ptr, &ticket, &error, &max_spins, &max_ticks, &p->hold,
-                    &d_final_state, &d_accept};
+                    &status, &p->agg.ptr, &p->jump.ptr, &ticket, &error, &max_spins, &max_ticks, &p->hold,
+                    &dead_flag, &d_final_state, &d_accept};
     // persistent grid: enough waves to fill every CU, never more than the work
     const int64_t waves_needed = (n_chunks + 63) / 64;
     const int64_t blocks = std::min<int64_t>((waves_needed + 3) / 4, (int64_t)device_cu_count() * 8);
     char kernel[48];
     std::snprintf(kernel, sizeof(kernel), "dfa16_chunks_%s%s%s", window ? "window" : "bytes", image ? "_img" : "",
-                  p->chains == 2 ? "_c2" : "");
-    return launch(kernel, (unsigned)std::max<int64_t>(blocks, 1), kBlock, 0, s, args);
+                  p->chains == 2 ? "_c2" : h->n_states <= 8 ? "_n8" : "");
+    TREX_TRY(launch(kernel, (unsigned)std::max<int64_t>(blocks, 1), kBlock, 0, s, args));
+    if (!dead_flag) return TREX_OK;
+    int64_t n_strings = p->n_strings;
+    void* d_args[] = {&dead_flag, &n_strings, &dead, &d_final_state, &d_accept};
+    return launch("dead_strings", (unsigned)std::min<int64_t>((n_strings + kBlock - 1) / kBlock, 4096), kBlock, 0, s,
+                  d_args);
 }
 
 }  // namespace
@@ -292,7 +295,7 @@ int trex_dfa_match_plan_image(trex_dfa* h, trex_plan* p, const uint8_t* d_image,
 int trex_plan_error(trex_plan* p, uint32_t* error, void* stream) {
     if (!p || !error) return fail(TREX_ERR_INVALID, "null argument");
     uint32_t host = 0;
-    hipError_t e = hipMemcpyAsync(&host, p->control.as<uint32_t>() + 1, 4, hipMemcpyDeviceToHost, (hipStream_t)stream);
+    hipError_t e = hipMemcpyAsync(&host, p->words.as<uint32_t>() + 1, 4, hipMemcpyDeviceToHost, (hipStream_t)stream);
     if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "read plan error word");
     *error = host;

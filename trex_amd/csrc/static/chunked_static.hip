@@ -145,10 +145,11 @@ int trex_dfa_match_chunked_static(trex_dfa* h, const uint8_t* d_bytes, int64_t b
     uint8_t* f2 = window ? h->d_f2 : h->d_t1;
     const int64_t* tile_off = nullptr;   // unused without an image
     uint32_t hold = 0;
+    uint32_t* dead_flag = nullptr;       // the dead state's slot stays in the composed functions
     int64_t n_chunks = n_bound;
     void* args[] = {&d_bytes, &tile_off, &cbegin, &cend, &csid, &cpred, &cflags, &n_chunks, &t2, &h->d_t1, &f2,
                     &h->d_acc, &win4, &start, &dead, &n_states, &status, &agg, &jump, &ticket, &d_error,
-                    &max_spins, &max_ticks, &hold, &d_final_state, &d_accept};
+                    &max_spins, &max_ticks, &hold, &dead_flag, &d_final_state, &d_accept};
     const int64_t waves_needed = (n_chunks + 63) / 64;
     const int64_t blocks = std::min<int64_t>((waves_needed + 3) / 4, (int64_t)device_cu_count() * 8);
     const char* kernel = window ? (kScanChains == 2 ? "dfa16_chunks_window_c2" : "dfa16_chunks_window")
