@@ -520,3 +520,31 @@ def test_plan_dead_strings(gpu_lib, n_states, dead, pure, n_bytes):
                 for b in data[begin[k]:end[k]]:
                     s = delta[s, b]
                 assert (f[k], a[k]) == (s, accept[s]), (k, int(end[k] - begin[k]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hold", [0, 20])
+@pytest.mark.parametrize("lengths", [[1 << 20, (1 << 20) + 77, 64 * 64 * 65],      # chains of up to 256 waves
+                                     [64 * (64 * k + r) for k in (1, 2, 63, 64, 65) for r in (0, 1, 63)],
+                                     [64 * 30 + 7] * 400, [64 * 12] * 33 + [64 * 700 + 1] * 9],   # several roots a wave
+                         ids=["long", "edges", "many", "mixed"])
+def test_plan_wave_look_back(gpu_lib, lengths, hold):
+    """Chains that never turn constant, of one wave and of many, with one chain
+    in a wave and with several, published in order and held back."""
+    from trex_amd.device import DeviceBuffer
+    from trex_amd.engine import ChunkPlan, DeviceBatch, DfaEngine
+    rng = np.random.default_rng(len(lengths))
+    delta, accept = _table(rng, 16, 0x41, 26, True, pure=True)
+    tab = DfaByteTable(delta, accept, 0, 15, 16)
+    data, offs = ragged_batch(rng, np.array(lengths, np.int64), 0x41, 0x41 + 26)
+    batch = DeviceBatch(data, offs, layout="csr")
+    plan = ChunkPlan.for_batch(batch, 64)
+    plan.set_hold(hold)
+    n = len(lengths)
+    d_f, d_a = DeviceBuffer(n), DeviceBuffer(n)
+    rf, ra = ocpu.dfa_walk(delta, accept, 0, data, offs)
+    eng = DfaEngine(tab)
+    for _ in range(3):
+        eng.match_plan(plan, batch.d_bytes.ptr, d_f.ptr, d_a.ptr)
+        assert plan.error() == 0
+        assert np.array_equal(d_f.download(np.uint8, n), rf) and np.array_equal(d_a.download(np.uint8, n), ra)

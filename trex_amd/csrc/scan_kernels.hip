@@ -20,7 +20,7 @@
 //    need not know. A chunk that ends dead sets its string's flag (dead_flag;
 //    dead_strings writes those strings' results after the launch), and every
 //    other chunk's state is right unless an earlier one died. Before this an
-//automaton that text does not kill composed every byte of it (9 states,
+//    automaton that text does not kill composed every byte of it (9 states,
 //    173 MB in 6 strings: 282 us, 61 us with the flags; 1 GiB in 16: 928 us,
 //    206 us). Tables of at most eight states compose in two words (Fn8).
 //    The chunk then publishes AGGREGATE (its function), or PREFIX (its final
@@ -29,7 +29,8 @@
 //  Phase 2 (look-back, cuda/monoid_scan.cu:128-222 restated over functions):
 //    walk back over predecessors, composing their aggregates, until one with
 //    PREFIX is found; the chunk's prefix state is F(acc(p)). Waiting is only
-//    for predecessors' phase-1 results, which never wait on anything.
+//    for predecessors' phase-1 results, which never wait on anything. A wave
+//    walks back 64 waves at a time (wave_look_back).
 //
 // Forward progress: chunks are claimed 256 at a time (one workgroup, 64 per
 // wave) from an atomic ticket in index order, and a chunk's predecessor
@@ -182,6 +183,69 @@ struct Scanner {
         w.all &= o.w.all;
     }
 };
+
+constexpr uint64_t kIdentity = 0xfedcba9876543210ull;
+constexpr int kWaveRoots = 4;
+
+// The state before chunk c whose predecessor is chunk j, read by a whole wave
+// (every lane passes the same j). The look-back of one lane is a chain of
+// dependent loads, one step per wave of the string before this one (its
+// aggregates reach back to their wave's first chunk of the string): about 2 us
+// a step. The chain of a long string passes every 64th chunk, so lane k loads
+// the words of chunk j - 64k at once, the lanes up to the first one that is a
+// prefix, not ready or off the chain are composed in six shuffled rounds, and
+// the walk goes on from there: a step covers 64 waves. Parity of the length
+// (never constant), 173 MB in 6 strings: 451 us a lane at a time, 96 us so;
+// 1 GiB in 16 strings: 445 us, 331 us. Most look-backs end at the first
+// chunk, so the rounds stop with the last lane that counts (all six always:
+// 202 us instead of 189 us where one wave in a few composes).
+// kWaveRoots: the chains of a wave take turns here; with more of them each
+// lane follows its own (they are then short, as are their look-backs).
+__device__ __forceinline__ uint32_t wave_look_back(int32_t j, uint32_t lane, const uint32_t* __restrict__ status,
+                                                   const uint64_t* __restrict__ agg,
+                                                   const int32_t* __restrict__ jump, uint32_t* __restrict__ error,
+                                                   uint32_t max_spins, uint64_t max_ticks, uint32_t dead) {
+    uint64_t acc_fn = kIdentity;
+    BoundedWait wait(max_spins, max_ticks);
+    while (true) {
+        const int32_t mine = j - 64 * (int32_t)lane;
+        const uint32_t st = mine >= 0 ? load_relaxed(&status[mine]) : 0u;
+        wait_stores();   // the loads below come after the status words'
+        const bool aggregate = (st & 0xffu) == kStatusAggregate, prefix = (st & 0xffu) == kStatusPrefix;
+        uint64_t fn = kIdentity;
+        int32_t next = mine;   // of a chunk that is not ready: itself, again
+        if (aggregate) {
+            fn = load_through(&agg[mine]);
+            next = (int32_t)load_relaxed(reinterpret_cast<const uint32_t*>(&jump[mine]));
+        } else if (prefix) {
+            fn = (uint64_t)((st >> 8) & 15u) * 0x1111111111111111ull;
+        }
+        // lanes before `stop` are aggregates that lead to the next lane's chunk
+        const uint64_t off = __ballot(!(aggregate && mine >= 64 && next == mine - 64));
+        const uint32_t stop = off != 0ull ? (uint32_t)__ffsll((unsigned long long)off) - 1u : 63u;
+        if (lane > stop) fn = kIdentity;
+#pragma unroll 1   // (unrolled, the kernels go over 128 VGPRs)
+        for (int d = 1; d <= (int)stop; d <<= 1) {
+            const uint64_t up = __shfl_down(fn, d, 64);
+            if (lane + d < 64u) fn = nib_then(up, fn);   // earlier chunks (higher lanes) apply first
+        }
+        acc_fn = nib_then(__shfl(fn, 0, 64), acc_fn);
+        if (__shfl((int)prefix, (int)stop, 64)) return nib(acc_fn, 0u);   // constant: from the prefix on
+        const bool ready = __shfl((int)aggregate, (int)stop, 64) != 0;
+        j = __shfl(next, (int)stop, 64);
+        if (j < 0) {   // cannot happen: a string's first chunk publishes a prefix
+            if (lane == 0) atomicOr(error, 2u);
+            return dead;
+        }
+        if (!ready) {
+            if (__ballot(wait.expired()) != 0ull) {
+                if (lane == 0) atomicOr(error, 1u);
+                return dead;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
+    }
+}
 
 // Always inlined into its kernels, at 8 vectors in flight (<= 106 VGPRs, no
 // stack). A build with 16 in flight compiled the byte kernels' copy as a
@@ -379,10 +443,13 @@ __device__ __forceinline__ void chunk_scan(const uint8_t* __restrict__ bytes, co
             if (known) {
                 store_relaxed(&status[c], kStatusPrefix | (kstate << 8));   // the word says it all
             } else {
-                agg[c] = my_fn;
-                jump[c] = root_pred;
-                store_release(&status[c], kStatusAggregate);   // agg and jump first
+                store_through(&agg[c], my_fn);
+                store_relaxed(reinterpret_cast<uint32_t*>(&jump[c]), (uint32_t)root_pred);
             }
+        }
+        if (__ballot(active && !known) != 0ull) {
+            wait_stores();   // agg and jump first
+            if (active && !known) store_relaxed(&status[c], kStatusAggregate);
         }
 
         // ---- phase 2: the root of each unresolved chain looks back ----
@@ -392,8 +459,17 @@ __device__ __forceinline__ void chunk_scan(const uint8_t* __restrict__ bytes, co
         // on this one. Waits are bounded by the spin count and by wall-clock
         // ticks; on expiry the error word is set and the wave moves on.
         uint32_t incoming = 0;
-        if (active && !known && root == lane) {
-            uint64_t acc_fn = 0xfedcba9876543210ull;   // identity
+        const bool looks = active && !known && root == lane;
+        uint64_t roots = __ballot(looks);
+        if (__popcll(roots) <= kWaveRoots) {
+            for (; roots != 0ull; roots &= roots - 1) {
+                const int r = __ffsll((unsigned long long)roots) - 1;
+                const uint32_t in =
+                    wave_look_back(__shfl(pred, r, 64), lane, status, agg, jump, error, max_spins, max_ticks, dead);
+                if ((int)lane == r) incoming = in;
+            }
+        } else if (looks) {
+            uint64_t acc_fn = kIdentity;
             int32_t j = pred;
             BoundedWait wait(max_spins, max_ticks);
             while (true) {
@@ -411,9 +487,9 @@ __device__ __forceinline__ void chunk_scan(const uint8_t* __restrict__ bytes, co
                     incoming = nib(acc_fn, (st >> 8) & 15u);
                     break;
                 }
-                fence_acquire();   // agg[j] and jump[j] were written before status[j] was released
-                acc_fn = nib_then(agg[j], acc_fn);   // earlier chunks apply first
-                j = jump[j];
+                wait_stores();   // the loads below come after the status word's
+                acc_fn = nib_then(load_through(&agg[j]), acc_fn);   // earlier chunks apply first
+                j = (int32_t)load_relaxed(reinterpret_cast<const uint32_t*>(&jump[j]));
                 if (j < 0) {   // cannot happen: a string's first chunk publishes a prefix
                     atomicOr(error, 2u);
                     incoming = dead;
@@ -529,7 +605,7 @@ chunk_table_count(const int64_t* __restrict__ begin, const int64_t* __restrict__
         }
         // inclusive scan within the wave, then across the 16 waves
         int64_t x = cnt;
-#pragma unroll
+#pragma unroll 1   // (unrolled, the kernels go over 128 VGPRs)
         for (int d = 1; d < 64; d <<= 1) {
             const int64_t y = __shfl_up(x, d, 64);
             if ((int)lane >= d) x += y;
