@@ -649,3 +649,37 @@ def test_chunk_mass_restore_in_fp32_drifts():
     # and about in proportion to the number of chunks
     d16 = _emulate_chunked_ll(T, start, accept, np.random.default_rng(100).integers(0, 32, 4000), 16, False)
     assert abs(drift[0]) > 2 * abs(d16) and np.sign(d16) == np.sign(drift[0]), (drift[0], d16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["f16x2", "bf16x2", "f16", "bf16"])
+@pytest.mark.parametrize("per_cu", [0, 1, 2, 4, 8, 16, 32])
+def test_gpu_small_batches_same_results(gpu_lib, mode, per_cu):
+    """A batch is cut into workgroups of 1 to 64 sequences by its size: at the
+    largest batch of each size and one above it, ragged (from empty on, skewed
+    symbols, some outside the alphabet), the results are those of workgroups
+    of 64 bit for bit, and a sample matches the FP64 oracle."""
+    from trex_amd import _lib
+    cus = _lib.device_info()["cus"]
+    rng = np.random.default_rng(per_cu)
+    T, start, accept = dirichlet_pnfa(rng, 32)
+    for n in (max(per_cu * cus - 1, 1), per_cu * cus + 1):
+        lengths = rng.integers(0, 9, size=n)
+        lengths[rng.integers(0, n, size=n // 50 + 1)] = rng.integers(60, 140, size=n // 50 + 1)
+        offsets = np.zeros(n + 1, np.int64)
+        np.cumsum(lengths, out=offsets[1:])
+        data = rng.integers(0, 32, size=int(offsets[-1]) + 1).astype(np.uint8)
+        data[rng.random(len(data)) < 0.3] = 7
+        data[rng.random(len(data)) < 0.001] = 77
+        data = data[:-1]
+        eng = _engine(T, start, accept)
+        eng.set_mode(mode)
+        ll, lm = eng.loglik_ragged(data, offsets)
+        eng.set_waves(8)
+        ll8, lm8 = eng.loglik_ragged(data, offsets)
+        assert np.array_equal(ll, ll8) and np.array_equal(lm, lm8)
+        for i in rng.integers(0, n, size=20):
+            ref, _ = oprob.forward_loglik(T, start, accept, data[offsets[i]:offsets[i + 1]][None, :])
+            assert np.isfinite(ref[0]) == np.isfinite(ll[i])
+            if np.isfinite(ref[0]):
+                assert abs(ll[i] - ref[0]) <= 1e-3 * max(abs(ref[0]), 1.0)

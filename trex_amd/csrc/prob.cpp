@@ -166,6 +166,7 @@ struct trex_pnfa {
     int n_symbols = 0;
     int mode = TREX_PNFA_F16X2;
     int waves = 8;           // waves per workgroup (4: eight symbols per wave, 8: four)
+    bool waves_set = false;  // chosen by the caller: the launch shape stays as asked for
     int64_t grid = 0;        // most workgroups per kernel launch (0: one per group of 64 sequences)
     bool f16_ok = true;      // every |T| fits binary16
     int e0 = 0;              // s0 = s0n * 2^e0 with max |s0n| in [0.5, 1)
@@ -305,6 +306,7 @@ int trex_pnfa_set_waves(trex_pnfa* h, int waves) {
     if (!h) return fail(TREX_ERR_INVALID, "null handle");
     if (waves != 4 && waves != 8) return fail(TREX_ERR_INVALID, "waves must be 4 or 8, got %d", waves);
     h->waves = waves;
+    h->waves_set = true;
     return TREX_OK;
 }
 
@@ -333,23 +335,43 @@ int trex_pnfa_rounded(const trex_pnfa* h, int mode, float* t_rounded, double* co
 
 namespace {
 
+// Sequences per workgroup: the fewest that still give every workgroup a CU of
+// its own. A workgroup's step waits for the slowest of its waves, and a wave's
+// time grows with the sequences on its symbols, so batches that leave CUs idle
+// at 64 are spread out (in workgroups of four waves, one per SIMD, which beat
+// eight at every size below 64). 64 and the size picked, FP16 split state:
+//     250 x 1000 symbols:  2,071 us and 1,109 us (1)
+//     600 x 64..1024:      1,706 us and 1,201 us (4; 2 gives 1,429 us)
+//     2,000 x 500:         1,065 us and 731 us (8; 4 gives 1,278 us)
+//     4,096 x 300:         659 us and 507 us (16)
+//     8,192 x 300:         680 us and 603 us (32)
+int64_t group_of(int64_t n_seq) {
+    const int64_t cus = device_cu_count();
+    int64_t g = 1;
+    while (g < kSeqPerGroup && n_seq > g * cus) g *= 2;
+    return g;
+}
+
 int pnfa_launch(trex_pnfa* h, const uint8_t* d_symbols, const int64_t* d_begin, const int64_t* d_end, int64_t n_seq,
                 int L, double* d_ll, double* d_logmass, void* stream) {
-    const int64_t groups = (n_seq + kSeqPerGroup - 1) / kSeqPerGroup;
+    const int64_t group = h->waves_set || h->grid > 0 ? kSeqPerGroup : group_of(n_seq);
+    const int64_t groups = (n_seq + group - 1) / group;
     if (groups > 0x7fffffff) return fail(TREX_ERR_INVALID, "too many sequences");
     const bool f16 = uses_f16(h->mode);
     const uint16_t* tlp = f16 ? h->d_q16 : h->d_qb16;
     const float* scale = f16 ? h->d_scale16 : h->d_scaleb16;
     int n_sym = h->n_symbols, e0 = h->e0;
     char name[48];
-    std::snprintf(name, sizeof(name), "pnfa64_%s_w%d", mode_name(h->mode), h->waves);
+    const int waves = group < kSeqPerGroup ? 4 : h->waves;
+    if (group < kSeqPerGroup) std::snprintf(name, sizeof(name), "pnfa64_%s_w4_g%d", mode_name(h->mode), (int)group);
+    else std::snprintf(name, sizeof(name), "pnfa64_%s_w%d", mode_name(h->mode), waves);
     // A grid cap splits the groups over consecutive launches on the stream.
     // Callers put long sequences first, so the first launch's longest group
     // sets the pace as it would for one workgroup taking every cap-th group.
     const int64_t per = h->grid > 0 ? h->grid : groups;
     for (int64_t g0 = 0; g0 < groups; g0 += per) {
-        const int64_t first = g0 * kSeqPerGroup;
-        int64_t n = std::min<int64_t>(n_seq - first, per * kSeqPerGroup);
+        const int64_t first = g0 * group;
+        int64_t n = std::min<int64_t>(n_seq - first, per * group);
         const uint8_t* sym = d_begin ? d_symbols : d_symbols + (d_symbols ? first * (int64_t)L : 0);
         const int64_t* b = d_begin ? d_begin + first : nullptr;
         const int64_t* e = d_end ? d_end + first : nullptr;
@@ -357,8 +379,8 @@ int pnfa_launch(trex_pnfa* h, const uint8_t* d_symbols, const int64_t* d_begin, 
         double* lm = d_logmass + first;
         void* args[] = {&tlp, &scale, &h->d_t32, &n_sym, &h->d_s0, &e0, &h->d_acc, &sym, &b, &e,
                         &n, &L, &ll, &lm};
-        const unsigned grid = (unsigned)((n + kSeqPerGroup - 1) / kSeqPerGroup);
-        TREX_TRY(launch(name, grid, 64u * (unsigned)h->waves, 0, (hipStream_t)stream, args));
+        const unsigned grid = (unsigned)((n + group - 1) / group);
+        TREX_TRY(launch(name, grid, 64u * (unsigned)waves, 0, (hipStream_t)stream, args));
     }
     return TREX_OK;
 }

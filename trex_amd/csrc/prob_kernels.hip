@@ -44,11 +44,10 @@ using namespace pnfadev;
 
 constexpr int kStates = 64;
 constexpr int kRow = kStates + 4;   // padded LDS row (floats) against bank conflicts
-constexpr int kSeqPerGroup = 64;
 constexpr int kMaxSymbols = 32;
 constexpr int kChunk = 64;          // symbols staged per sequence at a time
 
-template <bool BF16, bool SPLIT, int SPW>
+template <bool BF16, bool SPLIT, int SPW, int kSeqPerGroup>
 __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __restrict__ colscale,
                              const float* __restrict__ t32, int n_sym, const float* __restrict__ s0, int e0,
                              const float* __restrict__ accw, const uint8_t* __restrict__ symbols,
@@ -57,7 +56,9 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
 {
     typedef typename Lp<BF16>::vec vec;
     constexpr int kBlock = 64 * (kMaxSymbols / SPW);
-    constexpr int kTps = kBlock / kSeqPerGroup;   // threads per sequence in the last step
+    // threads per sequence in the last step; eight for every size below 64, as
+    // for 64 in eight waves, so that the sums have one order
+    constexpr int kTps = kBlock / kSeqPerGroup < 8 ? kBlock / kSeqPerGroup : 8;
     constexpr int kRing = 2 * kChunk;             // staged symbols per sequence: this chunk and the next
     constexpr uint8_t kDone = 0xfe;               // no rounded step at this position (the sequence has ended)
     // One state row per sequence, updated in place: a row is read and then
@@ -168,7 +169,7 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
         int seq, c;   // the first tile's column (lane & 15): its sequence and symbol
     };
     auto route_part = [&](Route& r, int t, int part) {
-        if (part == 0) r.cj = syms[lane][t % kRing];
+        if (part == 0) r.cj = kSeqPerGroup == 64 || lane < kSeqPerGroup ? syms[lane][t % kRing] : kDone;
         if (part == 1) {
             const bool sel = r.cj < n_sym && r.cj / SPW == wave;
             const uint64_t m = __ballot(sel);
@@ -183,7 +184,7 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
             const auto h = __builtin_amdgcn_permlane32_swap(v0, v0, false, false);   // lanes 32..63 <- 0..31
             const auto q = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);   // odd rows <- even rows
             const int v = (int)q[0];
-            r.seq = v & 0xff;
+            r.seq = v & (kSeqPerGroup - 1);   // any row of the workgroup for a lane past the columns
             // a lane past the tile's columns reads any row of the symbol tables
             r.c = (lane & 15) < r.cnt ? (v >> 8) & 0xff : wave * SPW;
         }
@@ -305,7 +306,7 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
                 const int n = g * 16 + (lane & 15);
                 const bool valid = n < r.cnt;
                 const int v = __shfl(again.colseq, valid ? n : g * 16, 64);
-                tile(v & 0xff, (v >> 8) & 0xff, valid, [](int) {});
+                tile(v & (kSeqPerGroup - 1), (v >> 8) & 0xff, valid, [](int) {});
             }
         }
         __syncthreads();
@@ -350,11 +351,16 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
 
 }  // namespace
 
-// Kernels: pnfa64_<mode>_w<W>, W = waves per workgroup (32 / symbols per wave);
-// one workgroup of 64 * W threads per 64 sequences. Sequence j is
+// Kernels: pnfa64_<mode>_w<W>[_g<G>], W = waves per workgroup (32 / symbols per
+// wave); one workgroup of 64 * W threads per 64 (G) sequences. A batch too small
+// for a workgroup of 64 on every CU is bound by the time of a step, which is
+// a wave's: a tile, sixteen MFMAs for each of its symbols that a sequence is
+// on. Fewer sequences a workgroup leave a wave fewer symbols at a step (1.7 us
+// a step at 64, 1.2 us at 4, 1.1 us at 1); a sequence's own arithmetic is the
+// same at every G (the other columns' zeros add nothing). Sequence j is
 // symbols[sbegin[j] .. send[j]), or symbols[j * L .. (j + 1) * L) when sbegin
 // is null.
-#define PNFA_KERNEL(NAME, BF16, SPLIT, SPW)                                                                       \
+#define PNFA_KERNEL(NAME, BF16, SPLIT, SPW, G)                                                                    \
     extern "C" __global__ void __launch_bounds__(64 * (32 / SPW))                                                  \
     __attribute__((amdgpu_waves_per_eu(32 / SPW / 4, 32 / SPW / 4)))                                              \
     NAME(const uint16_t* __restrict__ tlp, const float* __restrict__ colscale, const float* __restrict__ t32,     \
@@ -362,15 +368,21 @@ __device__ void pnfa_forward(const uint16_t* __restrict__ tlp, const float* __re
          const uint8_t* __restrict__ symbols, const int64_t* __restrict__ sbegin,                                 \
          const int64_t* __restrict__ send, int64_t n_seq, int L, double* __restrict__ out_ll,                     \
          double* __restrict__ out_logmass) {                                                                      \
-        pnfa_forward<BF16, SPLIT, SPW>(tlp, colscale, t32, n_sym, s0, e0, accw, symbols, sbegin, send, n_seq, L,  \
+        pnfa_forward<BF16, SPLIT, SPW, G>(tlp, colscale, t32, n_sym, s0, e0, accw, symbols, sbegin, send, n_seq, L,  \
                                        out_ll, out_logmass);                                                      \
     }
 
-#define PNFA_KERNELS(W, SPW)                                  \
-    PNFA_KERNEL(pnfa64_f16x2_w##W, false, true, SPW)          \
-    PNFA_KERNEL(pnfa64_bf16x2_w##W, true, true, SPW)          \
-    PNFA_KERNEL(pnfa64_f16_w##W, false, false, SPW)           \
-    PNFA_KERNEL(pnfa64_bf16_w##W, true, false, SPW)
+#define PNFA_KERNELS(TAG, SPW, G)                                   \
+    PNFA_KERNEL(pnfa64_f16x2_##TAG, false, true, SPW, G)           \
+    PNFA_KERNEL(pnfa64_bf16x2_##TAG, true, true, SPW, G)           \
+    PNFA_KERNEL(pnfa64_f16_##TAG, false, false, SPW, G)            \
+    PNFA_KERNEL(pnfa64_bf16_##TAG, true, false, SPW, G)
 
-PNFA_KERNELS(4, 8)
-PNFA_KERNELS(8, 4)
+PNFA_KERNELS(w4, 8, 64)
+PNFA_KERNELS(w8, 4, 64)
+PNFA_KERNELS(w4_g1, 8, 1)
+PNFA_KERNELS(w4_g2, 8, 2)
+PNFA_KERNELS(w4_g4, 8, 4)
+PNFA_KERNELS(w4_g8, 8, 8)
+PNFA_KERNELS(w4_g16, 8, 16)
+PNFA_KERNELS(w4_g32, 8, 32)
