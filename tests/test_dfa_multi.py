@@ -212,3 +212,46 @@ def test_gpu_multi_refuses_tables_without_a_window(gpu_lib):
     # an empty batch launches nothing and returns empty results
     f, a = multi.match_arrays(np.zeros(0, np.uint8), np.zeros(1, np.int64))
     assert f.shape == (1, 0) and a.shape == (1, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_strings", [700, 17000])   # one wave a workgroup, and 256 threads
+@pytest.mark.parametrize("sizes", [[9], [9, 8, 4], [16, 3], [10, 2, 2, 2], [5, 9, 9, 9, 4, 3, 2, 1],
+                                   [9, 9, 9, 9, 9, 9, 9, 9], [16, 15, 10, 9, 9, 9, 9, 9], [4] * 8, [3, 9, 16, 7] * 3],
+                         ids=str)
+def test_contiguous_strings_by_state_count(gpu_lib, sizes, n_strings):
+    """Patterns of every width a launch can mix (at most 4 states, at most
+    eight live ones, 16; the dead state first, in the middle, last), strings
+    of every alignment and of no byte, bytes outside a pattern's alphabet or
+    window at either end: the default form gives each pattern's walk, in the
+    layout it is given."""
+    from oracle import cpu as ocpu
+    from trex_amd.engine import DfaEngine, DfaMultiEngine
+    from trex_amd.tables import DfaByteTable
+    rng = np.random.default_rng(len(sizes) + n_strings)
+    tabs = []
+    for i, n in enumerate(sizes):
+        dead = (0, n // 2, n - 1)[i % 3]
+        delta = np.full((n, 256), dead, np.uint8)
+        live = [s for s in range(n) if s != dead] or [dead]
+        for b in range(0x41, 0x41 + 26):
+            delta[live, b] = rng.choice(live, len(live))
+        delta[live[0], 0x45] = dead
+        delta[dead] = dead
+        accept = rng.integers(0, 2, n).astype(np.uint8)
+        accept[dead] = 0
+        tabs.append(DfaByteTable(delta, accept, live[-1], dead, n))
+    lengths = rng.integers(0, 70, n_strings)
+    lengths[::50] = rng.integers(100, 700, len(lengths[::50]))
+    offsets = np.zeros(n_strings + 1, np.int64)
+    np.cumsum(lengths, out=offsets[1:])
+    data = rng.integers(0x41, 0x41 + 26, int(offsets[-1])).astype(np.uint8)
+    data[data == 0x45] = np.where(rng.random(int((data == 0x45).sum())) < 0.05, 0x45, 0x46)
+    ends = np.concatenate([offsets[1:][lengths > 0][::7] - 1, offsets[:-1][lengths > 0][::11]])
+    data[ends] = rng.choice(np.frombuffer(b"[a\x00\xff", np.uint8), len(ends))
+    multi = DfaMultiEngine([DfaEngine(t) for t in tabs])
+    for layout in ("csr", "staggered"):
+        final, acc = multi.match_arrays(data, offsets, layout=layout)
+        for i, t in enumerate(tabs):
+            rf, ra = ocpu.dfa_walk(t.delta, t.accept, t.start, data, offsets)
+            assert np.array_equal(final[i], rf) and np.array_equal(acc[i], ra), (layout, i)

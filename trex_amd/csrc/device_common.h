@@ -273,6 +273,25 @@ __device__ __forceinline__ void stage_table(uint8_t* __restrict__ dst, const uin
     for (int i = threadIdx.x; i < (n >> 4); i += blockDim.x) d4[i] = s4[i];
 }
 
+// Stages the table (its copy in LDS starts at byte 0, so that table offsets
+// are immediates) and finds the thread's string, -1 for none. Dynamic LDS:
+// tab_bytes, and order_bytes(256) more in workgroups of 256 threads.
+__device__ __forceinline__ int64_t stage_and_pick(uint8_t* lds, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
+                                                  const int64_t* __restrict__ begin,
+                                                  const int64_t* __restrict__ endp, int64_t n_strings) {
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x;
+    const uint32_t n_here = (uint32_t)min<int64_t>(n_strings - first, blockDim.x);
+    const int64_t mine = first + min(threadIdx.x, n_here - 1u);
+    const int64_t len = endp[mine] - begin[mine];
+    const bool order = blockDim.x == 256u;
+    uint32_t* count = reinterpret_cast<uint32_t*>(lds + tab_bytes);
+    stage_table(lds, tabg, (int)tab_bytes);
+    if (order && threadIdx.x < 64u) count[threadIdx.x] = 0u;
+    __syncthreads();
+    const uint32_t k = order ? order_by_length(count, n_here, len) : threadIdx.x;
+    return k < n_here ? first + k : -1;
+}
+
 // ---------------------------------------------------------------------------
 // 32-byte symbol windows
 // ---------------------------------------------------------------------------
@@ -290,9 +309,14 @@ struct WinCheck {
     }
 };
 
-// Pair index sym0 | sym1 << 5 of the low / high two bytes of a word (sym = byte & 31).
-__device__ __forceinline__ uint32_t pair_lo(uint32_t x) { return (x & 31u) | (((x >> 8) & 31u) << 5); }
-__device__ __forceinline__ uint32_t pair_hi(uint32_t x) { return ((x >> 16) & 31u) | (((x >> 24) & 31u) << 5); }
+// Pair index sym0 | sym1 << 5 of the low / high two bytes of a word (sym = byte
+// & 31): a byte dot product, one instruction where shifts and masks take three.
+__device__ __forceinline__ uint32_t pair_lo(uint32_t x) {
+    return __builtin_amdgcn_udot4(x & 0x1f1f1f1fu, 0x00002001u, 0u, false);
+}
+__device__ __forceinline__ uint32_t pair_hi(uint32_t x) {
+    return __builtin_amdgcn_udot4(x & 0x1f1f1f1fu, 0x20010000u, 0u, false);
+}
 
 // The eight pair functions (nibble s = successor of s) of a 16-byte vector:
 // table reads only, independent of the state.

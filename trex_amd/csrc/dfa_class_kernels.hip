@@ -49,25 +49,6 @@ constexpr int kClsBytes = 256;    // byte -> class * 8
 constexpr int kMapBytes = 1040;   // map[257] of the wide form, padded
 constexpr int kPF = 4;            // vectors in flight ahead of the block being walked
 
-// Stages the table (its copy in LDS starts at byte 0, so that table offsets
-// are immediates) and finds the thread's string, -1 for none. Dynamic LDS:
-// tab_bytes, and order_bytes(256) more in workgroups of 256 threads.
-__device__ __forceinline__ int64_t stage_and_pick(uint8_t* lds, const uint8_t* __restrict__ tabg, uint32_t tab_bytes,
-                                                  const int64_t* __restrict__ begin,
-                                                  const int64_t* __restrict__ endp, int64_t n_strings) {
-    const int64_t first = (int64_t)blockIdx.x * blockDim.x;
-    const uint32_t n_here = (uint32_t)min<int64_t>(n_strings - first, blockDim.x);
-    const int64_t mine = first + min(threadIdx.x, n_here - 1u);
-    const int64_t len = endp[mine] - begin[mine];
-    const bool order = blockDim.x == 256u;
-    uint32_t* count = reinterpret_cast<uint32_t*>(lds + tab_bytes);
-    stage_table(lds, tabg, (int)tab_bytes);
-    if (order && threadIdx.x < 64u) count[threadIdx.x] = 0u;
-    __syncthreads();
-    const uint32_t k = order ? order_by_length(count, n_here, len) : threadIdx.x;
-    return k < n_here ? first + k : -1;
-}
-
 // Function words by number of states: the field of state s holds its successor,
 // and the walk keeps its state as the shift amount of its field, so that a step
 // is as few dependent instructions as the width allows.

@@ -30,6 +30,13 @@ constexpr int kMultiMax = 8;          // patterns per launch (kernels exist for 
 constexpr int kMultiGroup = 4;        // default patterns per launch
 constexpr int kMultiPatterns = 256;   // patterns per handle
 
+// Contiguous strings of the compact form: from this many strings on, 256
+// threads a workgroup, which orders its strings by length; below, one wave a
+// workgroup, so that the waves spread over the CUs (8 patterns, 50,000 x
+// 200..3000 bytes: 85 us, one wave a workgroup 190 us, most of it staging;
+// 2,000 x 2000..4000: 108 us by waves, 117 us by 256).
+constexpr int64_t kCompactBlockFrom = 16384;
+
 // Kernel argument block; the layout of MultiParams in dfa_multi_kernels.hip.
 struct MultiParams {
     uint32_t win4[kMultiMax];
@@ -49,10 +56,12 @@ struct CompactParams {
 };
 
 // One launch of the compact form: NF full and NB byte patterns, its tables
-// at byte offsets into the handle's compact buffers.
+// at byte offsets into the handle's compact buffer (n8_off: those of
+// bytes, if no full pattern has more than eight states besides the dead one).
 struct CompactLaunch {
     int nf = 0, nb = 0;
-    size_t words_off = 0, syms_off = 0;
+    size_t words_off = 0, n8_off = 0;
+    bool n8 = false;
     CompactParams prm{};
 };
 
@@ -73,8 +82,8 @@ struct trex_dfa_multi {
     int fp_group = -1;            // the group d_fp was built for
     std::vector<uint64_t> h_f1;   // [n][32] single-symbol functions (host copy)
     std::vector<int> n_states;
-    uint8_t* d_fc = nullptr;      // compact pair tables of the current grouping
-    uint8_t* d_fcs = nullptr;     // and the launches' single-symbol tables in launch order
+    bool picked = true;           // the form and the group are the handle's own choice
+    uint8_t* d_fc = nullptr;      // compact tables of the current grouping
     std::vector<CompactLaunch> fc;
     int fc_group = -1;            // the group d_fc was built for
 };
@@ -129,15 +138,36 @@ uint64_t byte_function(uint64_t f) {
     return b;
 }
 
-// Compact tables for the current grouping: per launch, its full patterns
+// Entry of a compact table: the 1,024 pairs, single symbols, the identity
+// (layout in dfa_compact_kernels.hip).
+constexpr int kCompactEntries = 1058;
+
+uint64_t entry_function(const trex_dfa_multi* m, int p, int x) {
+    if (x < 1024) return m->h_f2[(size_t)p * 1024 + x];
+    if (x < 1056) return m->h_f1[(size_t)p * 32 + (x - 1024)];
+    return 0xfedcba9876543210ull;   // nibble s = s
+}
+
+// A full function of at most eight states besides the dead one: a byte for each
+// of them, the successor's number among them or 0xff for the dead state.
+uint64_t n8_function(uint64_t f, int n, int dead) {
+    uint64_t out = 0;
+    for (int s = 0, at = 0; s < n; ++s) {
+        if (s == dead) continue;
+        const int next = (int)((f >> (4 * s)) & 15u);
+        out |= (uint64_t)(next == dead ? 0xff : next - (next > dead ? 1 : 0)) << (8 * at++);
+    }
+    return out;
+}
+
+// Compact tables in launches of `group` patterns: per launch, its full patterns
 // first (one 64-bit word each), then its patterns of at most 4 states (eight
 // bytes to a word); the words of entry x stored pair by pair (NW / 2 tables of
-// 1024 x 16 bytes, then 1024 x 8 bytes for an odd last word), and the
-// single-symbol functions in the same pattern order.
-int build_compact(trex_dfa_multi* m) {
-    std::vector<uint64_t> words, syms;
+// 16 bytes an entry, then 8 bytes an entry for an odd last word).
+int build_compact(trex_dfa_multi* m, int group) {
+    std::vector<uint64_t> words;
     std::vector<CompactLaunch> fc;
-    for (const auto& [p0, P] : launches_of(m->n, m->group)) {
+    for (const auto& [p0, P] : launches_of(m->n, group)) {
         std::vector<int> order;
         for (int k = p0; k < p0 + P; ++k)
             if (!narrow(m, k)) order.push_back(k);
@@ -147,26 +177,31 @@ int build_compact(trex_dfa_multi* m) {
         CompactLaunch L;
         L.nf = nf;
         L.nb = P - nf;
-        L.words_off = words.size() * 8;
-        L.syms_off = syms.size() * 8;
+        L.n8 = nf > 0;
+        for (int k = 0; k < nf; ++k) L.n8 = L.n8 && m->n_states[order[k]] <= 9;
         const int nw = nf + (L.nb + 7) / 8;
-        std::vector<uint64_t> entry((size_t)1024 * nw, 0);   // [x][word]
-        for (int x = 0; x < 1024; ++x) {
-            for (int k = 0; k < nf; ++k) entry[(size_t)x * nw + k] = m->h_f2[(size_t)order[k] * 1024 + x];
-            for (int i = 0; i < L.nb; ++i)
-                entry[(size_t)x * nw + nf + i / 8] |=
-                    byte_function(m->h_f2[(size_t)order[nf + i] * 1024 + x]) << (8 * (i % 8));
-        }
-        for (int j = 0; j < nw / 2; ++j)
-            for (int x = 0; x < 1024; ++x) {
-                words.push_back(entry[(size_t)x * nw + 2 * j]);
-                words.push_back(entry[(size_t)x * nw + 2 * j + 1]);
+        for (int n8 = 0; n8 <= (L.n8 ? 1 : 0); ++n8) {
+            std::vector<uint64_t> entry((size_t)kCompactEntries * nw, 0);   // [x][word]
+            for (int x = 0; x < kCompactEntries; ++x) {
+                for (int k = 0; k < nf; ++k) {
+                    const uint64_t f = entry_function(m, order[k], x);
+                    entry[(size_t)x * nw + k] = n8 ? n8_function(f, m->n_states[order[k]], (int)m->dead[order[k]]) : f;
+                }
+                for (int i = 0; i < L.nb; ++i)
+                    entry[(size_t)x * nw + nf + i / 8] |= byte_function(entry_function(m, order[nf + i], x))
+                                                          << (8 * (i % 8));
             }
-        if (nw & 1)
-            for (int x = 0; x < 1024; ++x) words.push_back(entry[(size_t)x * nw + nw - 1]);
+            (n8 ? L.n8_off : L.words_off) = words.size() * 8;
+            for (int j = 0; j < nw / 2; ++j)
+                for (int x = 0; x < kCompactEntries; ++x) {
+                    words.push_back(entry[(size_t)x * nw + 2 * j]);
+                    words.push_back(entry[(size_t)x * nw + 2 * j + 1]);
+                }
+            if (nw & 1)
+                for (int x = 0; x < kCompactEntries; ++x) words.push_back(entry[(size_t)x * nw + nw - 1]);
+        }
         for (int k = 0; k < P; ++k) {
             const int q = order[k];
-            for (int c = 0; c < 32; ++c) syms.push_back(m->h_f1[(size_t)q * 32 + c]);
             L.prm.win4[k] = m->win4[q];
             L.prm.start[k] = m->start[q];
             L.prm.dead[k] = m->dead[q];
@@ -176,13 +211,11 @@ int build_compact(trex_dfa_multi* m) {
         fc.push_back(L);
     }
     hipFree(m->d_fc);
-    hipFree(m->d_fcs);
-    m->d_fc = m->d_fcs = nullptr;
+    m->d_fc = nullptr;
     m->fc_group = -1;
     TREX_TRY(upload((void**)&m->d_fc, words.data(), words.size() * 8));
-    TREX_TRY(upload((void**)&m->d_fcs, syms.data(), syms.size() * 8));
     m->fc = std::move(fc);
-    m->fc_group = m->group;
+    m->fc_group = group;
     return TREX_OK;
 }
 
@@ -196,10 +229,20 @@ int auto_form(const trex_dfa_multi* m) {
     return small >= 2 ? TREX_DFA_MULTI_K2F_COMPACT : TREX_DFA_MULTI_K2F_PAIRED;
 }
 
+// Patterns per launch of the compact form where the handle uses it, else 0:
+// contiguous strings run it whatever the default form is, unless the caller
+// chose a form or a group: its kernels read aligned vectors and order the
+// strings (2 patterns of 9 states, 50,000 x 200..3000 bytes: 59 us paired, 44
+// us so; 262,144 x 4 KiB: 281 us and 257 us).
+int compact_group(const trex_dfa_multi* m) {
+    return m->form == TREX_DFA_MULTI_K2F_COMPACT ? m->group : m->picked ? kMultiMax : 0;
+}
+
 // (Re)builds the tables the handle's form needs for its grouping.
 int ensure_tables(trex_dfa_multi* m) {
     if (m->form == TREX_DFA_MULTI_K2F_PAIRED && m->fp_group != m->group) TREX_TRY(build_paired(m));
-    if (m->form == TREX_DFA_MULTI_K2F_COMPACT && m->fc_group != m->group) TREX_TRY(build_compact(m));
+    const int group = compact_group(m);
+    if (group > 0 && m->fc_group != group) TREX_TRY(build_compact(m, group));
     return TREX_OK;
 }
 
@@ -215,7 +258,6 @@ int trex_dfa_multi_destroy(trex_dfa_multi* m) {
     hipFree(m->d_t1);
     hipFree(m->d_fp);
     hipFree(m->d_fc);
-    hipFree(m->d_fcs);
     delete m;
     return TREX_OK;
 }
@@ -283,15 +325,21 @@ int trex_dfa_multi_create(trex_dfa* const* patterns, int n_patterns, trex_dfa_mu
 
 int trex_dfa_multi_set_form(trex_dfa_multi* m, int form) {
     if (!m) return fail(TREX_ERR_INVALID, "null handle");
-    if (form == TREX_DFA_AUTO) form = auto_form(m);
+    const bool picked = form == TREX_DFA_AUTO;
+    if (picked) form = auto_form(m);
     if (form != TREX_DFA_K2_WINDOW_F && form != TREX_DFA_K2_WINDOW && form != TREX_DFA_MULTI_K2F_PAIRED &&
         form != TREX_DFA_MULTI_K2F_COMPACT)
         return fail(TREX_ERR_INVALID, "form %d: use TREX_DFA_K2_WINDOW_F, TREX_DFA_K2_WINDOW, "
                     "TREX_DFA_MULTI_K2F_PAIRED or TREX_DFA_MULTI_K2F_COMPACT", form);
     const int prev = m->form;
+    const bool prev_picked = m->picked;
     m->form = form;
+    m->picked = picked;
     const int rc = ensure_tables(m);
-    if (rc) m->form = prev;
+    if (rc) {
+        m->form = prev;
+        m->picked = prev_picked;
+    }
     return rc;
 }
 
@@ -299,6 +347,7 @@ int trex_dfa_multi_set_group(trex_dfa_multi* m, int group) {
     if (!m) return fail(TREX_ERR_INVALID, "null handle");
     if (group < 1 || group > kMultiMax) return fail(TREX_ERR_INVALID, "group=%d outside 1..%d", group, kMultiMax);
     m->group = group;
+    m->picked = false;
     return ensure_tables(m);
 }
 
@@ -320,19 +369,21 @@ int multi_dispatch(trex_dfa_multi* m, const uint8_t* d_bytes, const int64_t* d_b
     if (n_strings < 0) return fail(TREX_ERR_INVALID, "n_strings < 0");
     if (n_strings == 0) return TREX_OK;
     if (!d_bytes || !d_begin || !d_end || !d_final_state || !d_accept) return fail(TREX_ERR_INVALID, "null buffer");
-    const int64_t grid64 = (n_strings + kBlock - 1) / kBlock;
+    const bool compact = m->form == TREX_DFA_MULTI_K2F_COMPACT || (m->picked && !il);
+    const unsigned block = compact && !il && n_strings < kCompactBlockFrom ? 64u : (unsigned)kBlock;
+    const int64_t grid64 = (n_strings + block - 1) / block;
     if (grid64 > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");
     const unsigned grid = (unsigned)grid64;
-    if (m->form == TREX_DFA_MULTI_K2F_COMPACT) {
-        if (m->fc_group != m->group) return fail(TREX_ERR_INVALID, "compact tables not built");
+    if (compact) {
+        if (m->fc_group != compact_group(m)) return fail(TREX_ERR_INVALID, "compact tables not built");
         for (const CompactLaunch& L : m->fc) {
-            const uint8_t* words = m->d_fc + L.words_off;
-            const uint8_t* syms = m->d_fcs + L.syms_off;
+            const bool n8 = L.n8 && !il;
+            const uint8_t* words = m->d_fc + (n8 ? L.n8_off : L.words_off);
             CompactParams prm = L.prm;
-            void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &words, &syms, &prm, &d_final_state, &d_accept};
+            void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &words, &prm, &d_final_state, &d_accept};
             char name[48];
-            std::snprintf(name, sizeof(name), "dfa16_multi_k2fc_f%d_b%d%s", L.nf, L.nb, il ? "_il" : "");
-            TREX_TRY(launch(name, grid, kBlock, 0, (hipStream_t)stream, args));
+            std::snprintf(name, sizeof(name), "dfa16_multi_k2fc_f%d_b%d%s", L.nf, L.nb, il ? "_il" : n8 ? "_n8" : "");
+            TREX_TRY(launch(name, grid, block, 0, (hipStream_t)stream, args));
         }
         return TREX_OK;
     }
