@@ -155,8 +155,11 @@ int trex_dfa_set_prefetch(trex_dfa* h, int vectors);
  * transition function of the part read first until it turns constant. Equal
  * strings packed back to back are then not all read at the same offset
  * modulo 4 KiB at once, which crowds a few HBM channels. Same results.
- * mode -1 (default): on when the table synchronises (some word over its
- * window bytes sends every state that can occur to one state); 0 off; 1 on.
+ * mode -1 (default): on for batches of 131,072 strings and more whose table
+ * synchronises (some word over its window bytes sends every state that can
+ * occur to one state), for the workgroups whose strings are alike; 0 off; 1 on
+ * for every launch of that kernel. With a mode of 0 or 1 contiguous strings
+ * are walked in the handle's variant, otherwise by byte classes.
  * No counterpart in the reference (its kernels read strings as packed,
  * cuda/monoid_batch.cu:58-95). trex_dfa_rotation reports whether launches
  * use it and whether the table synchronises. */
@@ -214,7 +217,9 @@ int trex_dfa_multi_destroy(trex_dfa_multi* m);
  * full functions: fewer table reads per byte pair; rebuilt when the group
  * changes), TREX_DFA_K2_WINDOW_F (8 KB of LDS per pattern) or
  * TREX_DFA_K2_WINDOW (16 KB per pattern). TREX_DFA_AUTO (and a new handle):
- * compact when at least two patterns have at most 4 states, else paired. */
+ * compact when at least two patterns have at most 4 states, else paired;
+ * contiguous strings then always run the compact form, 8 patterns a launch,
+ * unless a group is set. */
 #define TREX_DFA_MULTI_K2F_PAIRED 7
 #define TREX_DFA_MULTI_K2F_COMPACT 8
 int trex_dfa_multi_set_form(trex_dfa_multi* m, int form);
@@ -258,7 +263,9 @@ int trex_nfa_create(const uint64_t* succ, int n_symbols, const int16_t* byte_to_
 int trex_nfa_destroy(trex_nfa* h);
 /* The variant chosen at create time: TREX_NFA_WINDOW6 when every byte outside
  * one aligned 32-byte window rejects, else TREX_NFA_BYTES; set_variant forces
- * another the automaton allows. */
+ * another the automaton allows. Without a forced variant, an automaton that
+ * reaches at most 256 state sets walks contiguous strings as a DFA over those
+ * sets (same results). */
 int trex_nfa_info(const trex_nfa* h, int* variant, int* window_base);
 int trex_nfa_set_variant(trex_nfa* h, int variant);
 /* Final state mask and accept bit ((mask & accept) != 0) per string. */
@@ -311,7 +318,9 @@ int trex_pnfa_destroy(trex_pnfa* h);
 int trex_pnfa_info(const trex_pnfa* h, int* mode, int* n_symbols, int* f16_ok, int* waves);
 int trex_pnfa_set_mode(trex_pnfa* h, int mode);
 /* Waves per 64-sequence workgroup: 4 (eight symbols' matrices per wave) or 8
- * (four per wave, two waves per SIMD). */
+ * (four per wave, two waves per SIMD). Until it is called, batches of at most
+ * 32 sequences per compute unit run in workgroups of four waves and fewer
+ * sequences, as few as leave each workgroup a compute unit (same results). */
 int trex_pnfa_set_waves(trex_pnfa* h, int waves);
 /* Most workgroups per kernel launch (0, the default: one per group of 64
  * sequences). With fewer, the groups go out in consecutive launches on the
@@ -374,7 +383,11 @@ int trex_mix_destroy(trex_mix* m);
 /* String i = bytes[begin[i] .. end[i]) is matched against pattern
  * pattern_of[i]. Strings longer than dfa_split / nfa_split bytes are cut into
  * chunks of dfa_chunk (multiple of 16) / nfa_chunk (multiple of ck) bytes;
- * NFA chunks record their state set every ck bytes (ck multiple of 16).
+ * NFA chunks record their state set every ck bytes (ck multiple of 16). In a
+ * batch too small to fill the device with such chunks, lengths above 4,096 are
+ * upper bounds: strings are cut shorter, down to 1,024 (DFA) and 512 (NFA)
+ * bytes, and NFA chunks then start from the set a walk of the bytes ahead of
+ * them reaches instead of recording sets. Results are the same.
  * Host work only: the plan is staged in pinned memory and copied to the
  * device, asynchronously and by a copy kernel, by the next trex_mix_run or
  * trex_mix_capture on that call's stream (device buffers grow there too, in

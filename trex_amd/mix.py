@@ -30,7 +30,9 @@ BLOCK = 512   # lane items per work batch (one workgroup)
 @dataclass
 class MixParams:
     """Split lengths, chunk lengths and checkpoint spacing of a plan, and the
-    NFA table form ("nibble" / "slice"; None keeps the engine's form)."""
+    NFA table form ("nibble" / "slice"; None keeps the engine's form). Lengths
+    above 4,096 are upper bounds: a batch too small to fill the device with
+    such chunks is cut shorter."""
     dfa_split: int = 256 << 10
     dfa_chunk: int = 64 << 10
     nfa_split: int = 32 << 10
