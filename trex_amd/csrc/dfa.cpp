@@ -342,13 +342,18 @@ int trex_dfa_match_host(trex_dfa* h, const uint8_t* bytes, const int64_t* offset
     std::lock_guard<std::mutex> lock(h->mu);
     const size_t n = (size_t)n_strings, row = align_up(n, 16);
     const size_t bytes_at = align_up(sizeof(int64_t) * (n + 1), 256);   // device batch: offsets, then bytes
-    const bool offsets_staged = bytes_at <= kPinnedIn, bytes_staged = bytes_at + (size_t)total <= kPinnedIn;
-    const bool results_staged = 2 * row <= kPinnedOut;
+    // (without pinned memory to be had, everything is copied as it is)
+    if (!h->pinned && hipHostMalloc((void**)&h->pinned, kPinnedIn + kPinnedOut, hipHostMallocDefault) != hipSuccess) {
+        h->pinned = nullptr;
+        (void)hipGetLastError();
+    }
+    const bool offsets_staged = h->pinned && bytes_at <= kPinnedIn;
+    const bool bytes_staged = h->pinned && bytes_at + (size_t)total <= kPinnedIn;
+    const bool results_staged = h->pinned && 2 * row <= kPinnedOut;
     TREX_TRY(h->in_bytes.reserve(bytes_at + (size_t)total + 16));
     TREX_TRY(h->out_state.reserve(results_staged ? 0 : n));
     TREX_TRY(h->out_accept.reserve(results_staged ? 0 : n));
     TREX_TRY(ensure_host_dispatch(h->stream, h->ev));
-    if (!h->pinned) TREX_HIP(hipHostMalloc((void**)&h->pinned, kPinnedIn + kPinnedOut, hipHostMallocDefault), "pinned staging");
     // Offsets are rebased so the device batch starts at byte 0.
     std::vector<int64_t> unstaged(offsets_staged ? 0 : n + 1);
     int64_t* rebased = offsets_staged ? reinterpret_cast<int64_t*>(h->pinned) : unstaged.data();
