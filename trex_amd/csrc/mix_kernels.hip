@@ -475,9 +475,9 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
                 stage_table(lds + 20480, P.f2, 8192);
                 stage_table(lds + 28672, P.acc, 16);
             } else if constexpr (SLICE) {
-                stage_table(lds, P.ntab, (int)kTab6Bytes);
+                stage_table_far(lds, P.ntab, (int)kTab6Bytes);
             } else {
-                stage_table(lds, P.ntab, kNfaClasses * 2048);
+                stage_table_far(lds, P.ntab, kNfaClasses * 2048);
                 stage_table(lds + kNfaClasses * 2048, P.ncls, 256);
             }
             __syncthreads();

@@ -111,7 +111,7 @@ __device__ __forceinline__ void nfa_slice5_kernel(const uint8_t* __restrict__ by
                                             uint8_t* __restrict__ out_accept)
 {
     __shared__ __attribute__((aligned(16))) char tb[kTab5Bytes];
-    stage_table(reinterpret_cast<uint8_t*>(tb), tabg, (int)kTab5Bytes);
+    stage_table_far(reinterpret_cast<uint8_t*>(tb), tabg, (int)kTab5Bytes);
     auto step = [&](uint32_t k, uint64_t x) { return nfa5_step(tb, k, x); };
     __syncthreads();
 
@@ -164,7 +164,7 @@ __device__ __forceinline__ void nfa_slice6_kernel(const uint8_t* __restrict__ by
     __shared__ __attribute__((aligned(16))) char tb[kTab6Bytes + (LANES == 1 ? order_bytes(TREX_NFA5_BLOCK) : 0u)];
     const uint32_t q = threadIdx.x % LANES;
     int64_t sid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
-    stage_table(reinterpret_cast<uint8_t*>(tb), tabg, (int)kTab6Bytes);
+    stage_table_far(reinterpret_cast<uint8_t*>(tb), tabg, (int)kTab6Bytes);
     if constexpr (LANES == 1) {
         const int64_t first = (int64_t)blockIdx.x * blockDim.x;
         const uint32_t n_here = (uint32_t)min<int64_t>(n_strings - first, blockDim.x);
