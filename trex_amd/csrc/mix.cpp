@@ -50,6 +50,8 @@ struct MixPattern {
     uint64_t nstart;
     uint64_t naccept;
     uint64_t nguess;
+    uint64_t nsecond;
+    Sticky sticky[kSticky];
     const uint8_t* t1;
     const uint8_t* t2;
     const uint8_t* f2;
@@ -80,6 +82,7 @@ struct MixArgs {
     uint64_t* agg;
     uint32_t* done;
     uint32_t* unmet;
+    uint64_t* found;
     uint64_t* ckpt;
     uint64_t* spec_exit;
     uint32_t* error;
@@ -150,7 +153,7 @@ struct trex_mix {
     hipEvent_t staged = nullptr;   // recorded behind the last upload from h_stage
     bool staged_pending = false;
     DevBuf d_plan;
-    DevBuf d_words;   // ticket, error, converged, done[n_slots], unmet[n_slots], status[n_items]
+    DevBuf d_words;   // ticket, error, converged, 0, found[n_slots] (64 bits each), done[n_slots], unmet[n_slots], status[n_items]
     DevBuf d_agg, d_ckpt, d_exit;
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -216,10 +219,10 @@ int stage_plan(trex_mix* m) {
         if (sizes[i]) std::memcpy(m->h_stage + m->off[i], srcs[i], sizes[i]);
     m->plan_bytes = total;
     m->need[0] = total;
-    m->need[1] = 4 * (3 + 2 * (size_t)Q.n_slots + Q.items());
+    m->need[1] = 4 * (4 + 4 * (size_t)Q.n_slots + Q.items());
     m->need[2] = 16 * std::max<size_t>(Q.items(), 1);
     m->need[3] = 8 * std::max<size_t>((size_t)Q.n_spec * Q.n_ck, 1);
-    m->need[4] = 8 * std::max<size_t>((size_t)Q.n_spec, 1);
+    m->need[4] = 16 * std::max<size_t>((size_t)Q.n_spec, 1);
     m->dirty = true;
     return TREX_OK;
 }
@@ -319,6 +322,8 @@ int trex_mix_create(const int32_t* kinds, const void* const* handles, int32_t n_
                 P.nstart = f->start;
                 P.naccept = f->accept;
                 P.nguess = f->guess;
+                P.nsecond = f->second;
+                std::copy(f->sticky, f->sticky + kSticky, P.sticky);
                 P.ntab = reinterpret_cast<const uint8_t*>(f->d_tab_win);
                 P.ncls = f->d_cls_win;
             }
@@ -552,7 +557,7 @@ int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint
     hipStream_t s = (hipStream_t)stream;
     TREX_TRY(upload_plan(m, s));
     uint32_t* words = m->d_words.as<uint32_t>();
-    int64_t n_words = 3 + 2 * Q.n_slots + (int64_t)Q.items();
+    int64_t n_words = 4 + 4 * Q.n_slots + (int64_t)Q.items();
     uint32_t zero = 0;
     {
         const unsigned grid = (unsigned)std::min<int64_t>((n_words + kBlock - 1) / kBlock, 4096);
@@ -581,7 +586,8 @@ int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint
     a.ticket = words;
     a.error = words + 1;
     a.converged = words + 2;
-    a.done = words + 3;
+    a.found = reinterpret_cast<uint64_t*>(words + 4);
+    a.done = words + 4 + 2 * Q.n_slots;
     a.unmet = a.done + Q.n_slots;
     a.status = a.unmet + Q.n_slots;
     a.agg = m->d_agg.as<uint64_t>();

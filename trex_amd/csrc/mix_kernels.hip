@@ -15,19 +15,20 @@
 //   NFA_SPEC   one chunk of a long string: the first chunk of the string is
 //              walked from the start set; every other chunk is walked from
 //              the pattern's guess set `warm` bytes ahead of it, which makes a
-//              guess of the set it is entered with, and on to its end. The
-//              guess is right when the chunk before it ends in that set (taken
-//              from the neighbouring lane, or published by the wave before)
-//              and was entered with the right set itself. Long chunks also
-//              record their set every kCk bytes (checkpoints)
+//              guess of the set it is entered with, and on to its end (some
+//              patterns have a second guess: NFA handle). Its end is known when
+//              the chunk before it ends in that set (taken from the
+//              neighbouring lane, or published by the wave before) and was
+//              entered with the right set itself, up to sticky sets
+//              (known_end(): text that was found before stays found). Long chunks also record their set every kCk bytes (checkpoints)
 //   NFA_FIXUP  one lane per long string, after all its NFA_SPEC chunks are
-//              done: when every guess was its predecessor's end, the last end
-//              is the string's. Otherwise it goes from chunk to chunk: where
-//              the true set is the guess, the chunk's end is known; any other
-//              chunk is walked again from the true set, with checkpoints only
-//              until the set equals the one recorded at the same position,
-//              after which both walks coincide. An empty set ends it (the
-//              empty set is absorbing). The result is exact either way.
+//              done: when every chunk's guess was right, the last end and the
+//              sticky sets found on the way are the string's. Otherwise it goes
+//              from chunk to chunk: where the guesses make the chunk's end
+//              known, that is taken; any other chunk is walked again from the
+//              true set, with checkpoints only until the set recorded at the
+//              same position makes the end known. An empty set ends it (the empty set is absorbing).
+//              The result is exact either way.
 //
 // Forward progress: the queue puts every batch that is waited on before the
 // batches that wait on it (DFA chunks after their predecessors, fix-ups after
@@ -55,6 +56,13 @@ constexpr uint32_t kStatusAggregate = 1u, kStatusPrefix = 2u;
 constexpr int kNfaClasses = 34;   // window bytes 0..31, reject, skip
 constexpr int kFixupBlock = 4;    // chunks a fix-up reads at once
 
+constexpr int kSticky = 4;
+
+struct Sticky {
+    uint64_t state;   // a state outside the start set that every symbol keeps (a mask; 0: unused)
+    uint64_t set;     // what it leads to, closed under every symbol
+};
+
 // Pattern descriptor (host layout in mix.cpp).
 struct MixPattern {
     uint32_t kind;        // 0 DFA, 1 NFA
@@ -66,6 +74,8 @@ struct MixPattern {
     uint64_t nstart;      // NFA start set
     uint64_t naccept;     // NFA accept set
     uint64_t nguess;      // NFA set a chunk's guess is walked from
+    uint64_t nsecond;     // and its second guess, 0: none
+    Sticky sticky[kSticky];   // of NFAs whose guesses are walked from the start set
     const uint8_t* t1;    // DFA byte table [256][16]
     const uint8_t* t2;    // DFA pair rows [1024][16]
     const uint8_t* f2;    // DFA pair functions [1024] x uint64
@@ -93,11 +103,12 @@ struct MixArgs {
     int32_t warm;             // bytes walked ahead of a NFA_SPEC chunk for its guess (at most a chunk)
     uint32_t* ticket;
     uint32_t* status;         // per item (DFA_CHUNK; NFA_SPEC: 1 once its end is published)
-    uint64_t* agg;            // two words per item (DFA_CHUNK: function, item to go on from; NFA_SPEC: guess)
+    uint64_t* agg;            // two words per item (DFA_CHUNK: function, item to go on from; NFA_SPEC: both guesses)
     uint32_t* done;           // per NFA string slot: finished NFA_SPEC chunks
-    uint32_t* unmet;          // per NFA string slot: chunks whose guess is not their predecessor's end
+    uint32_t* unmet;          // per NFA string slot: chunks whose guess is wrong after their predecessor's end
+    uint64_t* found;          // per NFA string slot: sticky sets reached in some chunk, missing from the next one's guess
     uint64_t* ckpt;           // [n_spec][n_ck]
-    uint64_t* spec_exit;      // [n_spec]
+    uint64_t* spec_exit;      // [n_spec][2], of both guesses
     uint32_t* error;
     uint32_t* converged;      // chunks whose end the fix-ups took as recorded
     uint32_t max_spins;       // wait bound in polls (0: none)
@@ -394,12 +405,42 @@ __device__ uint64_t nfa_walk_record(const uint8_t* __restrict__ bytes, int64_t p
     return nw.s;
 }
 
-// Walks [p, end) from set s and stops at the first multiple of ck whose set
-// equals ck_in[idx] (as nfa_walk_record stored them), reported through `met`.
+// The sticky sets that a set of states has reached.
+__device__ __forceinline__ uint64_t sticky_of(const MixPattern& P, uint64_t t) {
+    uint64_t u = 0;
+#pragma unroll 1   // (unrolled, the nibble kernel goes over 128 VGPRs)
+    for (int k = 0; k < kSticky && P.sticky[k].state != 0ull; ++k)
+        u |= (t & P.sticky[k].state) != 0ull ? P.sticky[k].set : 0ull;
+    return u;
+}
+
+// The end of a walk from `t` when walks over the same bytes from other sets make
+// it known. A step is linear in the set: a walk from g0 | g1 | sticky ends in
+// the ends of both guesses and the sticky sets, which stay as they are unless a
+// byte rejects and empties everything. (g0 holds a start state that every
+// symbol keeps unless it is empty itself: its end e0 is empty only then.)
+__device__ __forceinline__ bool known_end(const MixPattern& P, uint64_t t, uint64_t g0, uint64_t e0, uint64_t g1,
+                                          uint64_t e1, uint64_t& out) {
+    if (t == g0) {
+        out = e0;
+        return true;
+    }
+    if (g0 == 0ull) return false;
+    const uint64_t sticky = sticky_of(P, t);
+    if (t == (g0 | sticky)) e1 = 0ull;
+    else if (P.nsecond == 0ull || t != (g0 | g1 | sticky)) return false;   // (no second guess: g1, e1 not written)
+    out = e0 != 0ull ? e0 | e1 | sticky : 0ull;
+    return true;
+}
+
+// Walks [p, end) from set s, up to the first multiple of ck where the set
+// recorded there (ck_in, by nfa_walk_record; `stop` is that walk's end) makes
+// the end known: reported through `met`.
 template <bool SLICE>
 __device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
-                                  const void* tab, const uint8_t* cls, uint32_t win4, int32_t ck,
-                                  const uint64_t* __restrict__ ck_in, int32_t n_ck, bool& met) {
+                                  const void* tab, const uint8_t* cls, const MixPattern& P, int32_t ck,
+                                  const uint64_t* __restrict__ ck_in, int32_t n_ck, uint64_t stop, bool& met) {
+    const uint32_t win4 = P.win4;
     NfaWalker<SLICE> nw{tab, cls, s, {}};
     nw.w.init();
     met = false;
@@ -427,11 +468,9 @@ __device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, 
         next_ck += ck;
         if (idx < n_ck) {
             nw.settle(win4);
-            if (nw.s == ck_in[idx]) {
-                met = true;
-                return nw.s;
-            }
-            ++idx;
+            uint64_t out;
+            met = known_end(P, nw.s, ck_in[idx++], stop, 0ull, 0ull, out);
+            if (met) return out;
         }
     }
     nw.settle(win4);
@@ -463,7 +502,7 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
         __syncthreads();   // the previous batch is finished with LDS and s_batch
         if (threadIdx.x == 0) s_batch = (int32_t)atomicAdd(A.ticket, 1u);
         __syncthreads();
-        const int32_t b = s_batch;
+        const int32_t b = __builtin_amdgcn_readfirstlane(s_batch);   // uniform: the pattern is read by scalar loads
         if (b >= A.n_batches) break;
         const int32_t pat = A.bpattern[b];
         const uint32_t role = (uint32_t)A.brole[b];
@@ -505,17 +544,20 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
             const bool first = (A.iflags[item] & 1u) != 0;
             const int32_t o = A.ic[item];
             const int64_t p = A.ibeg[item], end = A.iend[item];
-            bool met;
-            uint64_t guess = 0, s = first ? P.nstart : P.nguess;
+            uint64_t guess = 0, s = 0, exit = 0;   // of the first guess
+            const int parts = P.nsecond != 0ull && !first ? 4 : 2;
 #pragma unroll 1
-            for (int part = 0; part < 2; ++part) {   // the bytes ahead, then the chunk: one copy of the walk
-                const int64_t from = part == 0 && !first ? p - A.warm : p;
+            for (int part = 0; part < parts; ++part) {   // the bytes ahead, then the chunk: one copy of the walk
+                const bool ahead = (part & 1) == 0;
+                if (ahead) s = first ? P.nstart : part == 0 ? P.nguess : P.nsecond;
+                else store_through(&A.agg[2 * item + (part >> 1)], s);
+                const int64_t from = ahead && !first ? p - A.warm : p;
                 if (part == 1) guess = s;
-                s = nfa_walk_record<SLICE>(A.bytes, from, part ? end : p, s, ntab, ncls, P.win4, A.ck,
-                                           A.ckpt + (int64_t)o * A.n_ck, part ? A.n_ck : 0);
+                s = nfa_walk_record<SLICE>(A.bytes, from, ahead ? p : end, s, ntab, ncls, P.win4, A.ck,
+                                           A.ckpt + (int64_t)o * A.n_ck, part == 1 ? A.n_ck : 0);
+                if (!ahead) store_through(&A.spec_exit[2 * (int64_t)o + (part >> 1)], s);
+                if (part == 1) exit = s;
             }
-            store_through(&A.spec_exit[o], s);
-            store_through(&A.agg[2 * item], guess);
             // the chunk before this one is the item before it: the lane below,
             // or the last lane of the wave before (of this batch or an earlier
             // one), which publishes before it waits itself
@@ -523,21 +565,27 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
             if (A.n_ck) __threadfence();   // checkpoints are ordinary stores
             wait_stores();
             if (lane == 63u || (int32_t)threadIdx.x == count - 1) store_relaxed(&A.status[item], 1u);
-            uint64_t before = (uint64_t)(uint32_t)__shfl_up((int)(uint32_t)s, 1, 64) |
-                              ((uint64_t)(uint32_t)__shfl_up((int)(uint32_t)(s >> 32), 1, 64) << 32);
-            met = first || lane > 0u;
+            uint64_t before = (uint64_t)(uint32_t)__shfl_up((int)(uint32_t)exit, 1, 64) |
+                              ((uint64_t)(uint32_t)__shfl_up((int)(uint32_t)(exit >> 32), 1, 64) << 32);
+            bool met = first || lane > 0u;
             if (!met) {
                 BoundedWait wait(A.max_spins, A.max_ticks);
                 while (!(met = load_relaxed(&A.status[item - 1]) != 0u) && !wait.expired())
                     __builtin_amdgcn_s_sleep(2);
-                before = load_through(&A.spec_exit[o - 1]);
+                before = load_through(&A.spec_exit[2 * (int64_t)(o - 1)]);
                 if (!met) atomicOr(A.error, 4u);
             }
-            met = met && (first || before == guess);
+            const int32_t slot = A.ia[item];
+            if (!first && before != guess) {
+                const uint64_t sticky = sticky_of(P, before);
+                met = met && guess != 0ull && before == (guess | sticky);   // as in known_end
+                // (once a string and sticky set, as a rule: later chunks find it there)
+                if (met && (sticky & ~load_through(&A.found[slot])) != 0ull)
+                    atomicOr(reinterpret_cast<unsigned long long*>(&A.found[slot]), (unsigned long long)sticky);
+            }
             // one atomic per string and wave (they are served one after another,
             // about 70 ns each: one per chunk of a long string adds up)
             wait_stores();
-            const int32_t slot = A.ia[item];
             bool left = true;
             for (uint64_t todo; (todo = __ballot(left)) != 0ull;) {
                 const int32_t of = __shfl(slot, (int)__builtin_ctzll(todo), 64);
@@ -570,32 +618,36 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
             uint32_t converged = 0;
             if (ok) {   // guesses and ends were written through before each chunk counted itself
                 if (A.n_ck) fence_acquire();
-                const int32_t o0 = A.ic[c0];
-                s = load_through(&A.spec_exit[o0]);   // the first chunk was walked from the start set
+                const int64_t o0 = A.ic[c0];
+                s = load_through(&A.spec_exit[2 * o0]);   // the first chunk was walked from the start set
                 int64_t from = c0 + 1;
                 if (load_relaxed(&A.unmet[A.ia[item]]) == 0u) {
                     converged = (uint32_t)(c1 - from);
-                    s = load_through(&A.spec_exit[o0 + (c1 - 1 - c0)]);
+                    s = load_through(&A.spec_exit[2 * (o0 + (c1 - 1 - c0))]);
+                    if (s != 0ull) s |= load_through(&A.found[A.ia[item]]);
                     from = c1;
                 }
                 // the empty set is absorbing: once the true set is empty, so are all later exits
                 for (int64_t c = from; c < c1 && s != 0; c += kFixupBlock) {
                     // guesses and ends of the next chunks (items and ordinals of a string are
                     // consecutive), read together
-                    uint64_t ends[kFixupBlock], guesses[kFixupBlock];
+                    uint64_t ends[kFixupBlock][2] = {}, guesses[kFixupBlock][2] = {};
 #pragma unroll
                     for (int k = 0; k < kFixupBlock; ++k) {
-                        const int64_t j = min(c + k, c1 - 1);
-                        ends[k] = load_through(&A.spec_exit[o0 + (j - c0)]);
-                        guesses[k] = load_through(&A.agg[2 * j]);
+                        const int64_t j = min(c + k, c1 - 1), o = o0 + (j - c0);
+                        ends[k][0] = load_through(&A.spec_exit[2 * o]);
+                        guesses[k][0] = load_through(&A.agg[2 * j]);
+                        if (P.nsecond != 0ull) {
+                            ends[k][1] = load_through(&A.spec_exit[2 * o + 1]);
+                            guesses[k][1] = load_through(&A.agg[2 * j + 1]);
+                        }
                     }
-                    bool known = true;   // all of them entered as guessed
+                    bool known = true;
                     uint64_t t = s;
 #pragma unroll
-                    for (int k = 0; k < kFixupBlock; ++k) {
-                        known = known && (c + k >= c1 || t == guesses[k]);
-                        if (c + k < c1) t = ends[k];
-                    }
+                    for (int k = 0; k < kFixupBlock; ++k)
+                        if (c + k < c1)
+                            known = known && known_end(P, t, guesses[k][0], ends[k][0], guesses[k][1], ends[k][1], t);
                     if (known) {
                         s = t;
                         converged += (uint32_t)min<int64_t>(kFixupBlock, c1 - c);
@@ -603,12 +655,12 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
                     }
                     for (int64_t j = c; j < min(c + kFixupBlock, c1) && s != 0; ++j) {
                         const int64_t o = o0 + (j - c0);
-                        const uint64_t stop = load_through(&A.spec_exit[o]);
-                        bool met = s == load_through(&A.agg[2 * j]);
+                        const uint64_t stop = load_through(&A.spec_exit[2 * o]);
+                        bool met = known_end(P, s, load_through(&A.agg[2 * j]), stop, load_through(&A.agg[2 * j + 1]),
+                                             load_through(&A.spec_exit[2 * o + 1]), s);
                         if (!met)
-                            s = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], s, ntab, ncls, P.win4, A.ck,
-                                                     A.ckpt + o * A.n_ck, A.n_ck, met);
-                        if (met) s = stop;
+                            s = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], s, ntab, ncls, P, A.ck,
+                                                     A.ckpt + o * A.n_ck, A.n_ck, stop, met);
                         converged += met ? 1u : 0u;
                     }
                 }

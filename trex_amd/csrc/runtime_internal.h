@@ -58,6 +58,15 @@ constexpr uint32_t kWaitBoundUs = 100000;
 // (each chunk walked front to back) or 2 (its two halves side by side).
 constexpr int kScanChains = 1;
 
+// A state outside the start set that every symbol keeps, with the set that every
+// symbol leads to from it. The set is closed under every symbol, so once it is
+// reached it stays as it is until a byte rejects: what a search automaton is in
+// when its text was found.
+struct Sticky {
+    uint64_t state, set;   // masks; state 0: unused
+};
+constexpr int kSticky = 4;
+
 // Byte-class form of a byte table (dfa_class_kernels.hip); d_tab is null when
 // the table has too many classes for it.
 struct ClassForm {
@@ -114,10 +123,10 @@ struct trex_dfa {
 struct trex_nfa {
     int n_symbols = 0;
     uint64_t start = 0, accept = 0;
-    // what walks of later chunks of a string start from: all states, or the start
-    // set for automata that keep a state outside it once it is reached (a text
-    // found stays found): from all states such a state is never lost again
-    uint64_t guess = ~0ull;
+    // What walks of later chunks of a string start from (see plan_guesses), and
+    // what the states outside the start set become once they are reached.
+    uint64_t guess = ~0ull, second = 0;
+    trex::Sticky sticky[trex::kSticky] = {};
     int window_base = -1;
     int variant = TREX_NFA_BYTES;
     int n_classes = 0, n_classes_win = 0;
