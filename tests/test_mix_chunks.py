@@ -82,3 +82,65 @@ def test_words_and_rejects_around_chunk_ends(gpu_lib, form):
                 if reject is not None:
                     data[base + int(rng.choice([at - 40, at - 1, at + 5, at + 300, size // 2, size - 1]) % size)] = reject
         _run(eng, data, offsets, MixParams(form=form))
+
+
+def _run_ms(eng, data, offsets, params):
+    """Time of the second of two runs."""
+    from trex_amd.device import DeviceBuffer, Event, Stream
+    n = len(offsets) - 1
+    m = MixEngine([eng])
+    m.plan(offsets[:-1], offsets[1:], np.zeros(n, np.int32), params)
+    stream = Stream()
+    d = DeviceBuffer.from_array(data, stream)
+    d_mask, d_acc = DeviceBuffer(8 * n), DeviceBuffer(n)
+    a, b = Event(), Event()
+    for event in (Event(), a):
+        event.record(stream)
+        m.run(d.ptr, d_mask.ptr, d_acc.ptr, stream)
+    b.record(stream)
+    stream.synchronize()
+    assert m.error(stream) == 0
+    return a.elapsed_ms(b)
+
+
+@pytest.mark.parametrize("form", ["nibble", "slice"])
+@pytest.mark.parametrize("params", [{}, {"nfa_split": 2048, "nfa_chunk": 1024}], ids=["open", "1 KiB"])
+def test_sets_that_coincide_late(gpu_lib, params, form):
+    """Walks from different sets coincide at a letter that comes every hundred
+    bytes: the walk ahead of a chunk mostly does not reach one, the chunk mostly
+    does. Walked again by one lane per string, chunk after chunk, 16 strings of
+    1 MiB take 180 ms and more."""
+    rng = np.random.default_rng(7)
+    eng = NfaEngine.from_matrices(compile_nfa_matrices("(([A-Y][A-Y][A-Y])*([A-Y]|[A-Y][A-Y])?Z)*([A-Y][A-Y][A-Y])*"))
+    params = MixParams(form=form, **params)
+    data, offsets = _strings(rng, np.array([200_000, 0, 5000, 64, 40_001, 33_000]))
+    data[data == ord("Z")] = ord("A")
+    rare = data.copy()
+    rare[rng.random(len(data)) < 0.002] = ord("Z")
+    _run(eng, rare, offsets, params)
+    data[rng.random(len(data)) < 0.01] = ord("Z")
+    _run(eng, data, offsets, params)
+    data, offsets = _strings(rng, np.full(16, 1 << 20))
+    data[data == ord("Z")] = ord("A")
+    data[rng.random(len(data)) < 0.01] = ord("Z")
+    assert _run_ms(eng, data, offsets, params) < 40
+
+
+@pytest.mark.parametrize("form", ["nibble", "slice"])
+@pytest.mark.parametrize("n", [500, 700])
+def test_fixups_by_wave_and_by_lane(gpu_lib, n, form):
+    """Up to two fix-ups a CU a wave each, beyond them a lane each: guesses that
+    are right, wrong to some letter, and always wrong, the empty set, and a
+    string of more than 64 chunks."""
+    rng = np.random.default_rng(n)
+    for pattern in ("(([A-Y][A-Y][A-Y])*([A-Y]|[A-Y][A-Y])?Z)*([A-Y][A-Y][A-Y])*", "([A-Z][A-Z][A-Z])*",
+                    "[A-Z]*ERROR[A-Z]*WARN[A-Z]*", "[A-Y]*(WARN)[A-Z]*"):
+        eng = NfaEngine.from_matrices(compile_nfa_matrices(pattern))
+        lengths = rng.integers(1100, 4000, n)
+        lengths[5] = 200_000
+        data, offsets = _strings(rng, lengths)
+        data[data == ord("Z")] = ord("A")
+        data[rng.random(len(data)) < 0.002] = ord("Z")
+        for at in rng.integers(0, len(data) - 5, 400):
+            data[at:at + 5] = np.frombuffer(rng.choice([b"ERROR", b"WARNE"]), np.uint8)
+        _run(eng, data, offsets, MixParams(nfa_split=1024, nfa_chunk=1024, ck=64, form=form))

@@ -102,6 +102,7 @@ struct Plan {
     int64_t n_spec = 0, n_slots = 0, n_chunks = 0, n_strings = 0;
     int32_t ck = 64, n_ck = 0, warm = 0;
     int32_t block = kMixBlock;   // lane items per batch = workgroup size of the form planned for
+    bool wave_fixups = false;    // fix-ups: one to a batch, by a wave each
 
     int32_t add(int64_t b, int64_t e, int32_t a, int32_t out, int32_t c, uint32_t flags) {
         ibeg.push_back(b);
@@ -417,11 +418,16 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
         const int64_t share = lanes / (kBatchesPerCu * device_cu_count());
         most = (int32_t)std::min<int64_t>(P.block, std::max<int64_t>((share + 63) / 64 * 64, 64));
     }
+    // A fix-up whose guesses were wrong walks chunks again, one after another by a
+    // lane, 64 at a time by a wave (measured in mix_kernels.hip): a wave each while
+    // all of them find a workgroup's place at once; beyond that lanes are more.
+    P.wave_fixups = fixups > 0 && m->has_device && fixups <= kBatchesPerCu * device_cu_count();
     std::vector<BatchRef> spec_b, chunk_b, fix_b, whole_b;
     auto cut = [&](int32_t first, int32_t n, int32_t pat, int32_t role, std::vector<BatchRef>& out,
                    const std::vector<int64_t>& keys) {
-        for (int32_t o = 0; o < n; o += most)
-            out.push_back({first + o, std::min(most, n - o), pat, role, keys.empty() ? 0 : keys[o]});
+        const int32_t width = role == (int32_t)kRoleNfaFixup && P.wave_fixups ? 1 : most;
+        for (int32_t o = 0; o < n; o += width)
+            out.push_back({first + o, std::min(width, n - o), pat, role, keys.empty() ? 0 : keys[o]});
     };
 
     // 1. NFA speculative chunks: each long string's chunks contiguous
@@ -506,7 +512,8 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
     // queue order
     std::stable_sort(chunk_b.begin(), chunk_b.end(), [](const BatchRef& a, const BatchRef& b) { return a.key < b.key; });
     std::stable_sort(whole_b.begin(), whole_b.end(), [](const BatchRef& a, const BatchRef& b) { return a.key < b.key; });
-    for (const auto* sec : {&spec_b, &chunk_b, &fix_b, &whole_b})
+    // (fix-ups that take a workgroup's place each wait behind the whole strings)
+    for (const auto* sec : {&spec_b, &chunk_b, P.wave_fixups ? &whole_b : &fix_b, P.wave_fixups ? &fix_b : &whole_b})
         for (const BatchRef& b : *sec) {
             P.bfirst.push_back(b.first);
             P.bcount.push_back(b.count);
@@ -605,8 +612,11 @@ int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint
     const int64_t want = m->grid > 0 ? m->grid : (sl ? 1 : 2) * (int64_t)device_cu_count();
     const unsigned grid = (unsigned)std::min<int64_t>(want, (int64_t)Q.bfirst.size());
     void* args[] = {&a};
-    if (sl) return launch("mix_persistent_slice", grid, kMixBlockSlice, kTabSliceBytes, s, args);
-    return launch("mix_persistent", grid, kMixBlock, kNfaClasses * 2048 + 256, s, args);
+    if (sl)
+        return launch(Q.wave_fixups ? "mix_persistent_slice_waves" : "mix_persistent_slice", grid, kMixBlockSlice,
+                      kTabSliceBytes, s, args);
+    return launch(Q.wave_fixups ? "mix_persistent_waves" : "mix_persistent", grid, kMixBlock, kNfaClasses * 2048 + 256,
+                  s, args);
 }
 
 int trex_mix_set_form(trex_mix* m, int form) {

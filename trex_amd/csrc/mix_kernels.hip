@@ -21,14 +21,14 @@
 //              neighbouring lane, or published by the wave before) and was
 //              entered with the right set itself, up to sticky sets
 //              (known_end(): text that was found before stays found). Long chunks also record their set every kCk bytes (checkpoints)
-//   NFA_FIXUP  one lane per long string, after all its NFA_SPEC chunks are
-//              done: when every chunk's guess was right, the last end and the
-//              sticky sets found on the way are the string's. Otherwise it goes
-//              from chunk to chunk: where the guesses make the chunk's end
-//              known, that is taken; any other chunk is walked again from the
-//              true set, with checkpoints only until the set recorded at the
-//              same position makes the end known. An empty set ends it (the empty set is absorbing).
-//              The result is exact either way.
+//   NFA_FIXUP  one per long string, after all its NFA_SPEC chunks are done:
+//              when every chunk's guess was right, the last end and the sticky
+//              sets found on the way are the string's. Otherwise it goes over
+//              the chunks: where the guesses make a chunk's end known, that is
+//              taken; any other chunk is walked again from the set it is
+//              entered with, with checkpoints only until the set recorded at
+//              the same position makes the end known. The result is exact
+//              either way. Many strings take a lane each, few a wave each
 //
 // Forward progress: the queue puts every batch that is waited on before the
 // batches that wait on it (DFA chunks after their predecessors, fix-ups after
@@ -54,7 +54,7 @@ using namespace trexdev;
 constexpr uint32_t kRoleDfaWhole = 0, kRoleDfaChunk = 1, kRoleNfaWhole = 2, kRoleNfaSpec = 3, kRoleNfaFixup = 4;
 constexpr uint32_t kStatusAggregate = 1u, kStatusPrefix = 2u;
 constexpr int kNfaClasses = 34;   // window bytes 0..31, reject, skip
-constexpr int kFixupBlock = 4;    // chunks a fix-up reads at once
+constexpr int kFixupBlock = 4;    // chunks a fix-up of one lane reads at once
 
 constexpr int kSticky = 4;
 
@@ -136,7 +136,7 @@ __device__ __forceinline__ uint32_t k2f_word(const uint64_t* __restrict__ f2, ui
     return (uint32_t)(b >> (s << 2)) & 15u;
 }
 
-__device__ uint32_t dfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, const DfaLds& L,
+__device__ __forceinline__ uint32_t dfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, const DfaLds& L,
                              const MixPattern& P) {
     uint32_t s = P.start;
     const Span sp(bytes, p, end);
@@ -355,7 +355,7 @@ struct NfaWalker {
 };
 
 template <bool SLICE>
-__device__ uint64_t nfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
+__device__ __forceinline__ uint64_t nfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
                              const void* tab, const uint8_t* cls, uint32_t win4) {
     NfaWalker<SLICE> nw{tab, cls, s, {}};
     nw.w.init();
@@ -374,7 +374,7 @@ __device__ uint64_t nfa_walk(const uint8_t* __restrict__ bytes, int64_t p, int64
 // is a multiple of ck (ck a multiple of 16) into ck_out[0..n_ck); n_ck = 0
 // stores none.
 template <bool SLICE>
-__device__ uint64_t nfa_walk_record(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
+__device__ __forceinline__ uint64_t nfa_walk_record(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
                                     const void* tab, const uint8_t* cls, uint32_t win4, int32_t ck,
                                     uint64_t* __restrict__ ck_out, int32_t n_ck) {
     NfaWalker<SLICE> nw{tab, cls, s, {}};
@@ -414,30 +414,37 @@ __device__ __forceinline__ uint64_t sticky_of(const MixPattern& P, uint64_t t) {
     return u;
 }
 
-// The end of a walk from `t` when walks over the same bytes from other sets make
-// it known. A step is linear in the set: a walk from g0 | g1 | sticky ends in
-// the ends of both guesses and the sticky sets, which stay as they are unless a
-// byte rejects and empties everything. (g0 holds a start state that every
-// symbol keeps unless it is empty itself: its end e0 is empty only then.)
-__device__ __forceinline__ bool known_end(const MixPattern& P, uint64_t t, uint64_t g0, uint64_t e0, uint64_t g1,
-                                          uint64_t e1, uint64_t& out) {
-    if (t == g0) {
-        out = e0;
+// The end of a walk from `t` when a walk over the same bytes from g, which ends
+// in e, makes it known. A step is linear in the set: a walk from g | sticky ends
+// in e and the sticky sets, which stay as they are unless a byte rejects and
+// empties everything. (g holds a start state that every symbol keeps unless it
+// is empty itself: e is empty only then.)
+__device__ __forceinline__ bool known_end(const MixPattern& P, uint64_t t, uint64_t g, uint64_t e, uint64_t& out) {
+    if (t == g) {
+        out = e;
         return true;
     }
-    if (g0 == 0ull) return false;
     const uint64_t sticky = sticky_of(P, t);
-    if (t == (g0 | sticky)) e1 = 0ull;
-    else if (P.nsecond == 0ull || t != (g0 | g1 | sticky)) return false;   // (no second guess: g1, e1 not written)
-    out = e0 != 0ull ? e0 | e1 | sticky : 0ull;
+    if (g == 0ull || t != (g | sticky)) return false;
+    out = e != 0ull ? e | sticky : 0ull;
     return true;
+}
+
+// The same with a second guess, whose set and end are g1 and e1 (in memory:
+// written, and needed, for few patterns).
+__device__ __forceinline__ bool known_end(const MixPattern& P, uint64_t t, uint64_t g, uint64_t e,
+                                          const uint64_t* __restrict__ g1, const uint64_t* __restrict__ e1,
+                                          uint64_t& out) {
+    if (known_end(P, t, g, e, out)) return true;
+    return P.nsecond != 0ull && g != 0ull &&
+           known_end(P, t, g | load_through(g1), e != 0ull ? e | load_through(e1) : 0ull, out);
 }
 
 // Walks [p, end) from set s, up to the first multiple of ck where the set
 // recorded there (ck_in, by nfa_walk_record; `stop` is that walk's end) makes
 // the end known: reported through `met`.
 template <bool SLICE>
-__device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
+__device__ __forceinline__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, int64_t end, uint64_t s,
                                   const void* tab, const uint8_t* cls, const MixPattern& P, int32_t ck,
                                   const uint64_t* __restrict__ ck_in, int32_t n_ck, uint64_t stop, bool& met) {
     const uint32_t win4 = P.win4;
@@ -469,7 +476,7 @@ __device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, 
         if (idx < n_ck) {
             nw.settle(win4);
             uint64_t out;
-            met = known_end(P, nw.s, ck_in[idx++], stop, 0ull, 0ull, out);
+            met = known_end(P, nw.s, ck_in[idx++], stop, out);
             if (met) return out;
         }
     }
@@ -479,15 +486,167 @@ __device__ uint64_t nfa_walk_meet(const uint8_t* __restrict__ bytes, int64_t p, 
     return nw.s;
 }
 
+// Waits for the chunks of a fix-up's string. True when its end is known, false
+// when some guess was wrong; s is then the end of the first chunk.
+__device__ __forceinline__ bool fixup_known(const MixArgs& A, int64_t item, uint64_t& s, uint32_t& converged) {
+    const int64_t c0 = A.ibeg[item], c1 = A.iend[item];
+    const uint32_t need = (uint32_t)(c1 - c0);
+    const int32_t slot = A.ia[item];
+    const int64_t o0 = A.ic[c0];
+    s = 0;
+    converged = 0;
+    BoundedWait wait(A.max_spins, A.max_ticks);
+    while (load_relaxed(&A.done[slot]) < need) {
+        if (wait.expired()) {
+            atomicOr(A.error, 4u);
+            return true;
+        }
+        __builtin_amdgcn_s_sleep(8);
+    }
+    // guesses and ends were written through before each chunk counted itself
+    if (A.n_ck) fence_acquire();
+    const uint64_t first = load_through(&A.spec_exit[2 * o0]), last = load_through(&A.spec_exit[2 * (o0 + need - 1)]);
+    const uint64_t found = load_through(&A.found[slot]);
+    const bool known = load_relaxed(&A.unmet[slot]) == 0u;
+    s = !known ? first : last != 0ull ? last | found : 0ull;   // (the first chunk was walked from the start set)
+    if (known) converged = need - 1u;
+    return known;
+}
+
+__device__ __forceinline__ void fixup_result(const MixArgs& A, const MixPattern& P, int64_t item, uint64_t s,
+                                             uint32_t converged) {
+    if (converged != 0u) atomicAdd(A.converged, converged);
+    A.out_mask[A.ib[item]] = s;
+    A.out_accept[A.ib[item]] = (s & P.naccept) != 0 ? 1 : 0;
+}
+
+// A string's fix-up by one lane, chunk after chunk.
+template <bool SLICE>
+__device__ __forceinline__ void fixup_lane(const MixArgs& A, const MixPattern& P, const void* ntab,
+                                           const uint8_t* ncls, int64_t item) {
+    uint64_t s;
+    uint32_t converged;
+    if (!fixup_known(A, item, s, converged)) {
+        const int64_t c0 = A.ibeg[item], c1 = A.iend[item], o0 = A.ic[c0];
+        // the empty set is absorbing: once the true set is empty, so are all later exits
+        for (int64_t c = c0 + 1; c < c1 && s != 0; c += kFixupBlock) {
+            // guesses and ends of the next chunks (items and ordinals of a string are
+            // consecutive), read together
+            uint64_t ends[kFixupBlock], guesses[kFixupBlock];
+#pragma unroll
+            for (int k = 0; k < kFixupBlock; ++k) {
+                const int64_t j = min(c + k, c1 - 1);
+                ends[k] = load_through(&A.spec_exit[2 * (o0 + (j - c0))]);
+                guesses[k] = load_through(&A.agg[2 * j]);
+            }
+            bool known = true;
+            uint64_t t = s;
+#pragma unroll
+            for (int k = 0; k < kFixupBlock; ++k) {
+                const int64_t j = c + k;
+                if (j < c1)
+                    known = known && known_end(P, t, guesses[k], ends[k], &A.agg[2 * j + 1],
+                                               &A.spec_exit[2 * (o0 + (j - c0)) + 1], t);
+            }
+            if (known) {
+                s = t;
+                converged += (uint32_t)min<int64_t>(kFixupBlock, c1 - c);
+                continue;
+            }
+            for (int64_t j = c; j < min(c + kFixupBlock, c1) && s != 0; ++j) {
+                const int64_t o = o0 + (j - c0);
+                const uint64_t stop = load_through(&A.spec_exit[2 * o]);
+                bool met = known_end(P, s, load_through(&A.agg[2 * j]), stop, &A.agg[2 * j + 1],
+                                     &A.spec_exit[2 * o + 1], s);
+                if (!met)
+                    s = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], s, ntab, ncls, P, A.ck,
+                                             A.ckpt + o * A.n_ck, A.n_ck, stop, met);
+                converged += met ? 1u : 0u;
+            }
+        }
+    }
+    fixup_result(A, P, item, s, converged);
+}
+
+// A string's fix-up by a whole wave, 64 chunks at a time: lane k has chunk k
+// enter with what chunk k - 1 ends in as far as it is known, and walks it again
+// where the guesses do not give its end for that set, until no entry set changes
+// any more. The first chunk's entry set is the true one, so each round makes at
+// least one more chunk final: where sets coincide somewhere in a chunk, one or
+// two rounds do, where they never do it takes as long as one lane. Walks that
+// coincide at a letter every 50 / 100 / 200 / 500 bytes, 16 strings of 1 MiB in
+// 512 byte chunks: 179 / 185 / 182 / 184 ms by a lane, 3.7 / 4.1 / 7.2 / 16.5 ms
+// by a wave; at no letter 185 and 220 ms.
+template <bool SLICE>
+__device__ __forceinline__ void fixup_wave(const MixArgs& A, const MixPattern& P, const void* ntab,
+                                           const uint8_t* ncls, int64_t item, uint64_t t) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const int64_t c0 = A.ibeg[item], c1 = A.iend[item], o0 = A.ic[c0];
+    uint32_t converged = 0;
+    auto lane_of = [](uint64_t x, int from) {
+        return (uint64_t)(uint32_t)__shfl((int)(uint32_t)x, from, 64) |
+               ((uint64_t)(uint32_t)__shfl((int)(uint32_t)(x >> 32), from, 64) << 32);
+    };
+    for (int64_t c = c0 + 1; c < c1 && t != 0ull; c += 64) {   // t: the true set so far, the same in every lane
+        const int64_t j = min(c + lane, c1 - 1), o = o0 + (j - c0);
+        const bool have = c + lane < c1;
+        const uint64_t g = load_through(&A.agg[2 * j]), e = load_through(&A.spec_exit[2 * o]);
+        auto entry = [&](uint64_t outs) {
+            const uint64_t up = lane_of(outs, (int)max(lane, 1u) - 1);
+            return lane > 0u ? up : t;
+        };
+        uint64_t in = entry(e), out = 0, walked_in = 0, walked_out = 0;   // (an empty set stays empty)
+        bool known;
+        while (true) {
+            known = known_end(P, in, g, e, &A.agg[2 * j + 1], &A.spec_exit[2 * o + 1], out);
+            if (!known) {
+                if (have && in != walked_in) {
+                    bool met;
+                    walked_in = in;
+                    walked_out = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], in, ntab, ncls, P, A.ck,
+                                                      A.ckpt + o * A.n_ck, A.n_ck, e, met);
+                }
+                out = walked_out;
+            }
+            const uint64_t next = entry(out);
+            if (__ballot(have && next != in) == 0ull) break;
+            in = next;
+        }
+        converged += (uint32_t)__popcll(__ballot(have && known));
+        t = lane_of(out, (int)min<int64_t>(c1 - 1 - c, 63));
+    }
+    if (lane == 0u) fixup_result(A, P, item, t, converged);
+}
+
+// Puts a pattern's tables in LDS unless they are there (layout in mix_loop).
+template <bool SLICE>
+__device__ __forceinline__ void stage_pattern(uint8_t* lds, const MixPattern& P, int32_t pat, int32_t& loaded) {
+    if (pat == loaded) return;
+    if (P.kind == 0) {
+        stage_table(lds, P.t1, 4096);
+        stage_table(lds + 4096, P.t2, 16384);
+        stage_table(lds + 20480, P.f2, 8192);
+        stage_table(lds + 28672, P.acc, 16);
+    } else if constexpr (SLICE) {
+        stage_table_far(lds, P.ntab, (int)kTab6Bytes);
+    } else {
+        stage_table_far(lds, P.ntab, kNfaClasses * 2048);
+        stage_table(lds + kNfaClasses * 2048, P.ncls, 256);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) loaded = pat;
+}
+
 // One persistent workgroup's loop. Dynamic LDS: the NFA tables of the form
 // (nibble: kNfaClasses * 2048 + 256 bytes; 6/5-bit slices: kTab6Bytes); the
 // DFA tables use the first 29 KB of the same space.
-template <bool SLICE>
+template <bool SLICE, bool WAVES>
 __device__ __forceinline__ void mix_loop(const MixArgs& A)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ int32_t s_batch;
     __shared__ int32_t s_loaded;
+    __shared__ int32_t s_walk;
     if (threadIdx.x == 0) s_loaded = -1;
 
     DfaLds dl;
@@ -507,25 +666,25 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
         const int32_t pat = A.bpattern[b];
         const uint32_t role = (uint32_t)A.brole[b];
         const MixPattern& P = A.patterns[pat];
-        if (pat != s_loaded) {
-            if (P.kind == 0) {
-                stage_table(lds, P.t1, 4096);
-                stage_table(lds + 4096, P.t2, 16384);
-                stage_table(lds + 20480, P.f2, 8192);
-                stage_table(lds + 28672, P.acc, 16);
-            } else if constexpr (SLICE) {
-                stage_table_far(lds, P.ntab, (int)kTab6Bytes);
-            } else {
-                stage_table_far(lds, P.ntab, kNfaClasses * 2048);
-                stage_table(lds + kNfaClasses * 2048, P.ncls, 256);
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) s_loaded = pat;
-        }
         const int32_t count = A.bcount[b];
         const bool active = (int32_t)threadIdx.x < count;
         const int64_t item = (int64_t)A.bfirst[b] + threadIdx.x;
 
+        if (WAVES && role == kRoleNfaFixup) {   // one string, the first wave; tables only if it walks
+            uint64_t s = 0;
+            uint32_t converged;
+            if (threadIdx.x < 64u) {
+                const bool known = fixup_known(A, A.bfirst[b], s, converged);
+                if (threadIdx.x == 0u) s_walk = known ? 0 : 1;
+                if (threadIdx.x == 0u && known) fixup_result(A, P, A.bfirst[b], s, converged);
+            }
+            __syncthreads();
+            if (s_walk == 0) continue;
+            stage_pattern<SLICE>(lds, P, pat, s_loaded);
+            if (threadIdx.x < 64u) fixup_wave<SLICE>(A, P, ntab, ncls, A.bfirst[b], s);
+            continue;
+        }
+        stage_pattern<SLICE>(lds, P, pat, s_loaded);
         if (role == kRoleDfaChunk) {
             // every lane takes part: the look-back publishes before it waits
             dfa_chunk(A, P, dl, item, active);
@@ -601,90 +760,24 @@ __device__ __forceinline__ void mix_loop(const MixArgs& A)
                     left = false;
                 }
             }
-        } else if (role == kRoleNfaFixup) {
-            const int64_t c0 = A.ibeg[item], c1 = A.iend[item];
-            const uint32_t need = (uint32_t)(c1 - c0);
-            BoundedWait wait(A.max_spins, A.max_ticks);
-            bool ok = true;
-            while (load_relaxed(&A.done[A.ia[item]]) < need) {
-                if (wait.expired()) {
-                    atomicOr(A.error, 4u);
-                    ok = false;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(8);
-            }
-            uint64_t s = 0;
-            uint32_t converged = 0;
-            if (ok) {   // guesses and ends were written through before each chunk counted itself
-                if (A.n_ck) fence_acquire();
-                const int64_t o0 = A.ic[c0];
-                s = load_through(&A.spec_exit[2 * o0]);   // the first chunk was walked from the start set
-                int64_t from = c0 + 1;
-                if (load_relaxed(&A.unmet[A.ia[item]]) == 0u) {
-                    converged = (uint32_t)(c1 - from);
-                    s = load_through(&A.spec_exit[2 * (o0 + (c1 - 1 - c0))]);
-                    if (s != 0ull) s |= load_through(&A.found[A.ia[item]]);
-                    from = c1;
-                }
-                // the empty set is absorbing: once the true set is empty, so are all later exits
-                for (int64_t c = from; c < c1 && s != 0; c += kFixupBlock) {
-                    // guesses and ends of the next chunks (items and ordinals of a string are
-                    // consecutive), read together
-                    uint64_t ends[kFixupBlock][2] = {}, guesses[kFixupBlock][2] = {};
-#pragma unroll
-                    for (int k = 0; k < kFixupBlock; ++k) {
-                        const int64_t j = min(c + k, c1 - 1), o = o0 + (j - c0);
-                        ends[k][0] = load_through(&A.spec_exit[2 * o]);
-                        guesses[k][0] = load_through(&A.agg[2 * j]);
-                        if (P.nsecond != 0ull) {
-                            ends[k][1] = load_through(&A.spec_exit[2 * o + 1]);
-                            guesses[k][1] = load_through(&A.agg[2 * j + 1]);
-                        }
-                    }
-                    bool known = true;
-                    uint64_t t = s;
-#pragma unroll
-                    for (int k = 0; k < kFixupBlock; ++k)
-                        if (c + k < c1)
-                            known = known && known_end(P, t, guesses[k][0], ends[k][0], guesses[k][1], ends[k][1], t);
-                    if (known) {
-                        s = t;
-                        converged += (uint32_t)min<int64_t>(kFixupBlock, c1 - c);
-                        continue;
-                    }
-                    for (int64_t j = c; j < min(c + kFixupBlock, c1) && s != 0; ++j) {
-                        const int64_t o = o0 + (j - c0);
-                        const uint64_t stop = load_through(&A.spec_exit[2 * o]);
-                        bool met = known_end(P, s, load_through(&A.agg[2 * j]), stop, load_through(&A.agg[2 * j + 1]),
-                                             load_through(&A.spec_exit[2 * o + 1]), s);
-                        if (!met)
-                            s = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], s, ntab, ncls, P, A.ck,
-                                                     A.ckpt + o * A.n_ck, A.n_ck, stop, met);
-                        converged += met ? 1u : 0u;
-                    }
-                }
-                atomicAdd(A.converged, converged);
-            }
-            A.out_mask[A.ib[item]] = s;
-            A.out_accept[A.ib[item]] = (s & P.naccept) != 0 ? 1 : 0;
+        } else if constexpr (!WAVES) {
+            fixup_lane<SLICE>(A, P, ntab, ncls, item);
         }
     }
 }
 
 }  // namespace
 
-// Nibble NFA tables: two 512-thread workgroups per CU (70 KB of LDS each).
-extern "C" __global__ void __launch_bounds__(MIX_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-mix_persistent(MixArgs A)
-{
-    mix_loop<false>(A);
-}
+// Nibble NFA tables: two 512-thread workgroups per CU (70 KB of LDS each). _waves:
+// a fix-up is one string to a batch and a wave, otherwise one to a lane.
+#define MIX_KERNEL(NAME, BLOCK, ...)                                                                       \
+    extern "C" __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) NAME(MixArgs A) { \
+        mix_loop<__VA_ARGS__>(A);                                                                          \
+    }
+MIX_KERNEL(mix_persistent, MIX_BLOCK, false, false)
+MIX_KERNEL(mix_persistent_waves, MIX_BLOCK, false, true)
 
 // 6/5-bit slice NFA tables (12 reads per byte instead of 16): one
 // 1024-thread workgroup per CU (128 KB of LDS).
-extern "C" __global__ void __launch_bounds__(MIX_BLOCK_SLICE) __attribute__((amdgpu_waves_per_eu(4)))
-mix_persistent_slice(MixArgs A)
-{
-    mix_loop<true>(A);
-}
+MIX_KERNEL(mix_persistent_slice, MIX_BLOCK_SLICE, true, false)
+MIX_KERNEL(mix_persistent_slice_waves, MIX_BLOCK_SLICE, true, true)
