@@ -404,7 +404,7 @@ int trex_mix_layout(const trex_mix* m, int64_t* ibeg, int64_t* iend, int32_t* ia
  * only written, so they may be pinned host memory (trex_host_alloc): the
  * results then need no copy back. d_out_mask[i] = DFA final state or NFA final set,
  * d_out_accept[i] = accept bit, for every planned string. Every wait of the
- * launch (a DFA chunk on an earlier chunk of another wave, a fix-up on its
+ * launch (a chunk on an earlier chunk of another wave, a fix-up on its
  * string's speculative chunks) ends after max_spins polls (0: no count limit)
  * or 100 ms of device wall-clock time, whichever comes first; on expiry the
  * launch still ends and trex_mix_error reports it. */
@@ -430,8 +430,9 @@ int trex_mix_set_form(trex_mix* m, int form);
 int trex_mix_status(trex_mix* m, void* dst, void* stream);
 /* Error word of the last run (0: no wait expired). Synchronises `stream`. */
 int trex_mix_error(trex_mix* m, uint32_t* error, void* stream);
-/* Speculative NFA chunks of the last run whose fix-up met a checkpoint (the
- * rest were walked to their end). Synchronises `stream`. */
+/* Speculative NFA chunks of the last run whose end was taken as recorded, their
+ * guess being right or its walk met at a checkpoint (the rest were walked again
+ * to their end). Synchronises `stream`. */
 int trex_mix_stats(trex_mix* m, uint32_t* converged, void* stream);
 /* Captures trex_mix_run into a HIP graph (non-default stream), replayed by
  * trex_mix_replay with the same buffers. */

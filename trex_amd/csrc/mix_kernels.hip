@@ -33,11 +33,11 @@
 // Forward progress: the queue puts every batch that is waited on before the
 // batches that wait on it (DFA chunks after their predecessors, fix-ups after
 // all NFA_SPEC batches), so every waited-on item has been claimed by a running
-// workgroup, and no waited-on work waits itself. A DFA chunk never waits on
-// a chunk of its own wave (those come by shuffle). Waits are bounded by a
+// workgroup, which publishes it before it waits itself. A DFA chunk never waits
+// on a chunk of its own wave (those come by shuffle). Waits are bounded by a
 // poll count (max_spins) and by wall-clock ticks (max_ticks); on expiry the
-// error word is set and the wave moves on (a NFA_SPEC lane that does not see
-// the end set before it in time leaves its chunk to the fix-up, no error).
+// error word is set and the wave moves on. Fix-ups of a wave each stand behind
+// the whole strings, since each holds a workgroup while it waits.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -130,7 +130,8 @@ class MixEngine:
         return e.value
 
     def converged(self, stream: Stream | None = None) -> int:
-        """Speculative NFA chunks of the last run whose fix-up met a checkpoint."""
+        """Speculative NFA chunks of the last run whose end was taken as recorded
+        (the guess of their entry set was right, or met the true one at a checkpoint)."""
         c = ctypes.c_uint32()
         _lib.call("trex_mix_stats", self.handle, ctypes.byref(c), stream.handle if stream else None)
         return c.value
