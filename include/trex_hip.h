@@ -383,11 +383,9 @@ int trex_mix_destroy(trex_mix* m);
 /* String i = bytes[begin[i] .. end[i]) is matched against pattern
  * pattern_of[i]. Strings longer than dfa_split / nfa_split bytes are cut into
  * chunks of dfa_chunk (multiple of 16) / nfa_chunk (multiple of ck) bytes;
- * NFA chunks record their state set every ck bytes (ck multiple of 16). In a
- * batch too small to fill the device with such chunks, lengths above 4,096 are
- * upper bounds: strings are cut shorter, down to 1,024 (DFA) and 512 (NFA)
- * bytes, and NFA chunks then start from the set a walk of the bytes ahead of
- * them reaches instead of recording sets. Results are the same.
+ * NFA chunks are entered with the set a walk of the bytes ahead of them
+ * reaches; those of 8,192 bytes and more also record their state set every ck
+ * bytes (ck multiple of 16).
  * Host work only: the plan is staged in pinned memory and copied to the
  * device, asynchronously and by a copy kernel, by the next trex_mix_run or
  * trex_mix_capture on that call's stream (device buffers grow there too, in
@@ -410,6 +408,10 @@ int trex_mix_layout(const trex_mix* m, int64_t* ibeg, int64_t* iend, int32_t* ia
  * launch still ends and trex_mix_error reports it. */
 int trex_mix_run(trex_mix* m, const uint8_t* d_bytes, uint64_t* d_out_mask, uint8_t* d_out_accept, uint32_t max_spins,
                  void* stream);
+/* Whether later plans take their lengths as upper bounds: with `on`, a batch too
+ * small to fill the device at the given lengths is cut shorter, down to 1,024
+ * (DFA) and 512 (NFA) bytes. 0 (a new handle): as given. Same results. */
+int trex_mix_set_refine(trex_mix* m, int on);
 /* Persistent workgroups of later runs (0: two per compute unit). Fewer leave
  * compute units to kernels on other streams. */
 int trex_mix_set_grid(trex_mix* m, int64_t workgroups);

@@ -104,6 +104,7 @@ _SIGNATURES = {
     # mixed batches
     "trex_mix_create": (c_int, [c_void_p, c_void_p, c_int, vpp]),
     "trex_mix_destroy": (c_int, [c_void_p]),
+    "trex_mix_set_refine": (c_int, [c_void_p, c_int]),
     "trex_mix_plan": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
                               c_int]),
     "trex_mix_info": (c_int, [c_void_p, i64p, i64p, i64p, i64p]),

@@ -87,14 +87,14 @@ def _length_summary(lengths: np.ndarray) -> list:
 
 def tune_mix(engines, begin, end, pattern_of, d_bytes: int, stream: Stream, sample: int = 4096,
              grid: dict | None = None, seed: int = 0, use_cache: bool = True, log=None):
-    """Best :class:`MixParams` for this batch, and a dict describing the choice."""
+    """Best :class:`MixParams` for this batch (upper bounds), and a dict describing the choice."""
     begin = np.asarray(begin, np.int64)
     end = np.asarray(end, np.int64)
     pattern_of = np.asarray(pattern_of, np.int32)
     mix = MixEngine(engines)
     kinds = mix.kinds.tolist()
     lengths = end - begin
-    key = _key("mix", sorted(MIX_GRID.items()), _lib.device_name(), kinds, _length_summary(lengths),
+    key = _key("mix", "candidates as given", sorted(MIX_GRID.items()), _lib.device_name(), kinds, _length_summary(lengths),
                int(np.log2(max(len(begin), 1))))
     if use_cache:
         hit = _load().get(key)
@@ -109,7 +109,8 @@ def tune_mix(engines, begin, end, pattern_of, d_bytes: int, stream: Stream, samp
     names = list(grid)
     results = []
     for values in itertools.product(*(grid[k] for k in names)):
-        params = MixParams(**dict(zip(names, values)))
+        # timed with the lengths it names: the sample is smaller than the batch
+        params = MixParams(**dict(zip(names, values)), at_most=False)
         if params.nfa_chunk % params.ck or params.dfa_split < params.dfa_chunk or params.nfa_split < params.nfa_chunk:
             continue
         try:
@@ -131,6 +132,7 @@ def tune_mix(engines, begin, end, pattern_of, d_bytes: int, stream: Stream, samp
     off = lambda p: sum(getattr(p, f) != getattr(default, f) for f in ("dfa_split", "dfa_chunk", "nfa_split",
                                                                         "nfa_chunk", "ck"))
     ms, best = min((r for r in results if r[0] <= fastest * (1 + NEAR)), key=lambda r: (off(r[1]), r[0]))
+    best.at_most = True   # of a batch of this kind that fills the device; a smaller one is cut shorter
     _store(key, {"params": best.__dict__, "ms": ms, "sample_strings": n, "candidates": len(results)})
     return best, {"source": "tuned", "key": key, "ms": ms, "candidates": len(results), "sample_strings": n}
 

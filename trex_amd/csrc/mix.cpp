@@ -159,6 +159,7 @@ struct trex_mix {
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     int64_t grid = 0;   // persistent workgroups (0: two per compute unit)
+    bool refine = false;   // plans may cut strings shorter than asked for
 };
 
 namespace {
@@ -246,17 +247,15 @@ int upload_plan(trex_mix* m, hipStream_t s) {
 namespace {
 
 // Split and chunk lengths of a batch too small to fill the chip at the given
-// ones: every lane walks its string or chunk alone, so a batch lasts at least
+// ones, where the caller left them open (trex_mix_set_refine): every lane walks its string or chunk alone, so a batch lasts at least
 // as long as one chunk (a 32 KiB NFA chunk: 3 to 7 ms), however little there is
 // of it. Chunks become as short as gives every CU kLanesPerCu lanes of either
 // kind, within the lengths below and the given ones; a batch that fills the
-// chip keeps the given ones, and so do callers that ask for short ones
-// themselves (kTakenAsGiven). True when something became shorter. 16 patterns,
+// chip keeps the given ones. True when DFA chunks became shorter. 16 patterns,
 // 1,024 strings of 32 B to 1 MiB (101 MB): 8.3 ms at 32 / 64 KiB, 345 us at
 // 1 KiB NFA chunks, 278 us at 512 B, 296 us at 256 B.
 constexpr int64_t kLanesPerCu = 512;
 constexpr int64_t kBatchesPerCu = 2;
-constexpr int64_t kTakenAsGiven = 4096;
 constexpr int64_t kLeastNfaChunk = 512, kLeastDfaChunk = 1024;
 
 bool refine(const trex_mix* m, const int64_t* begin, const int64_t* end, const int32_t* pattern_of, int64_t n_strings,
@@ -268,16 +267,11 @@ bool refine(const trex_mix* m, const int64_t* begin, const int64_t* end, const i
     auto up = [](int64_t x, int64_t step) { return (x + step - 1) / step * step; };
     const int64_t dfa = up(std::max(bytes[0] / lanes, kLeastDfaChunk), 16);
     const int64_t nfa = up(std::max(bytes[1] / lanes, kLeastNfaChunk), ck);
-    bool finer = false;
-    auto cut = [&](int64_t& length, int64_t to) {
-        if (length <= kTakenAsGiven || length <= to) return;
-        length = to;
-        finer = true;
-    };
-    cut(dfa_chunk, dfa);
-    cut(dfa_split, std::max(dfa, std::min(dfa_chunk, dfa_split)));
-    cut(nfa_chunk, nfa);
-    cut(nfa_split, std::max(nfa, std::min(nfa_chunk, nfa_split)));
+    const bool finer = dfa < dfa_chunk;
+    dfa_chunk = std::min(dfa_chunk, dfa);
+    dfa_split = std::min(dfa_split, std::max(dfa, dfa_chunk));
+    nfa_chunk = std::min(nfa_chunk, nfa);
+    nfa_split = std::min(nfa_split, std::max(nfa, nfa_chunk));
     return finer;
 }
 
@@ -388,7 +382,7 @@ int trex_mix_plan(trex_mix* m, const int64_t* begin, const int64_t* end, const i
     Plan P;
     P.block = m->form == TREX_MIX_FORM_SLICE ? kMixBlockSlice : kMixBlock;
     const int32_t np = m->n_patterns;
-    const bool finer = m->has_device && refine(m, begin, end, pattern_of, n_strings, ck, dfa_split, dfa_chunk,
+    const bool finer = m->refine && m->has_device && refine(m, begin, end, pattern_of, n_strings, ck, dfa_split, dfa_chunk,
                                                nfa_split, nfa_chunk);
     P.ck = ck;
     P.n_ck = nfa_chunk >= kRecordFrom ? (int32_t)(nfa_chunk / ck) : 0;
@@ -627,6 +621,12 @@ int trex_mix_set_form(trex_mix* m, int form) {
         return fail(TREX_ERR_INVALID, "an NFA pattern has no slice tables");
     m->form = form;
     drop_graph(m);
+    return TREX_OK;
+}
+
+int trex_mix_set_refine(trex_mix* m, int on) {
+    if (!m) return fail(TREX_ERR_INVALID, "null handle");
+    m->refine = on != 0;
     return TREX_OK;
 }
 

@@ -596,12 +596,11 @@ __device__ __forceinline__ void fixup_wave(const MixArgs& A, const MixPattern& P
             return lane > 0u ? up : t;
         };
         uint64_t in = entry(e), out = 0, walked_in = 0, walked_out = 0;   // (an empty set stays empty)
-        bool known;
+        bool known, met = false;
         while (true) {
             known = known_end(P, in, g, e, &A.agg[2 * j + 1], &A.spec_exit[2 * o + 1], out);
             if (!known) {
                 if (have && in != walked_in) {
-                    bool met;
                     walked_in = in;
                     walked_out = nfa_walk_meet<SLICE>(A.bytes, A.ibeg[j], A.iend[j], in, ntab, ncls, P, A.ck,
                                                       A.ckpt + o * A.n_ck, A.n_ck, e, met);
@@ -612,7 +611,7 @@ __device__ __forceinline__ void fixup_wave(const MixArgs& A, const MixPattern& P
             if (__ballot(have && next != in) == 0ull) break;
             in = next;
         }
-        converged += (uint32_t)__popcll(__ballot(have && known));
+        converged += (uint32_t)__popcll(__ballot(have && (known || met)));
         t = lane_of(out, (int)min<int64_t>(c1 - 1 - c, 63));
     }
     if (lane == 0u) fixup_result(A, P, item, t, converged);

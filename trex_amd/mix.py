@@ -30,18 +30,23 @@ BLOCK = 512   # lane items per work batch (one workgroup)
 @dataclass
 class MixParams:
     """Split lengths, chunk lengths and checkpoint spacing of a plan, and the
-    NFA table form ("nibble" / "slice"; None keeps the engine's form). Lengths
-    above 4,096 are upper bounds: a batch too small to fill the device with
-    such chunks is cut shorter."""
+    NFA table form ("nibble" / "slice"; None keeps the engine's form).
+    ``at_most``: the lengths are upper bounds, and a batch too small to fill the
+    device with such chunks is cut shorter; None means so while all lengths are
+    the defaults, and as given where one is named."""
     dfa_split: int = 256 << 10
     dfa_chunk: int = 64 << 10
     nfa_split: int = 32 << 10
     nfa_chunk: int = 32 << 10
     ck: int = 64
     form: str | None = None
+    at_most: bool | None = None
 
     def astuple(self):
         return (int(self.dfa_split), int(self.dfa_chunk), int(self.nfa_split), int(self.nfa_chunk), int(self.ck))
+
+    def upper_bounds(self) -> bool:
+        return self.at_most if self.at_most is not None else self.astuple() == MixParams().astuple()
 
 
 MIX_FORMS = {"nibble": 0, "slice": 1}
@@ -85,6 +90,7 @@ class MixEngine:
             raise ValueError("begin, end and pattern_of must have the same length")
         if params.form is not None:
             self.set_form(params.form)
+        _lib.call("trex_mix_set_refine", self.handle, int(params.upper_bounds()))
         _lib.call("trex_mix_plan", self.handle, self._begin.ctypes.data, self._end.ctypes.data, self._pat.ctypes.data,
                   n, *params.astuple())
         self.n_strings = n
