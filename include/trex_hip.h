@@ -249,6 +249,7 @@ int trex_dfa_multi_match_interleaved(trex_dfa_multi* m, const uint8_t* d_bytes, 
  * ------------------------------------------------------------------------ */
 typedef struct trex_nfa trex_nfa;
 
+#define TREX_NFA_AUTO 0
 #define TREX_NFA_BYTES 1   /* any byte -> class map */
 #define TREX_NFA_WINDOW 2  /* every byte outside one aligned 32-byte window rejects */
 #define TREX_NFA_WINDOW5 3 /* as 2, 5-bit state slices: 13 table reads per byte instead of 16 */
@@ -263,9 +264,9 @@ int trex_nfa_create(const uint64_t* succ, int n_symbols, const int16_t* byte_to_
 int trex_nfa_destroy(trex_nfa* h);
 /* The variant chosen at create time: TREX_NFA_WINDOW6 when every byte outside
  * one aligned 32-byte window rejects, else TREX_NFA_BYTES; set_variant forces
- * another the automaton allows. Without a forced variant, an automaton that
- * reaches at most 256 state sets walks contiguous strings as a DFA over those
- * sets (same results). */
+ * another the automaton allows (TREX_NFA_AUTO restores the default). Without a
+ * forced variant, an automaton that reaches at most 256 state sets walks
+ * contiguous strings as a DFA over those sets (same results). */
 int trex_nfa_info(const trex_nfa* h, int* variant, int* window_base);
 int trex_nfa_set_variant(trex_nfa* h, int variant);
 /* Final state mask and accept bit ((mask & accept) != 0) per string. */
@@ -318,8 +319,8 @@ int trex_pnfa_destroy(trex_pnfa* h);
 int trex_pnfa_info(const trex_pnfa* h, int* mode, int* n_symbols, int* f16_ok, int* waves);
 int trex_pnfa_set_mode(trex_pnfa* h, int mode);
 /* Waves per 64-sequence workgroup: 4 (eight symbols' matrices per wave) or 8
- * (four per wave, two waves per SIMD). Until it is called, batches of at most
- * 32 sequences per compute unit run in workgroups of four waves and fewer
+ * (four per wave, two waves per SIMD). 0 (a new handle): 8, but batches of at
+ * most 32 sequences per compute unit run in workgroups of four waves and fewer
  * sequences, as few as leave each workgroup a compute unit (same results). */
 int trex_pnfa_set_waves(trex_pnfa* h, int waves);
 /* Most workgroups per kernel launch (0, the default: one per group of 64

@@ -1,0 +1,73 @@
+"""A handle's own choice of kernel: restored after a setting, and among the
+candidates of the tuners."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _time(fn, stream, reps=20):
+    from trex_amd.device import Event
+    fn()
+    a, b = Event(), Event()
+    a.record(stream)
+    for _ in range(reps):
+        fn()
+    b.record(stream)
+    stream.synchronize()
+    return a.elapsed_ms(b) / reps
+
+
+def test_nfa_default_is_restored(gpu_lib):
+    """Words over an automaton of few sets: 28 us as a DFA, 300 us and more bit-parallel."""
+    from trex_amd.device import DeviceBuffer, Stream
+    from trex_amd.engine import DeviceBatch, NfaEngine
+    from trex_amd.nfa_matrices import compile_nfa_matrices
+    rng = np.random.default_rng(1)
+    eng = NfaEngine.from_matrices(compile_nfa_matrices("[a-z0-9 ]*(error|warning|fail) [a-z0-9 ]*"))
+    n = 30_000
+    offsets = np.zeros(n + 1, np.int64)
+    np.cumsum(rng.integers(300, 1000, n), out=offsets[1:])
+    data = rng.choice(np.frombuffer(b"abcdefghil ", np.uint8), int(offsets[-1]))
+    stream = Stream()
+    batch = DeviceBatch(data, offsets, "csr")
+    d_mask, d_acc = DeviceBuffer(8 * n), DeviceBuffer(n)
+    run = lambda: eng.match_batch_device(batch, d_mask.ptr, d_acc.ptr, stream)
+    default = eng.info()["variant"]
+    own = _time(run, stream)
+    want = d_mask.download(np.uint64, n, stream)
+    eng.set_variant("bytes")
+    forced = _time(run, stream)
+    assert np.array_equal(d_mask.download(np.uint64, n, stream), want)
+    eng.set_variant("auto")
+    assert eng.info()["variant"] == default
+    again = _time(run, stream)
+    assert np.array_equal(d_mask.download(np.uint64, n, stream), want)
+    assert own < forced / 2 and again < forced / 2
+
+
+def test_pnfa_default_is_restored(gpu_lib):
+    """100 sequences: workgroups of one sequence beat two of 64, whatever the box."""
+    from trex_amd.device import DeviceBuffer, Stream
+    from trex_amd.engine import ProbNfaEngine
+    from trex_amd.workloads import dirichlet_pnfa
+    rng = np.random.default_rng(2)
+    T, start, accept = dirichlet_pnfa(rng)
+    eng = ProbNfaEngine(T, start, accept)
+    n, length = 100, 500
+    stream = Stream()
+    d = DeviceBuffer.from_array(rng.integers(0, T.shape[0], n * length, dtype=np.uint8), stream)
+    d_ll, d_lm = DeviceBuffer(8 * n), DeviceBuffer(8 * n)
+    run = lambda: eng.loglik_device(d.ptr, n, length, d_ll.ptr, d_lm.ptr, stream)
+    own = _time(run, stream, 5)
+    want = d_ll.download(np.float64, n, stream)
+    eng.set_waves(8)
+    forced = _time(run, stream, 5)
+    eng.set_waves(0)
+    assert eng.info()["waves"] == 8
+    again = _time(run, stream, 5)
+    assert np.array_equal(d_ll.download(np.float64, n, stream), want)
+    assert own < 0.8 * forced and again < 0.8 * forced

@@ -255,7 +255,8 @@ int trex_nfa_create(const uint64_t* succ, int n_symbols, const int16_t* byte_to_
         }
     }
     if (rc) { trex_nfa_destroy(h); return rc; }
-    h->variant = h->d_tab6 ? TREX_NFA_WINDOW6 : h->window_base >= 0 ? TREX_NFA_WINDOW : TREX_NFA_BYTES;
+    h->auto_variant = h->d_tab6 ? TREX_NFA_WINDOW6 : h->window_base >= 0 ? TREX_NFA_WINDOW : TREX_NFA_BYTES;
+    h->variant = h->auto_variant;
     *out = h;
     return TREX_OK;
 }
@@ -289,6 +290,11 @@ int trex_nfa_info(const trex_nfa* h, int* variant, int* window_base) {
 
 int trex_nfa_set_variant(trex_nfa* h, int variant) {
     if (!h) return fail(TREX_ERR_INVALID, "null handle");
+    if (variant == TREX_NFA_AUTO) {
+        h->variant = h->auto_variant;
+        h->forced = false;
+        return TREX_OK;
+    }
     if (variant == TREX_NFA_BYTES || (variant == TREX_NFA_WINDOW && h->window_base >= 0) ||
         (variant == TREX_NFA_WINDOW5 && h->d_tab5) || (variant == TREX_NFA_WINDOW6 && h->d_tab6)) {
         h->variant = variant;

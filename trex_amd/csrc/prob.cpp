@@ -304,9 +304,10 @@ int trex_pnfa_set_mode(trex_pnfa* h, int mode) {
 
 int trex_pnfa_set_waves(trex_pnfa* h, int waves) {
     if (!h) return fail(TREX_ERR_INVALID, "null handle");
-    if (waves != 4 && waves != 8) return fail(TREX_ERR_INVALID, "waves must be 4 or 8, got %d", waves);
-    h->waves = waves;
-    h->waves_set = true;
+    if (waves != 0 && waves != 4 && waves != 8)
+        return fail(TREX_ERR_INVALID, "waves must be 4, 8 or 0 (the handle's choice), got %d", waves);
+    h->waves = waves ? waves : 8;
+    h->waves_set = waves != 0;
     return TREX_OK;
 }
 

@@ -128,7 +128,7 @@ struct trex_nfa {
     uint64_t guess = ~0ull, second = 0;
     trex::Sticky sticky[trex::kSticky] = {};
     int window_base = -1;
-    int variant = TREX_NFA_BYTES;
+    int variant = TREX_NFA_BYTES, auto_variant = TREX_NFA_BYTES;
     int n_classes = 0, n_classes_win = 0;
     uint64_t* d_tab = nullptr;      // [n_symbols + 2][16][16]: symbols, reject, skip (bank-swizzled)
     uint8_t* d_cls = nullptr;       // [256] byte -> class

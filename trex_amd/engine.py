@@ -352,7 +352,7 @@ class DeviceBatch:
             b.free()
 
 
-NFA_VARIANTS = {"bytes": 1, "window": 2, "window5": 3, "window6": 4}
+NFA_VARIANTS = {"auto": 0, "bytes": 1, "window": 2, "window5": 3, "window6": 4}
 NFA_VARIANT_NAMES = {v: k for k, v in NFA_VARIANTS.items()}
 
 
@@ -545,6 +545,8 @@ class ProbNfaEngine:
         return {"mode": PNFA_MODE_NAMES[m.value], "n_symbols": n.value, "f16_ok": bool(ok.value), "waves": w.value}
 
     def set_waves(self, waves: int) -> None:
+        """Waves per workgroup of 64 sequences: 4 or 8; 0 (default) leaves the
+        launch shape to the batch."""
         _lib.call("trex_pnfa_set_waves", self.handle, int(waves))
 
     def set_grid(self, workgroups: int) -> None:
