@@ -71,3 +71,32 @@ def test_pnfa_default_is_restored(gpu_lib):
     again = _time(run, stream, 5)
     assert np.array_equal(d_ll.download(np.float64, n, stream), want)
     assert own < 0.8 * forced and again < 0.8 * forced
+
+
+def test_tuners_know_the_engines_own_choice(gpu_lib, tmp_path, monkeypatch):
+    """Lines of unequal lengths (half the time of any variant) and 100 sequences."""
+    from trex_amd.autotune import tune_dfa, tune_pnfa
+    from trex_amd.device import DeviceBuffer, Stream
+    from trex_amd.engine import DeviceBatch, DfaEngine, ProbNfaEngine
+    from trex_amd.regex_to_dfa import compile_regex
+    from trex_amd.tables import dfa_byte_table
+    from trex_amd.workloads import dirichlet_pnfa
+    monkeypatch.setenv("TREX_AMD_TUNE_CACHE", str(tmp_path / "tune.json"))
+    rng = np.random.default_rng(3)
+    stream = Stream()
+    n = 100_000
+    offsets = np.zeros(n + 1, np.int64)
+    np.cumsum(rng.integers(20, 400, n), out=offsets[1:])
+    batch = DeviceBatch(rng.integers(32, 127, int(offsets[-1]), dtype=np.uint8), offsets, "csr")
+    d_out = [DeviceBuffer(n) for _ in range(2)]
+    table = dfa_byte_table(compile_regex(".*(error|warn).*"))
+    for source in ("tuned", "cache"):
+        eng = DfaEngine(table)
+        choice = tune_dfa(eng, batch, d_out[0].ptr, d_out[1].ptr, stream)
+        assert (choice["source"], choice["variant"], choice["prefetch"]) == (source, "auto", 8)
+    T, start, accept = dirichlet_pnfa(rng)
+    n, length = 100, 500
+    d = DeviceBuffer.from_array(rng.integers(0, T.shape[0], n * length, dtype=np.uint8), stream)
+    d_ll = [DeviceBuffer(8 * n) for _ in range(2)]
+    choice = tune_pnfa(ProbNfaEngine(T, start, accept), d.ptr, n, length, d_ll[0].ptr, d_ll[1].ptr, stream)
+    assert choice["waves"] == 0

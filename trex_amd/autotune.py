@@ -8,6 +8,8 @@ caches the choice.
 * :func:`tune_dfa` -- kernel variant and loads in flight of a DFA-16 engine;
 * :func:`tune_pnfa` -- waves per workgroup of a probabilistic NFA engine.
 
+The engine's own choice is a candidate of the last two.
+
 Choices are cached in a JSON file (``$TREX_AMD_TUNE_CACHE``, default
 ``~/.cache/trex_amd/tune.json``) under a key made of the device, the kind of
 work and a coarse summary of the workload (pattern kinds, log2 length
@@ -140,7 +142,7 @@ def tune_mix(engines, begin, end, pattern_of, d_bytes: int, stream: Stream, samp
 def tune_dfa(engine, batch, d_final: int, d_accept: int, stream: Stream, use_cache: bool = True) -> dict:
     """Kernel variant and prefetch depth of one DFA engine on a device batch."""
     mean_len = batch.payload_bytes // max(1, batch.n_strings)
-    key = _key("dfa", _lib.device_name(), engine.table.n_states, engine.info()["window_base"] >= 0,
+    key = _key("dfa", "auto too", _lib.device_name(), engine.table.n_states, engine.info()["window_base"] >= 0,
                int(np.log2(max(batch.n_strings, 1))), int(np.log2(max(mean_len, 1))))
     if use_cache:
         hit = _load().get(key)
@@ -149,8 +151,8 @@ def tune_dfa(engine, batch, d_final: int, d_accept: int, stream: Stream, use_cac
             engine.set_prefetch(hit["prefetch"])
             return {"source": "cache", **hit}
     options = []
-    for variant in ("k2_window_f", "k2_window", "k1_16", "k1_generic"):
-        for pf in (8, 16):
+    for variant in ("auto", "k2_window_f", "k2_window", "k1_16", "k1_generic"):
+        for pf in (8,) if variant == "auto" else (8, 16):
             try:
                 engine.set_variant(variant)
                 engine.set_prefetch(pf)
@@ -168,9 +170,9 @@ def tune_dfa(engine, batch, d_final: int, d_accept: int, stream: Stream, use_cac
 
 def tune_pnfa(engine, d_symbols: int, n_seq: int, length: int, d_ll: int, d_lm: int, stream: Stream,
               use_cache: bool = True) -> dict:
-    """Waves per workgroup of a probabilistic NFA engine (its mode is kept)."""
+    """Waves per workgroup of a probabilistic NFA engine, 0: by the batch (its mode is kept)."""
     mode = engine.info()["mode"]
-    key = _key("pnfa", _lib.device_name(), mode, engine.n_symbols, int(np.log2(max(n_seq, 1))),
+    key = _key("pnfa", "auto too", _lib.device_name(), mode, engine.n_symbols, int(np.log2(max(n_seq, 1))),
                int(np.log2(max(length, 1))))
     if use_cache:
         hit = _load().get(key)
@@ -178,7 +180,7 @@ def tune_pnfa(engine, d_symbols: int, n_seq: int, length: int, d_ll: int, d_lm: 
             engine.set_waves(hit["waves"])
             return {"source": "cache", **hit}
     options = []
-    for waves in (4, 8):
+    for waves in (0, 4, 8):
         engine.set_waves(waves)
         options.append((_time(lambda: engine.loglik_device(d_symbols, n_seq, length, d_ll, d_lm, stream), stream, 2),
                         waves))
