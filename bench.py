@@ -369,7 +369,9 @@ def dfa_leg(args, data, offsets, batch, stream, result: dict, copy_gbs) -> int:
                 eng.set_rotation(-1)
             c_ms = float(np.mean([a.elapsed_ms(b) for a, b in c_evs[N_PATTERNS:]]))
             c_ach = alg_bytes / (c_ms * 1e-3) / 1e9
-            kname = "dfa16_k2f_rot_pf8" if all(rotated) else kernel_name(variants[0], args.prefetch, "csr")
+            kname = kernel_name(variants[0], args.prefetch, "csr")
+            if mode == -1 and args.variant == "auto" and args.prefetch == 8:   # walked by byte classes
+                kname = "dfa16_cls_*_left + dfa16_k2f_rot_pf8" if all(rotated) else "dfa16_cls_*"
             csr_res[key] = {"kernel": kname, "patterns_rotated": int(sum(rotated)),
                             "kernel_avg_ms": round(c_ms, 5), "achieved_gbs": round(c_ach, 1),
                             "frac": round(c_ach / HBM_PEAK_GBS, 4), "same_results_as_interleaved": csr_same}
@@ -430,9 +432,12 @@ def dfa_leg(args, data, offsets, batch, stream, result: dict, copy_gbs) -> int:
         b.free()
 
     kernel = kernel_name(variants[0], args.prefetch, args.layout)
-    if (args.layout != "interleaved" and kernel == "dfa16_k2f_pf8"
-            and all(eng.rotation()[0] for eng in engines)):
-        kernel = "dfa16_k2f_rot_pf8"
+    if args.layout != "interleaved" and kernel == "dfa16_k2f_pf8":
+        rotated = all(eng.rotation()[0] for eng in engines)
+        if args.variant == "auto":
+            kernel = "dfa16_cls_*_left + dfa16_k2f_rot_pf8" if rotated else "dfa16_cls_*"
+        elif rotated:
+            kernel = "dfa16_k2f_rot_pf8"
     result.update({
         "metric": "Gchars/s (DFA-16, NFA-64) + %HBM roofline; p50/p99 latency served vs plain",
         "value": round(gchars, 2),

@@ -139,7 +139,9 @@ int trex_dfa_destroy(trex_dfa* h);
 #define TREX_DFA_K2_WINDOW_FR 6 /* as 5, four interleaved copies of the table in LDS (fewer bank conflicts) */
 
 /* Reports the kernel variant chosen at create time, the window base byte
- * (-1 if none) and the dead state (-1 if none). */
+ * (-1 if none) and the dead state (-1 if none). The variant is what interleaved
+ * strings run; contiguous ones are walked by byte classes unless a variant, a
+ * rotation mode or a prefetch of 16 is set. */
 int trex_dfa_info(const trex_dfa* h, int* variant, int* window_base, int* dead_state);
 /* Forces a variant (TREX_DFA_AUTO restores the default); fails if the table
  * does not allow it. */
@@ -157,12 +159,15 @@ int trex_dfa_set_prefetch(trex_dfa* h, int vectors);
  * modulo 4 KiB at once, which crowds a few HBM channels. Same results.
  * mode -1 (default): on for batches of 131,072 strings and more whose table
  * synchronises (some word over its window bytes sends every state that can
- * occur to one state), for the workgroups whose strings are alike; 0 off; 1 on
- * for every launch of that kernel. With a mode of 0 or 1 contiguous strings
- * are walked in the handle's variant, otherwise by byte classes.
+ * occur to one state) and has no state but the dead one that every live byte
+ * keeps, for the workgroups whose strings are alike; 0 off; 1 on for every
+ * launch of that kernel. With a mode of 0 or 1 contiguous strings are walked in
+ * the handle's variant, otherwise by byte classes (a forced variant at mode -1
+ * is rotated for every table that synchronises).
  * No counterpart in the reference (its kernels read strings as packed,
  * cuda/monoid_batch.cu:58-95). trex_dfa_rotation reports whether launches
- * use it and whether the table synchronises. */
+ * (of enough alike strings, for the default) use it and whether the table
+ * synchronises. */
 int trex_dfa_set_rotation(trex_dfa* h, int mode);
 int trex_dfa_rotation(const trex_dfa* h, int* active, int* synchronizes);
 

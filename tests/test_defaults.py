@@ -100,3 +100,20 @@ def test_tuners_know_the_engines_own_choice(gpu_lib, tmp_path, monkeypatch):
     d_ll = [DeviceBuffer(8 * n) for _ in range(2)]
     choice = tune_pnfa(ProbNfaEngine(T, start, accept), d.ptr, n, length, d_ll[0].ptr, d_ll[1].ptr, stream)
     assert choice["waves"] == 0
+
+
+def test_rotation_is_reported_as_launched(gpu_lib):
+    """A search table synchronises, but its functions stay apart until the text is
+    found, so its launches are not rotated unless a variant or a mode asks for it."""
+    from trex_amd.engine import DfaEngine
+    from trex_amd.regex_to_dfa import compile_regex
+    from trex_amd.tables import dfa_byte_table
+    search = DfaEngine(dfa_byte_table(compile_regex("[A-Z]*(ERROR|WARN|FAIL)[A-Z]*")))
+    recent = DfaEngine(dfa_byte_table(compile_regex("(A|B|C|D)*(A|B)(C|D)")))
+    assert search.rotation() == (False, True) and recent.rotation() == (True, True)
+    search.set_variant("k2_window_f")
+    assert search.rotation() == (True, True)
+    search.set_variant("auto")
+    assert search.rotation() == (False, True)
+    search.set_rotation(1)
+    assert search.rotation() == (True, True)

@@ -228,6 +228,17 @@ int trex_dfa_set_variant(trex_dfa* h, int variant) {
     return TREX_OK;
 }
 
+namespace {
+
+// Whether contiguous strings are walked by byte classes (no variant, read order
+// or prefetch was asked for), and whether the variant's walk of them is rotated.
+bool walks_by_classes(const trex_dfa* h) {
+    return h->cls.d_tab && !h->forced && h->rotation == -1 && h->prefetch == 8;
+}
+bool rotates_variant(const trex_dfa* h) { return h->rotation == 1 || (h->rotation == -1 && h->synchronizes); }
+
+}  // namespace
+
 int trex_dfa_set_rotation(trex_dfa* h, int mode) {
     if (!h) return fail(TREX_ERR_INVALID, "null handle");
     if (mode < -1 || mode > 1) return fail(TREX_ERR_INVALID, "rotation mode %d: -1 (auto), 0 or 1", mode);
@@ -238,7 +249,7 @@ int trex_dfa_set_rotation(trex_dfa* h, int mode) {
 int trex_dfa_rotation(const trex_dfa* h, int* active, int* synchronizes) {
     if (!h) return fail(TREX_ERR_INVALID, "null handle");
     const bool usable = h->window_base >= 0 && h->n_states <= 16;
-    if (active) *active = usable && (h->rotation == 1 || (h->rotation == -1 && h->synchronizes)) ? 1 : 0;
+    if (active) *active = usable && (walks_by_classes(h) ? h->rotate : rotates_variant(h)) ? 1 : 0;
     if (synchronizes) *synchronizes = h->synchronizes ? 1 : 0;
     return TREX_OK;
 }
@@ -278,7 +289,7 @@ int dfa_dispatch(trex_dfa* h, const uint8_t* d_bytes, const int64_t* d_begin, co
     uint32_t start = (uint32_t)h->start;
     const char* il_tag = il ? "_il" : "";
     char name[48];
-    if (!il && h->cls.d_tab && !h->forced && h->rotation == -1 && h->prefetch == 8) {
+    if (!il && walks_by_classes(h)) {
         const bool rot = h->rotate && n_strings >= kRotateFrom;
         TREX_TRY(launch_class_form(h->cls, d_bytes, d_begin, d_end, n_strings, rot, d_final_state, nullptr, d_accept, s));
         return rot ? launch_rotated(h, d_bytes, d_begin, d_end, n_strings, 1u, d_final_state, d_accept, s) : TREX_OK;
@@ -289,9 +300,7 @@ int dfa_dispatch(trex_dfa* h, const uint8_t* d_bytes, const int64_t* d_begin, co
         uint32_t dead = (uint32_t)h->dead;
         uint8_t* table = h->variant == TREX_DFA_K2_WINDOW ? h->d_t2 : h->d_f2;
         const char* form = h->variant == TREX_DFA_K2_WINDOW ? "k2w" : h->variant == TREX_DFA_K2_WINDOW_F ? "k2f" : "k2fr";
-        int rot = 0;
-        trex_dfa_rotation(h, &rot, nullptr);
-        if (!il && rot && h->variant == TREX_DFA_K2_WINDOW_F && h->prefetch == 8) {
+        if (!il && rotates_variant(h) && h->variant == TREX_DFA_K2_WINDOW_F && h->prefetch == 8) {
             // contiguous strings, read order rotated per wave (spreads HBM channels)
             return launch_rotated(h, d_bytes, d_begin, d_end, n_strings, 0u, d_final_state, d_accept, s);
         }

@@ -99,13 +99,15 @@ class DfaEngine:
         _lib.call("trex_dfa_set_prefetch", self.handle, int(vectors))
 
     def set_rotation(self, mode: int) -> None:
-        """Read order of contiguous strings: -1 (default) rotated per wave when
-        the table synchronises, 0 never, 1 always (``trex_dfa_set_rotation``)."""
+        """Read order of contiguous strings: -1 (default) rotated per wave for
+        alike strings in batches of 131,072 and more when the table synchronises
+        and no state but the dead one is kept by every byte, 0 never, 1 always
+        (``trex_dfa_set_rotation``)."""
         _lib.call("trex_dfa_set_rotation", self.handle, int(mode))
 
     def rotation(self) -> tuple[bool, bool]:
-        """(launches over contiguous strings use the rotated read order,
-        the table synchronises)."""
+        """(launches over enough alike contiguous strings use the rotated read
+        order, the table synchronises)."""
         a, sy = ctypes.c_int(), ctypes.c_int()
         _lib.call("trex_dfa_rotation", self.handle, ctypes.byref(a), ctypes.byref(sy))
         return bool(a.value), bool(sy.value)
