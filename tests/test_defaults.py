@@ -117,3 +117,32 @@ def test_rotation_is_reported_as_launched(gpu_lib):
     assert search.rotation() == (False, True)
     search.set_rotation(1)
     assert search.rotation() == (True, True)
+
+
+def test_multi_pattern_group_outlives_the_form(gpu_lib):
+    """A group of one is eight launches, also after the form went back to the
+    default; without a group the default form takes all patterns in one."""
+    from trex_amd.device import DeviceBuffer, Stream
+    from trex_amd import _lib
+    from trex_amd.engine import DeviceBatch, DfaEngine, DfaMultiEngine
+    from trex_amd.regex_to_dfa import compile_regex
+    from trex_amd.tables import dfa_byte_table
+    rng = np.random.default_rng(4)
+    words = ["ERROR", "TIMEOUT", "LOGIN", "LOGOUT", "REFUSED", "DENIED", "CLOSED", "BROKEN"]
+    engines = [DfaEngine(dfa_byte_table(compile_regex(f"[A-Z]*{w}[A-Z]*"))) for w in words]
+    multi = DfaMultiEngine(engines)
+    n = 50_000
+    offsets = np.zeros(n + 1, np.int64)
+    np.cumsum(rng.integers(300, 600, n), out=offsets[1:])
+    data = rng.integers(0x41, 0x5B, int(offsets[-1]), dtype=np.uint8)
+    stream = Stream()
+    batch = DeviceBatch(data, offsets, "csr")
+    d_out = [DeviceBuffer(len(words) * n) for _ in range(2)]
+    run = lambda: multi.match_batch_device(batch, d_out[0].ptr, d_out[1].ptr, stream)
+    together = _time(run, stream)
+    want = d_out[0].download(np.uint8, len(words) * n, stream)
+    multi.set_group(1)
+    apart = _time(run, stream)
+    _lib.call("trex_dfa_multi_set_form", multi.handle, 0)
+    assert _time(run, stream) > 0.6 * apart > 0.9 * together
+    assert np.array_equal(d_out[0].download(np.uint8, len(words) * n, stream), want)

@@ -82,7 +82,8 @@ struct trex_dfa_multi {
     int fp_group = -1;            // the group d_fp was built for
     std::vector<uint64_t> h_f1;   // [n][32] single-symbol functions (host copy)
     std::vector<int> n_states;
-    bool picked = true;           // the form and the group are the handle's own choice
+    bool form_set = false, group_set = false;   // chosen by the caller
+    bool picked() const { return !form_set && !group_set; }
     uint8_t* d_fc = nullptr;      // compact tables of the current grouping
     std::vector<CompactLaunch> fc;
     int fc_group = -1;            // the group d_fc was built for
@@ -235,7 +236,7 @@ int auto_form(const trex_dfa_multi* m) {
 // strings (2 patterns of 9 states, 50,000 x 200..3000 bytes: 59 us paired, 44
 // us so; 262,144 x 4 KiB: 281 us and 257 us).
 int compact_group(const trex_dfa_multi* m) {
-    return m->form == TREX_DFA_MULTI_K2F_COMPACT ? m->group : m->picked ? kMultiMax : 0;
+    return m->form == TREX_DFA_MULTI_K2F_COMPACT ? m->group : m->picked() ? kMultiMax : 0;
 }
 
 // (Re)builds the tables the handle's form needs for its grouping.
@@ -325,20 +326,20 @@ int trex_dfa_multi_create(trex_dfa* const* patterns, int n_patterns, trex_dfa_mu
 
 int trex_dfa_multi_set_form(trex_dfa_multi* m, int form) {
     if (!m) return fail(TREX_ERR_INVALID, "null handle");
-    const bool picked = form == TREX_DFA_AUTO;
-    if (picked) form = auto_form(m);
+    const bool set = form != TREX_DFA_AUTO;
+    if (!set) form = auto_form(m);
     if (form != TREX_DFA_K2_WINDOW_F && form != TREX_DFA_K2_WINDOW && form != TREX_DFA_MULTI_K2F_PAIRED &&
         form != TREX_DFA_MULTI_K2F_COMPACT)
         return fail(TREX_ERR_INVALID, "form %d: use TREX_DFA_K2_WINDOW_F, TREX_DFA_K2_WINDOW, "
                     "TREX_DFA_MULTI_K2F_PAIRED or TREX_DFA_MULTI_K2F_COMPACT", form);
     const int prev = m->form;
-    const bool prev_picked = m->picked;
+    const bool prev_set = m->form_set;
     m->form = form;
-    m->picked = picked;
+    m->form_set = set;
     const int rc = ensure_tables(m);
     if (rc) {
         m->form = prev;
-        m->picked = prev_picked;
+        m->form_set = prev_set;
     }
     return rc;
 }
@@ -347,7 +348,7 @@ int trex_dfa_multi_set_group(trex_dfa_multi* m, int group) {
     if (!m) return fail(TREX_ERR_INVALID, "null handle");
     if (group < 1 || group > kMultiMax) return fail(TREX_ERR_INVALID, "group=%d outside 1..%d", group, kMultiMax);
     m->group = group;
-    m->picked = false;
+    m->group_set = true;
     return ensure_tables(m);
 }
 
@@ -369,7 +370,7 @@ int multi_dispatch(trex_dfa_multi* m, const uint8_t* d_bytes, const int64_t* d_b
     if (n_strings < 0) return fail(TREX_ERR_INVALID, "n_strings < 0");
     if (n_strings == 0) return TREX_OK;
     if (!d_bytes || !d_begin || !d_end || !d_final_state || !d_accept) return fail(TREX_ERR_INVALID, "null buffer");
-    const bool compact = m->form == TREX_DFA_MULTI_K2F_COMPACT || (m->picked && !il);
+    const bool compact = m->form == TREX_DFA_MULTI_K2F_COMPACT || (m->picked() && !il);
     const unsigned block = compact && !il && n_strings < kCompactBlockFrom ? 64u : (unsigned)kBlock;
     const int64_t grid64 = (n_strings + block - 1) / block;
     if (grid64 > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");
