@@ -605,7 +605,7 @@ chunk_table_count(const int64_t* __restrict__ begin, const int64_t* __restrict__
         }
         // inclusive scan within the wave, then across the 16 waves
         int64_t x = cnt;
-#pragma unroll 1   // (unrolled, the kernels go over 128 VGPRs)
+#pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const int64_t y = __shfl_up(x, d, 64);
             if ((int)lane >= d) x += y;
