@@ -196,6 +196,9 @@ int trex_dfa_match_interleaved(trex_dfa* h, const uint8_t* d_bytes, const int64_
  * the copy+kernel+copy time, like the reference's dispatch outputs. */
 int trex_dfa_match_host(trex_dfa* h, const uint8_t* bytes, const int64_t* offsets, int64_t n_strings,
                         uint8_t* final_state, uint8_t* accept, float* kernel_ms, float* total_ms);
+/* Pinned host memory that the host dispatches of all handles stage through: 640
+ * KiB for each that ran at once, at most 16, freed with the last handle. */
+int trex_dfa_staging_bytes(int64_t* bytes);
 
 /* ------------------------------------------------------------------------
  * Several DFA-16 patterns in one pass over the bytes. The reference packs

@@ -58,6 +58,7 @@ _SIGNATURES = {
     "trex_dfa_create": (c_int, [u8p, u8p, c_int, c_int, vpp]),
     "trex_dfa_destroy": (c_int, [c_void_p]),
     "trex_dfa_info": (c_int, [c_void_p, intp, intp, intp]),
+    "trex_dfa_staging_bytes": (c_int, [POINTER(c_int64)]),
     "trex_dfa_set_variant": (c_int, [c_void_p, c_int]),
     "trex_dfa_set_prefetch": (c_int, [c_void_p, c_int]),
     "trex_dfa_set_rotation": (c_int, [c_void_p, c_int]),

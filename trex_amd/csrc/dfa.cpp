@@ -26,6 +26,78 @@ namespace {
 // would cost more than it saves.
 constexpr size_t kPinnedIn = 512 << 10, kPinnedOut = 128 << 10;
 
+// The staging blocks of the process: lent to a dispatch for its duration, so as
+// many exist as dispatches ran at once, at most kMost (a dispatch that finds
+// none copies from the caller's memory). They are freed with the last handle.
+// Allocating one takes longer than it saves once (a handle's first match of 48
+// strings: 230 us without, 330 us when each handle made its own), so a handle's
+// first dispatch only takes one that is there.
+class Staging {
+public:
+    uint8_t* take(bool make) {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (!idle_.empty()) {
+                uint8_t* p = idle_.back();
+                idle_.pop_back();
+                return p;
+            }
+            if (!make || made_ == kMost) return nullptr;
+            ++made_;
+        }
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kPinnedIn + kPinnedOut, hipHostMallocPortable) == hipSuccess) return (uint8_t*)p;
+        (void)hipGetLastError();   // without pinned memory to be had, everything is copied as it is
+        std::lock_guard<std::mutex> lock(mu_);
+        --made_;
+        return nullptr;
+    }
+    void give(uint8_t* p) {
+        std::lock_guard<std::mutex> lock(mu_);
+        idle_.push_back(p);
+    }
+    void handle_made() {
+        std::lock_guard<std::mutex> lock(mu_);
+        ++handles_;
+    }
+    void handle_gone() {
+        std::vector<uint8_t*> unused;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (--handles_ > 0) return;
+            unused.swap(idle_);
+            made_ -= (int)unused.size();
+        }
+        for (uint8_t* p : unused) hipHostFree(p);
+    }
+    int64_t bytes() {
+        std::lock_guard<std::mutex> lock(mu_);
+        return (int64_t)made_ * (int64_t)(kPinnedIn + kPinnedOut);
+    }
+
+private:
+    static constexpr int kMost = 16;
+    std::mutex mu_;
+    std::vector<uint8_t*> idle_;
+    int made_ = 0, handles_ = 0;
+};
+
+Staging& staging() {
+    static Staging* s = new Staging();   // outlives every handle
+    return *s;
+}
+
+// A block for one dispatch; given back once nothing on the stream uses it.
+struct Lease {
+    uint8_t* block;
+    hipStream_t stream = nullptr;   // set while the device may use the block
+    ~Lease() {
+        if (!block) return;
+        if (stream) (void)hipStreamSynchronize(stream);
+        staging().give(block);
+    }
+};
+
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Finds the absorbing non-accepting state, or -1.
@@ -151,6 +223,7 @@ int trex_dfa_create(const uint8_t* delta, const uint8_t* accept, int n_states, i
     TREX_TRY(ensure_module());
 
     trex_dfa* h = new trex_dfa();
+    staging().handle_made();
     h->n_states = n_states;
     h->start = start;
     h->stride = std::max(16, (n_states + 15) / 16 * 16);
@@ -201,12 +274,12 @@ int trex_dfa_destroy(trex_dfa* h) {
     hipFree(h->d_f2);
     h->cls.release();
     h->in_bytes.release();
-    if (h->pinned) hipHostFree(h->pinned);
     h->out_state.release();
     h->out_accept.release();
     for (auto& e : h->ev) if (e) hipEventDestroy(e);
     if (h->stream) hipStreamDestroy(h->stream);
     delete h;
+    staging().handle_gone();
     return TREX_OK;
 }
 
@@ -351,32 +424,32 @@ int trex_dfa_match_host(trex_dfa* h, const uint8_t* bytes, const int64_t* offset
     std::lock_guard<std::mutex> lock(h->mu);
     const size_t n = (size_t)n_strings, row = align_up(n, 16);
     const size_t bytes_at = align_up(sizeof(int64_t) * (n + 1), 256);   // device batch: offsets, then bytes
-    // (without pinned memory to be had, everything is copied as it is)
-    if (!h->pinned && hipHostMalloc((void**)&h->pinned, kPinnedIn + kPinnedOut, hipHostMallocDefault) != hipSuccess) {
-        h->pinned = nullptr;
-        (void)hipGetLastError();
-    }
-    const bool offsets_staged = h->pinned && bytes_at <= kPinnedIn;
-    const bool bytes_staged = h->pinned && bytes_at + (size_t)total <= kPinnedIn;
-    const bool results_staged = h->pinned && 2 * row <= kPinnedOut;
+    const bool fits = bytes_at <= kPinnedIn || 2 * row <= kPinnedOut;
+    Lease lease{fits ? staging().take(h->dispatched) : nullptr};
+    uint8_t* const pinned = lease.block;
+    h->dispatched = true;
+    const bool offsets_staged = pinned && bytes_at <= kPinnedIn;
+    const bool bytes_staged = pinned && bytes_at + (size_t)total <= kPinnedIn;
+    const bool results_staged = pinned && 2 * row <= kPinnedOut;
     TREX_TRY(h->in_bytes.reserve(bytes_at + (size_t)total + 16));
     TREX_TRY(h->out_state.reserve(results_staged ? 0 : n));
     TREX_TRY(h->out_accept.reserve(results_staged ? 0 : n));
     TREX_TRY(ensure_host_dispatch(h->stream, h->ev));
     // Offsets are rebased so the device batch starts at byte 0.
     std::vector<int64_t> unstaged(offsets_staged ? 0 : n + 1);
-    int64_t* rebased = offsets_staged ? reinterpret_cast<int64_t*>(h->pinned) : unstaged.data();
+    int64_t* rebased = offsets_staged ? reinterpret_cast<int64_t*>(pinned) : unstaged.data();
     for (size_t i = 0; i <= n; ++i) rebased[i] = offsets[i] - base;
-    if (bytes_staged && total > 0) memcpy(h->pinned + bytes_at, bytes + base, (size_t)total);
+    if (bytes_staged && total > 0) memcpy(pinned + bytes_at, bytes + base, (size_t)total);
 
     hipStream_t s = h->stream;
+    lease.stream = s;
     uint8_t* d_offsets = h->in_bytes.as<uint8_t>();
     uint8_t* d_bytes = d_offsets + bytes_at;
-    uint8_t* d_state = results_staged ? h->pinned + kPinnedIn : h->out_state.as<uint8_t>();
-    uint8_t* d_accept = results_staged ? h->pinned + kPinnedIn + row : h->out_accept.as<uint8_t>();
+    uint8_t* d_state = results_staged ? pinned + kPinnedIn : h->out_state.as<uint8_t>();
+    uint8_t* d_accept = results_staged ? pinned + kPinnedIn + row : h->out_accept.as<uint8_t>();
     TREX_HIP(hipEventRecord(h->ev[0], s), "hipEventRecord");
     if (offsets_staged)
-        TREX_TRY(trex_copy(d_offsets, h->pinned, align_up(bytes_at + (bytes_staged ? (size_t)total : 0), 16), s));
+        TREX_TRY(trex_copy(d_offsets, pinned, align_up(bytes_at + (bytes_staged ? (size_t)total : 0), 16), s));
     else
         TREX_HIP(hipMemcpyAsync(d_offsets, rebased, unstaged.size() * sizeof(int64_t), hipMemcpyHostToDevice, s), "H2D offsets");
     if (!bytes_staged && total > 0) TREX_HIP(hipMemcpyAsync(d_bytes, bytes + base, (size_t)total, hipMemcpyHostToDevice, s), "H2D bytes");
@@ -391,6 +464,7 @@ int trex_dfa_match_host(trex_dfa* h, const uint8_t* bytes, const int64_t* offset
         TREX_HIP(hipEventRecord(last, s), "hipEventRecord");
     }
     TREX_HIP(hipEventSynchronize(last), "hipEventSynchronize");
+    lease.stream = nullptr;
     if (results_staged) {
         memcpy(final_state, d_state, n);
         memcpy(accept, d_accept, n);
@@ -400,6 +474,12 @@ int trex_dfa_match_host(trex_dfa* h, const uint8_t* bytes, const int64_t* offset
     hipEventElapsedTime(&t, h->ev[0], last);
     if (kernel_ms) *kernel_ms = k;
     if (total_ms) *total_ms = t;
+    return TREX_OK;
+}
+
+int trex_dfa_staging_bytes(int64_t* bytes) {
+    if (!bytes) return fail(TREX_ERR_INVALID, "null argument");
+    *bytes = staging().bytes();
     return TREX_OK;
 }
 

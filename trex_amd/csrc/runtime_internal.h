@@ -113,7 +113,7 @@ struct trex_dfa {
     uint32_t rot_init[4] = {0, 0, 0, 0};  // starting function of the rotated kernel's composition
     // staging for trex_dfa_match_host
     trex::DevBuf in_bytes, out_state, out_accept;
-    uint8_t* pinned = nullptr;  // host memory the device reads and writes, made by the first host dispatch
+    bool dispatched = false;    // a host dispatch was made (dfa.cpp: Staging)
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     std::mutex mu;            // serialises host dispatches on this handle
