@@ -85,3 +85,33 @@ def test_alike_strings_take_the_rotated_order(gpu_lib):
     begin[600] += 3   # one string keeps its workgroup from being alike
     data[4096 * 5 + 77] = 0x20
     _check(table, data, begin, end)
+
+
+def _ranges_ms(eng, data, begin, end):
+    from trex_amd.device import Event, Stream
+    n = len(begin)
+    stream = Stream()
+    d, b, e = (DeviceBuffer.from_array(x, stream) for x in (data, begin, end))
+    outs = [DeviceBuffer(n) for _ in range(2)]
+    marks = Event(), Event()
+    for reps, mark in ((3, marks[0]), (20, marks[1])):
+        for _ in range(reps):
+            _lib.call("trex_dfa_match_ranges", eng.handle, d.ptr, b.ptr, e.ptr, n, outs[0].ptr, outs[1].ptr, stream.handle)
+        mark.record(stream)
+    stream.synchronize()
+    return marks[0].elapsed_ms(marks[1]) / 20
+
+
+@pytest.mark.parametrize("n_states,n_classes", [(17, 40), (100, 100), (256, 250)])
+def test_tables_without_pairs_are_no_slower_by_rows(gpu_lib, n_states, n_classes):
+    """100,000 strings of 1 to 2 KB: the rows' kernel against the generic one
+    (rows by class: 1.28 times its time)."""
+    rng = np.random.default_rng(n_states)
+    table = _table(rng, n_states, n_classes)
+    offsets = np.zeros(100_001, np.int64)
+    np.cumsum(rng.integers(1000, 2000, 100_000), out=offsets[1:])
+    data = rng.integers(0, 256, int(offsets[-1]) + 1, dtype=np.uint8)
+    eng = DfaEngine(table)
+    rows = _ranges_ms(eng, data, offsets[:-1].copy(), offsets[1:].copy())
+    eng.set_variant("k1_generic")
+    assert rows < 1.12 * _ranges_ms(eng, data, offsets[:-1].copy(), offsets[1:].copy())

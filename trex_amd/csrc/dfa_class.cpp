@@ -82,19 +82,23 @@ std::vector<uint8_t> class_tables(const uint8_t* delta, int n, const char** kern
         return out;
     }
     const int all = count + 1, stride = (n + 15) / 16 * 16;
-    const bool pair = all * all * stride <= kWidePairBytes;
-    const int rows = pair ? all * all : all;
-    if (rows * stride > 65536 - 1040) return out;
-    *kernel = pair ? "dfa_cls_pair" : "dfa_cls_single";
-    out.resize(1040 + (size_t)rows * stride, 0);
+    if (all * all * stride > kWidePairBytes) {
+        *kernel = "dfa_cls_rows";
+        *classes = stride;
+        out.resize((size_t)256 * stride, 0);
+        for (int b = 0; b < 256; ++b)
+            for (int s = 0; s < n; ++s) out[(size_t)b * stride + s] = delta[s * 256 + b];
+        return out;
+    }
+    *kernel = "dfa_cls_pair";
+    out.resize(1040 + (size_t)all * all * stride, 0);
     uint32_t* map = reinterpret_cast<uint32_t*>(out.data());
     for (int b = 0; b < 257; ++b) {
         const uint32_t c = b < 256 ? cls[b] : (uint32_t)count;
-        map[b] = pair ? (c * all * stride) | (c * stride) << 16 : c * stride;
+        map[b] = (c * all * stride) | (c * stride) << 16;
     }
-    for (int r = 0; r < rows; ++r)
-        for (int s = 0; s < n; ++s)
-            out[1040 + (size_t)r * stride + s] = (uint8_t)(pair ? next(next(s, r / all), r % all) : next(s, r));
+    for (int r = 0; r < all * all; ++r)
+        for (int s = 0; s < n; ++s) out[1040 + (size_t)r * stride + s] = (uint8_t)next(next(s, r / all), r % all);
     return out;
 }
 

@@ -8,15 +8,15 @@
 //  * dfa16_cls_n10 / _n15 / _n16 (at most that many states): the pair's whole
 //    function as one 64-bit word, so the reads do not wait for the state, and a
 //    step is one, two or three instructions (Width).
-//  * dfa_cls_pair / dfa_cls_single (17 to 256 states): the successor bytes of
-//    a pair (or of one byte, where the pairs' table would not fit), read at
-//    the state.
+//  * dfa_cls_pair (17 to 256 states): the successor bytes of a pair, read at the
+//    state;
+//  * dfa_cls_rows, where the pairs' table would not fit: the successor bytes of
+//    every byte, without classes.
 //
-// Every string is read by 16-byte loads from its first byte on, whatever its
-// alignment, and its last len % 16 bytes by at most four loads of 8, 4, 2 and
-// 1 bytes that are issued ahead of the walk: no byte loop, and no byte outside
-// the string is read. Missing bytes of the last vector take the identity
-// class.
+// Every string is read as the aligned 16-byte vectors that hold its bytes (Span),
+// so up to 15 bytes on either side of it are read and not used: no byte loop but
+// _rows' two ends, and no load that could leave a page that the string is on.
+// Missing bytes of the first and last vector take the identity class.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -31,7 +31,7 @@ struct ClassArgs {
     int64_t n_strings;
     const uint8_t* tab;
     uint32_t tab_bytes;
-    uint32_t classes;        // identity class included (at most 16 states)
+    uint32_t classes;        // identity class included (at most 16 states); _rows: bytes from row to row
     uint32_t accept;         // bit s: state s accepts (at most 16 states)
     uint32_t start;
     const uint8_t* acc;      // accept byte of every state
@@ -46,7 +46,7 @@ namespace {
 using namespace trexdev;
 
 constexpr int kClsBytes = 256;    // byte -> class * 8
-constexpr int kMapBytes = 1040;   // map[257] of the wide form, padded
+constexpr int kMapBytes = 1040;   // map[257] of the pair form, padded
 constexpr int kPF = 4;            // vectors in flight ahead of the block being walked
 
 // Function words by number of states: the field of state s holds its successor,
@@ -166,24 +166,18 @@ __device__ __forceinline__ void class_kernel(const ClassArgs& A)
     A.out_accept[sid] = (uint8_t)((A.accept >> s) & 1u);
 }
 
-// 17 to 256 states. map[byte] holds the byte's class times the strides of the
-// two positions of a pair: low half for the first byte, high half for the
-// second (PAIR), or the class's row for single bytes; map[256] is the identity
-// class. A step reads succ[row + s].
-template <bool PAIR>
-struct WideWalk {
+// 17 to 256 states, pairs of classes. map[byte] holds the byte's class times the
+// strides of the two positions of a pair: low half for the first byte, high half
+// for the second; map[256] is the identity class. A step reads succ[row + s].
+struct PairWalk {
+    static constexpr int kPF = 4;
     const uint32_t* map;    // [257]
     const uint8_t* succ;
     uint32_t s;
 
-    __device__ __forceinline__ void step2(uint32_t m0, uint32_t m1) {
-        if constexpr (PAIR) {
-            s = succ[(m0 & 0xffffu) + (m1 >> 16) + s];
-        } else {
-            s = succ[m0 + s];
-            s = succ[m1 + s];
-        }
-    }
+    __device__ __forceinline__ PairWalk(const uint8_t* lds, const ClassArgs& A)
+        : map(reinterpret_cast<const uint32_t*>(lds)), succ(lds + kMapBytes), s(A.start) {}
+    __device__ __forceinline__ void step2(uint32_t m0, uint32_t m1) { s = succ[(m0 & 0xffffu) + (m1 >> 16) + s]; }
     __device__ __forceinline__ void word(uint32_t x) {
         const uint32_t m0 = map[x & 255u], m1 = map[(x >> 8) & 255u], m2 = map[(x >> 16) & 255u], m3 = map[x >> 24];
         step2(m0, m1);
@@ -227,15 +221,45 @@ struct WideWalk {
     }
 };
 
-template <bool PAIR, bool MASK>
+// 17 to 256 states where the pairs' table would not fit: a row of successors for
+// every byte value. Rows by class need a second read a byte for the class, which
+// fills the LDS pipe: 100 states and classes, 100,000 strings of 1 to 2 KB: 94 us
+// by class, 74 us so; 262,144 x 4 KiB: 421 us, 268 us; 400,000 of 20 to 400
+// bytes: 55 us, 51 us. (The pairs' rows halve the chain of reads: 20,000 x 4 KiB
+// take 93 us, 131 us so.)
+struct RowWalk {
+    static constexpr int kPF = 8;
+    const uint8_t* succ;
+    uint32_t stride;
+    uint32_t s;
+
+    __device__ __forceinline__ RowWalk(const uint8_t* lds, const ClassArgs& A) : succ(lds), stride(A.classes), s(A.start) {}
+    __device__ __forceinline__ uint32_t next(uint32_t b) const { return succ[__umul24(b, stride) + s]; }
+    __device__ __forceinline__ void vector(const uint4& v) {
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s = next((x[i >> 2] >> (8 * (i & 3))) & 255u);
+    }
+    template <int PF>
+    __device__ __forceinline__ void block(const uint4 (&a)[PF]) {
+#pragma unroll
+        for (int k = 0; k < PF; ++k) vector(a[k]);
+    }
+    __device__ __forceinline__ void masked(const uint4& v, uint32_t lo, uint32_t n) {
+        each_byte(v, lo, n, [&](uint32_t b) { s = next(b); });
+    }
+};
+
+template <class Walk, bool MASK>
 __device__ __forceinline__ void wide_kernel(const ClassArgs& A)
 {
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // map (1,040 bytes), succ
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int64_t sid = stage_and_pick(lds, A.tab, A.tab_bytes, A.begin, A.end, A.n_strings);
     if (sid < 0) return;
     const Span sp(A.bytes, A.begin[sid], A.end[sid]);
     const uint4 first = sp.first(), last = sp.last();
-    WideWalk<PAIR> w{reinterpret_cast<const uint32_t*>(lds), lds + kMapBytes, A.start};
+    Walk w(lds, A);
+    constexpr int kPF = Walk::kPF;
     if (sp.n_first) w.masked(first, sp.lo, sp.n_first);
     stream_span<kPF>(sp.body, sp.full, [&](const uint4 (&a)[kPF]) { w.block(a); }, [&](const uint4& v) { w.vector(v); });
     if (sp.n_last) w.masked(last, 0u, sp.n_last);
@@ -267,13 +291,13 @@ TREX_CLASS_KERNELS(W10, n10)
 TREX_CLASS_KERNELS(W15, n15)
 TREX_CLASS_KERNELS(W16, n16)
 
-// tab: map[257] (uint32, padded to 1,040 bytes), then the successor rows of
-// the class pairs (pair) or classes (single), padded to 16 states. Dynamic LDS
-// as above.
+// _pair: tab is map[257] (uint32, padded to 1,040 bytes), then the successor
+// rows of the class pairs, padded to 16 states; _rows: the successor rows of the
+// 256 bytes (`classes` is their stride). Dynamic LDS as above.
 #define TREX_WIDE_KERNEL(NAME, ...) \
     extern "C" __global__ void __launch_bounds__(256) NAME(ClassArgs A) { wide_kernel<__VA_ARGS__>(A); }
 
-TREX_WIDE_KERNEL(dfa_cls_pair, true, false)
-TREX_WIDE_KERNEL(dfa_cls_pair_mask, true, true)
-TREX_WIDE_KERNEL(dfa_cls_single, false, false)
-TREX_WIDE_KERNEL(dfa_cls_single_mask, false, true)
+TREX_WIDE_KERNEL(dfa_cls_pair, PairWalk, false)
+TREX_WIDE_KERNEL(dfa_cls_pair_mask, PairWalk, true)
+TREX_WIDE_KERNEL(dfa_cls_rows, RowWalk, false)
+TREX_WIDE_KERNEL(dfa_cls_rows_mask, RowWalk, true)
