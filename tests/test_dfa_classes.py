@@ -102,6 +102,22 @@ def _ranges_ms(eng, data, begin, end):
     return marks[0].elapsed_ms(marks[1]) / 20
 
 
+@pytest.mark.parametrize("n_states,n_classes,n", [(200, 200, 60000), (256, 250, 33000), (256, 250, 60000)])
+def test_large_tables_take_whole_workgroups(gpu_lib, n_states, n_classes, n):
+    """Batches whose waves would not all find LDS for a table of their own: as
+    long as the next larger batch at most (twice as long by waves)."""
+    rng = np.random.default_rng(n)
+    table = _table(rng, n_states, n_classes)
+    lengths = rng.integers(1000, 2000, 65536)
+    offsets = np.zeros(65537, np.int64)
+    np.cumsum(lengths, out=offsets[1:])
+    data = rng.integers(0, 256, int(offsets[-1]) + 1, dtype=np.uint8)
+    eng = DfaEngine(table)
+    few = _ranges_ms(eng, data, offsets[:n].copy(), offsets[1:n + 1].copy())
+    assert few < 1.3 * _ranges_ms(eng, data, offsets[:-1].copy(), offsets[1:].copy())
+    _check(table, data, offsets[:n:37].copy(), offsets[1:n + 1:37].copy())
+
+
 @pytest.mark.parametrize("n_states,n_classes", [(17, 40), (100, 100), (256, 250)])
 def test_tables_without_pairs_are_no_slower_by_rows(gpu_lib, n_states, n_classes):
     """100,000 strings of 1 to 2 KB: the rows' kernel against the generic one

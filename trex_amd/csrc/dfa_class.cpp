@@ -50,8 +50,12 @@ struct ClassArgs {
 
 // Launch shape of the class kernels: from kClassBlockFrom strings on, 256
 // threads a workgroup, which orders its strings by length (kOrderBytes of LDS);
-// below, one wave a workgroup, so that the waves spread over the CUs.
+// below, one wave a workgroup, so that the waves spread over the CUs, while the
+// LDS holds the tables of all of them at once (60,000 strings and rows of 200
+// states, 50 KB: 1 to 2 KB a string 132 us by waves, 69 us by workgroups of 256;
+// 8 to 30 bytes: 10.9 and 6.4 us).
 constexpr int64_t kClassBlockFrom = 65536;
+constexpr int kLdsBytes = 160 << 10;   // of a compute unit
 constexpr unsigned kOrderBytes = 64 * 4 + 256 * 2;   // order_bytes(256) of device_common.h
 
 // Byte-class tables of the class kernels (layouts in dfa_class_kernels.hip)
@@ -123,7 +127,8 @@ int make_class_form(const uint8_t* delta, const uint8_t* accept, const uint64_t*
 int launch_class_form(const ClassForm& f, const uint8_t* d_bytes, const int64_t* d_begin, const int64_t* d_end,
                       int64_t n_strings, bool leave_alike, uint8_t* d_state, uint64_t* d_mask, uint8_t* d_accept,
                       hipStream_t stream) {
-    const unsigned block = n_strings >= kClassBlockFrom ? kBlock : 64u;
+    const int64_t resident = (int64_t)device_cu_count() * (kLdsBytes / f.tab_bytes);   // tables
+    const unsigned block = n_strings < kClassBlockFrom && n_strings <= 64 * resident ? 64u : kBlock;
     const int64_t blocks = (n_strings + block - 1) / block;
     if (blocks > 0x7fffffff) return fail(TREX_ERR_CAPACITY, "too many strings");
     const unsigned lds = (unsigned)f.tab_bytes + (block == kBlock ? kOrderBytes : 0u);
