@@ -159,8 +159,8 @@ int trex_dfa_set_prefetch(trex_dfa* h, int vectors);
  * modulo 4 KiB at once, which crowds a few HBM channels. Same results.
  * mode -1 (default): on for batches of 131,072 strings and more whose table
  * synchronises (some word over its window bytes sends every state that can
- * occur to one state) and has no state but the dead one that every live byte
- * keeps, for the workgroups whose strings are alike; 0 off; 1 on for every
+ * occur to one state) and, of several states that can occur, has none but the
+ * dead one that every live byte keeps, for the workgroups whose strings are alike; 0 off; 1 on for every
  * launch of that kernel. With a mode of 0 or 1 contiguous strings are walked in
  * the handle's variant, otherwise by byte classes (a forced variant at mode -1
  * is rotated for every table that synchronises).

@@ -110,7 +110,8 @@ def test_rotation_is_reported_as_launched(gpu_lib):
     from trex_amd.tables import dfa_byte_table
     search = DfaEngine(dfa_byte_table(compile_regex("[A-Z]*(ERROR|WARN|FAIL)[A-Z]*")))
     recent = DfaEngine(dfa_byte_table(compile_regex("(A|B|C|D)*(A|B)(C|D)")))
-    assert search.rotation() == (False, True) and recent.rotation() == (True, True)
+    only = DfaEngine(dfa_byte_table(compile_regex("[@-_]*")))   # one live state: every function is its constant
+    assert search.rotation() == (False, True) and recent.rotation() == (True, True) and only.rotation() == (True, True)
     search.set_variant("k2_window_f")
     assert search.rotation() == (True, True)
     search.set_variant("auto")

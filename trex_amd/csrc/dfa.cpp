@@ -178,14 +178,15 @@ void analyse_window(trex_dfa* h, const uint8_t* delta) {
         for (int q : states) all = all && good[p][q];
     h->synchronizes = all || live_bytes.empty();
     // a state that every live byte leaves alone (found text stays found) keeps
-    // functions from turning constant until the text has reached it
+    // functions from turning constant until the text has reached it (an only
+    // state is the constant)
     bool sticky = false;
     for (int s : states) {
         bool stays = s != dead;
         for (int b : live_bytes) stays = stays && delta[s * 256 + b] == s;
         sticky = sticky || stays;
     }
-    h->rotate = h->synchronizes && !sticky;
+    h->rotate = h->synchronizes && (!sticky || states.size() == 1);
 }
 
 // From kRotateFrom strings on (eight waves a CU; below, the rotated order is no
