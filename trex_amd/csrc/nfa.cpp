@@ -17,7 +17,12 @@ using namespace trex;
 namespace {
 constexpr int kNfaBlock = 512;
 constexpr int kNfa5Block = 1024;   // nfa64_window5: one 1024-thread workgroup per CU holds the 104 KB of tables
-constexpr int64_t kOneLaneFrom = 160, kTwoLanesFrom = 64;   // strings per CU
+// Strings per CU above which a string takes one lane, or two, of the slice
+// kernels. One / two / four lanes a string, us: 57,000 x 2 KiB 267 / 255, 65,536
+// 273 / 271, 100,000 392 / 483 (300 bytes: 45.5 / 44.0, 46.3 / 46.0, 67 / 80);
+// 20,000 x 2 KiB 179 / 172 with two / four, 24,000 181 / 177, 32,000 187 / 209
+// (100 to 1,000 bytes: 90 / 89, 90 / 89, 92 / 99).
+constexpr int64_t kOneLaneFrom = 256, kTwoLanesFrom = 96;
 constexpr int kMaxSymbols = 62;   // (62 + 2) classes x 2 KB of nibble tables fit one workgroup's LDS
 }
 
@@ -320,8 +325,8 @@ int trex_nfa_match_ranges(trex_nfa* h, const uint8_t* d_bytes, const int64_t* d_
         uint64_t start = h->start, accept = h->accept;
         void* args[] = {&d_bytes, &d_begin, &d_end, &n_strings, &tab5, &win4, &start, &accept, &d_final_mask, &d_accept};
         // one workgroup a CU (the tables fill its LDS), as many threads as
-        // spread the batch over all CUs; several lanes a string while that
-        // leaves a wave or so on each SIMD (measured in nfa_kernels.hip)
+        // spread the batch over all CUs; several lanes a string where they are
+        // faster (kOneLaneFrom)
         const int64_t cus = device_cu_count();
         const int64_t lanes = !six || n_strings > cus * kOneLaneFrom ? 1 : n_strings > cus * kTwoLanesFrom ? 2 : 4;
         const int64_t threads = (n_strings * lanes + cus - 1) / cus;
