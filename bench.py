@@ -521,8 +521,9 @@ def scan_leg(args, data, stream) -> dict:
     log(f"look-back scan: {n_long} x {per >> 20} MiB, {plan.n_chunks} chunks of {plan.chunk_len >> 10} KiB, "
         f"{ms:.4f} ms per launch, "
         f"{gchars:.1f} Gchars/s, {achieved:.0f} GB/s, error word {err}")
+    suffix = "_c2" if args.scan_chains == 2 else "_n8" if table.n_states <= 8 else ""
     out = {"workload": f"{n_long} strings x {per >> 20} MiB, {plan.chunk_len >> 10} KiB chunks chained by the look-back",
-           "kernel": "dfa16_chunks_window", "chunks": plan.n_chunks, "chunk_len": plan.chunk_len, "kernel_avg_ms": round(ms, 4),
+           "kernel": "dfa16_chunks_window" + suffix, "chunks": plan.n_chunks, "chunk_len": plan.chunk_len, "kernel_avg_ms": round(ms, 4),
            "value": round(gchars, 1), "unit": "Gchars/s", "error_word": int(err),
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4), "alg_bytes_per_launch": alg_bytes},
@@ -560,9 +561,9 @@ def scan_leg(args, data, stream) -> dict:
     log(f"look-back scan over the chunk image ({plan.image_size() >> 20} MiB, built on the host in "
         f"{t_build:.2f} s): {ims:.4f} ms per launch, {data.nbytes / (ims * 1e-3) / 1e9:.1f} Gchars/s, "
         f"{iach:.0f} GB/s, error word {ierr}")
-    out["csr"] = {"kernel": "dfa16_chunks_window", "kernel_avg_ms": out["kernel_avg_ms"], "value": out["value"],
+    out["csr"] = {"kernel": "dfa16_chunks_window" + suffix, "kernel_avg_ms": out["kernel_avg_ms"], "value": out["value"],
                   "roofline_frac": out["roofline"]["frac"]}
-    out.update({"kernel": "dfa16_chunks_window_img", "kernel_avg_ms": round(ims, 4),
+    out.update({"kernel": "dfa16_chunks_window_img" + suffix, "kernel_avg_ms": round(ims, 4),
                 "value": round(data.nbytes / (ims * 1e-3) / 1e9, 1), "error_word": int(ierr),
                 "layout": "chunk-interleaved image of the plan (tile of 64 chunks, 16-byte vectors side by side)"})
     out["roofline"].update({"achieved": round(iach, 1), "frac": round(iach / HBM_PEAK_GBS, 4)})

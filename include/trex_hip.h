@@ -376,8 +376,8 @@ int trex_pnfa_loglik_host(trex_pnfa* h, const uint8_t* symbols, int64_t n_seq, i
  * per library and one synchronous launch per batch and pattern,
  * cuda/monoid_batch.cu:596-671, cuda/nfa_tc_evolution.cu:943-1013); long DFA
  * strings are chained by the decoupled look-back of monoid_r3_kernel
- * (cuda/monoid_scan.cu:369-451), long NFA strings by speculative chunks with
- * checkpoints and an exact fix-up pass.
+ * (cuda/monoid_scan.cu:369-451), long NFA strings by speculative chunks and an
+ * exact fix-up pass.
  * ------------------------------------------------------------------------ */
 typedef struct trex_mix trex_mix;
 
@@ -434,7 +434,7 @@ int trex_mix_set_grid(trex_mix* m, int64_t workgroups);
 #define TREX_MIX_FORM_SLICE 1
 int trex_mix_set_form(trex_mix* m, int form);
 /* Enqueues on `stream`, behind the last run, a copy of the run's first four
- * queue words (ticket, error word, converged count, one flag) to dst:
+ * queue words (ticket, error word, converged count, 0) to dst:
  * 16 bytes, 16-byte aligned, device or pinned host memory, copied by a kernel
  * so the check never waits behind long copies on the copy engines. With no
  * planned work nothing is enqueued. No reference counterpart. */

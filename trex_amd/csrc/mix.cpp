@@ -6,9 +6,10 @@
 // chunks plus one fix-up item). Items are grouped per (role, pattern) into
 // batches of at most kMixBlock lane items, one workgroup each. Queue order:
 //   1. NFA_SPEC batches (no waiting, the heaviest bytes),
-//   2. DFA_CHUNK batches, in chunk-position order (a chunk's predecessor is
-//      in an earlier or the same batch),
-//   3. NFA_FIXUP batches (wait only on 1),
+//   2. DFA_CHUNK batches, in chunk-position order, or string by string where
+//      the plan made the chunks short (a chunk's predecessor is in an earlier
+//      or the same batch),
+//   3. NFA_FIXUP batches (wait only on 1); behind 4 when they are one to a wave,
 //   4. WHOLE batches, longest first (LPT: a batch lasts as long as its
 //      longest string; NFA bytes weigh kNfaWeight DFA bytes).
 

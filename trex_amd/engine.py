@@ -473,11 +473,11 @@ class NfaEngine:
 
     def match_split(self, data: np.ndarray, offsets: np.ndarray, params=None):
         """Host CSR batch through the mixed queue with this one pattern: strings
-        over the split length are cut into chunks walked in parallel from the
-        set of all states (the first from the start set), each with
-        checkpoints, then one fix-up lane per string walks the chunks again
-        from the true entry set until it meets a checkpoint; shorter strings
-        are walked whole. The reference walks every string on one thread
+        over the split length are cut into chunks walked in parallel, each
+        from the set that a walk of the bytes ahead of it reaches (the first
+        from the start set); then a fix-up per string takes the chunks' ends
+        where those guesses make them known and walks the others again from
+        the set they are entered with; shorter strings are walked whole. The reference walks every string on one thread
         (cuda/nfa_tc_evolution.cu:683-745). Returns (final mask, accept,
         kernel_ms, total_ms)."""
         import time

@@ -6,7 +6,8 @@ A :class:`MixEngine` holds many resident patterns. ``plan`` turns a batch
 length-sorted work queue; ``run`` is one launch sequence on a stream (it can
 be captured once into a HIP graph and replayed). Long strings are cut into
 chunks: DFA chunks are chained by the decoupled look-back, NFA chunks are
-walked speculatively from the set of all states and fixed up exactly.
+walked from a guess of the set they are entered with (what a walk of the bytes
+ahead of them reaches) and fixed up exactly.
 
 The reference has one global engine per library and one synchronous launch
 per pattern and batch (cuda/monoid_batch.cu:596-671).
@@ -127,7 +128,7 @@ class MixEngine:
 
     def status_to(self, dst: int, stream: Stream | None = None) -> None:
         """Enqueue a copy of the last run's queue words (ticket, error word, converged,
-        flag; 16 bytes) to dst (device or pinned host memory) behind the run."""
+        0; 16 bytes) to dst (device or pinned host memory) behind the run."""
         _lib.call("trex_mix_status", self.handle, dst, stream.handle if stream else None)
 
     def error(self, stream: Stream | None = None) -> int:
