@@ -318,7 +318,8 @@ struct WinCheck {
 };
 
 // Pair index sym0 | sym1 << 5 of the low / high two bytes of a word (sym = byte
-// & 31): a byte dot product, one instruction where shifts and masks take three.
+// & 31): a byte dot product, one instruction where shifts and masks take three,
+// and a longer wait for its result (PairIndex in dfa_kernels.hip).
 __device__ __forceinline__ uint32_t pair_lo(uint32_t x) {
     return __builtin_amdgcn_udot4(x & 0x1f1f1f1fu, 0x00002001u, 0u, false);
 }

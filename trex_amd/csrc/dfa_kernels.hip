@@ -57,27 +57,44 @@ using namespace trexdev;
 
 constexpr int kIlGroup = 64;   // strings per group of the interleaved layout (one wave)
 
+// The pair index by shifts and masks, or by the dot product. Contiguous strings
+// take the first (50 x 3,000 bytes: 41.0 us, by dot products 43.7; 16,000: 53.3 and
+// 55.1; 262,144 x 4,000..4,200: 302 and 308), interleaved rows the second (50:
+// 28.7 and 29.9 us, but 1,000: 32.6 and 31.2; 65,536 x 4 KiB: 49.5 and 47.0): their
+// loads are few instructions, so that the indices bound a full chip.
+template <bool DOT>
+struct PairIndex {
+    __device__ __forceinline__ static uint32_t lo(uint32_t x) {
+        return DOT ? pair_lo(x) : (x & 31u) | (((x >> 8) & 31u) << 5);
+    }
+    __device__ __forceinline__ static uint32_t hi(uint32_t x) {
+        return DOT ? pair_hi(x) : ((x >> 16) & 31u) | (((x >> 24) & 31u) << 5);
+    }
+};
+
 // Pair-step policies over the LDS pair table: stage() fills it from the
 // global table, lane_table() is where this lane reads it, word() takes two
 // pair steps.
+template <bool DOT>
 struct StepK2W {
     static constexpr int kTableBytes = 1024 * 16;
     __device__ __forceinline__ static void stage(uint8_t* dst, const uint8_t* src) { stage_table(dst, src, kTableBytes); }
     __device__ __forceinline__ static const uint8_t* lane_table(const uint8_t* t) { return t; }
     __device__ __forceinline__ static uint32_t word(const uint8_t* __restrict__ t, uint32_t s, uint32_t x) {
-        s = t[(pair_lo(x) << 4) | s];
-        return t[(pair_hi(x) << 4) | s];
+        s = t[(PairIndex<DOT>::lo(x) << 4) | s];
+        return t[(PairIndex<DOT>::hi(x) << 4) | s];
     }
 };
 
+template <bool DOT>
 struct StepK2F {
     static constexpr int kTableBytes = 1024 * 8;
     __device__ __forceinline__ static void stage(uint8_t* dst, const uint8_t* src) { stage_table(dst, src, kTableBytes); }
     __device__ __forceinline__ static const uint8_t* lane_table(const uint8_t* t) { return t; }
     __device__ __forceinline__ static uint32_t word(const uint8_t* __restrict__ t, uint32_t s, uint32_t x) {
         const uint64_t* f = reinterpret_cast<const uint64_t*>(t);
-        const uint64_t f0 = f[pair_lo(x)];
-        const uint64_t f1 = f[pair_hi(x)];
+        const uint64_t f0 = f[PairIndex<DOT>::lo(x)];
+        const uint64_t f1 = f[PairIndex<DOT>::hi(x)];
         s = (uint32_t)(f0 >> (s << 2)) & 15u;
         return (uint32_t)(f1 >> (s << 2)) & 15u;
     }
@@ -86,6 +103,7 @@ struct StepK2F {
 // k2f with the function table in kCopies interleaved copies: entry p of copy
 // c sits at (p * kCopies + c) * 8 bytes and lane l reads copy l % kCopies, so
 // the lanes of one LDS access that read different copies use disjoint banks.
+template <bool DOT>
 struct StepK2FR {
     static constexpr int kCopies = 4;
     static constexpr int kTableBytes = 1024 * 8 * kCopies;
@@ -99,8 +117,8 @@ struct StepK2FR {
     }
     __device__ __forceinline__ static uint32_t word(const uint8_t* __restrict__ t, uint32_t s, uint32_t x) {
         const uint64_t* f = reinterpret_cast<const uint64_t*>(t);
-        const uint64_t f0 = f[pair_lo(x) * kCopies];
-        const uint64_t f1 = f[pair_hi(x) * kCopies];
+        const uint64_t f0 = f[PairIndex<DOT>::lo(x) * kCopies];
+        const uint64_t f1 = f[PairIndex<DOT>::hi(x) * kCopies];
         s = (uint32_t)(f0 >> (s << 2)) & 15u;
         return (uint32_t)(f1 >> (s << 2)) & 15u;
     }
@@ -290,10 +308,10 @@ __device__ __forceinline__ void rot_kernel(const uint8_t* __restrict__ bytes, co
         for (int k = 0; k < 4; ++k) {
             w.add(words[k]);
             if (walking) {
-                sa = StepK2F::word(f2, sa, words[k]);
+                sa = StepK2F<false>::word(f2, sa, words[k]);
             } else {
-                f = fn_then(f, load_row(t2, pair_lo(words[k])));
-                f = fn_then(f, load_row(t2, pair_hi(words[k])));
+                f = fn_then(f, load_row(t2, PairIndex<false>::lo(words[k])));
+                f = fn_then(f, load_row(t2, PairIndex<false>::hi(words[k])));
             }
         }
         if (!walking && fn_is_const(f)) {
@@ -308,17 +326,17 @@ __device__ __forceinline__ void rot_kernel(const uint8_t* __restrict__ bytes, co
     stream_blocks<PF>(v + r, nvec - r, [&](const uint4 (&a)[PF]) {
         if (__ballot(!walking) == 0ull) {
 #pragma unroll
-            for (int k = 0; k < PF; ++k) sa = window_vec<StepK2F>(f2, sa, a[k], w);
+            for (int k = 0; k < PF; ++k) sa = window_vec<StepK2F<false>>(f2, sa, a[k], w);
         } else {
 #pragma unroll
             for (int k = 0; k < PF; ++k) mixed(a[k]);
         }
     }, [&](const uint4& x) {
-        if (__ballot(!walking) == 0ull) sa = window_vec<StepK2F>(f2, sa, x, w);
+        if (__ballot(!walking) == 0ull) sa = window_vec<StepK2F<false>>(f2, sa, x, w);
         else mixed(x);
     });
     // phase B: vectors 0 .. r-1 from the head's state
-    stream_body<PF>(v, r, [&](uint4 x) { s = window_vec<StepK2F>(f2, s, x, w); });
+    stream_body<PF>(v, r, [&](uint4 x) { s = window_vec<StepK2F<false>>(f2, s, x, w); });
     // the dead state is absorbing; `init` may leave its slot out (when no
     // window byte leads to it, it is reached only through a byte the window
     // check or the head's exact walk already sends to it)
@@ -350,10 +368,10 @@ __device__ __forceinline__ void rot_kernel(const uint8_t* __restrict__ bytes, co
     }
 
 #define TREX_WINDOW_KERNELS(BASE, STEP)                        \
-    TREX_WINDOW_KERNEL(BASE##_pf8, STEP, 8, false)             \
-    TREX_WINDOW_KERNEL(BASE##_pf16, STEP, 16, false)           \
-    TREX_WINDOW_KERNEL(BASE##_il_pf8, STEP, 8, true)           \
-    TREX_WINDOW_KERNEL(BASE##_il_pf16, STEP, 16, true)
+    TREX_WINDOW_KERNEL(BASE##_pf8, STEP<false>, 8, false)      \
+    TREX_WINDOW_KERNEL(BASE##_pf16, STEP<false>, 16, false)    \
+    TREX_WINDOW_KERNEL(BASE##_il_pf8, STEP<true>, 8, true)     \
+    TREX_WINDOW_KERNEL(BASE##_il_pf16, STEP<true>, 16, true)
 
 TREX_WINDOW_KERNELS(dfa16_k2w, StepK2W)
 TREX_WINDOW_KERNELS(dfa16_k2f, StepK2F)
