@@ -19,7 +19,10 @@
  * the message of the calling thread's last failure. A string batch is CSR:
  * bytes[offsets[i] .. offsets[i+1]) is string i, offsets has n_strings + 1
  * entries. "d_" arguments are device pointers, other pointers are host memory.
- * `stream` is a hipStream_t (NULL = the default stream).
+ * `stream` is a hipStream_t (NULL = the default stream). Contiguous strings in
+ * device memory are read as the aligned 16-byte vectors that hold their bytes:
+ * up to 15 bytes on either side of a string, on the page its end is on, are read
+ * and not used.
  */
 #ifndef TREX_HIP_H
 #define TREX_HIP_H
